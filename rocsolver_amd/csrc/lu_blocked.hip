@@ -3,12 +3,13 @@
 //
 // getrf, per block column j of width jb (reference structure:
 // library/src/lapack/roclapack_getrf.hpp:608-752, without rocBLAS):
-//   1. panel_kernel: one workgroup per matrix factors A[j:m, j:j+jb] with
-//      partial pivoting (workgroup arg-max per column), interchanging rows
-//      inside the panel at each column; then applies the panel's interchanges
-//      to every other column at once (roclapack_getf2.hpp:41-99 semantics:
-//      the same final rows); u12_kernel then solves U12 = L11^-1 A12 for the
-//      columns right of the panel, one thread per column.
+//   1. panel_reg (lu_panel.hip): one workgroup per matrix factors
+//      A[j:m, j:j+jb] in registers with partial pivoting, applies its
+//      interchanges to the other columns and solves U12 = L11^-1 A12.
+//      Panels too tall for the registers: panel_kernel, interchanging rows
+//      inside the panel at each column in global memory, then every other
+//      column at once (roclapack_getf2.hpp:41-99 semantics: the same final
+//      rows), and u12_kernel, one thread per column right of the panel.
 //   2. gemm_sub_kernel: A22 -= L21 * U12 on MFMA (v_mfma_f64_16x16x4f64 /
 //      v_mfma_f32_16x16x4f32), 64x64 tiles.
 // getrs (roclapack_getrs.hpp:117-150): laswp, then for each 64-row diagonal
@@ -21,9 +22,8 @@
 namespace rsa
 {
 
-constexpr int PANEL_NB = 32; // panel width
-constexpr int PANEL_THREADS = 256;
-constexpr int PANEL_TALL = 2048; // panels of this many rows or more: 2 * PANEL_THREADS
+constexpr int PANEL_NB = 32; // width of the panel in global memory
+constexpr int PANEL_THREADS = 512;
 constexpr int TRSM_NB = 64; // getrs diagonal block
 constexpr int64_t MAX_GRID_YZ = 65535; // grid y/z limit: larger batches are launched in chunks
 
@@ -45,13 +45,14 @@ rocblas_status reset_info(hipStream_t stream, int* info, int bc)
 }
 
 // ------------------------------------------------------------ panel + trsm
-template <typename T, bool PIVOT, int NT>
-__global__ __launch_bounds__(NT) void panel_kernel(int m, int n, Batch<T> AA, int lda,
+template <typename T, bool PIVOT>
+__global__ __launch_bounds__(PANEL_THREADS) void panel_kernel(int m, int n, Batch<T> AA, int lda,
                                                               int* __restrict__ ipivA,
                                                               int64_t strideP,
                                                               int* __restrict__ info, int j0,
                                                               int jb)
 {
+    constexpr int NT = PANEL_THREADS;
     constexpr int NW = NT / 64;
     __shared__ T s_key[NW];
     __shared__ int s_idx[NW];
@@ -447,30 +448,28 @@ rocblas_status getrf_blocked(hipStream_t stream, int m, int n, Batch<T> A, int l
     if(st != rocblas_status_success)
         return st;
     const int kmax = m < n ? m : n;
-    for(int j = 0; j < kmax; j += PANEL_NB)
+    for(int j = 0, jb = 0; j < kmax; j += jb)
     {
-        const int jb = (kmax - j) < PANEL_NB ? (kmax - j) : PANEL_NB;
-        // tall panels (2048 rows or more) with 512 threads: half the rows
-        // per thread in each column step; shorter ones with 256, whose
-        // update keeps two rows' loads in flight without spilling
-        if(pivot && m >= PANEL_TALL)
-            hipLaunchKernelGGL((panel_kernel<T, true, 2 * PANEL_THREADS>), dim3(bc),
-                               dim3(2 * PANEL_THREADS), 0, stream, m, n, A, lda, ipiv, strideP,
-                               info, j, jb);
-        else if(pivot)
-            hipLaunchKernelGGL((panel_kernel<T, true, PANEL_THREADS>), dim3(bc), dim3(PANEL_THREADS),
-                               0, stream, m, n, A, lda, ipiv, strideP, info, j, jb);
-        else if(m >= PANEL_TALL)
-            hipLaunchKernelGGL((panel_kernel<T, false, 2 * PANEL_THREADS>), dim3(bc),
-                               dim3(2 * PANEL_THREADS), 0, stream, m, n, A, lda, ipiv, strideP,
-                               info, j, jb);
-        else
-            hipLaunchKernelGGL((panel_kernel<T, false, PANEL_THREADS>), dim3(bc),
-                               dim3(PANEL_THREADS), 0, stream, m, n, A, lda, ipiv, strideP, info,
-                               j, jb);
-        RSA_LAUNCH_CHECK();
+        // panels that fit the registers of one workgroup; taller ones are
+        // factored in global memory
+        const int wreg = panel_reg_width<T>(m - j, lda);
+        const int width = wreg ? wreg : PANEL_NB;
+        jb = (kmax - j) < width ? (kmax - j) : width;
         const int r0 = j + jb;
-        if(r0 < n)
+        if(wreg)
+        {
+            st = panel_reg<T>(stream, m, A, lda, ipiv, strideP, info, j, jb, 0, n, bc, pivot);
+            if(st != rocblas_status_success)
+                return st;
+        }
+        else if(pivot)
+            hipLaunchKernelGGL((panel_kernel<T, true>), dim3(bc), dim3(PANEL_THREADS), 0, stream, m,
+                               n, A, lda, ipiv, strideP, info, j, jb);
+        else
+            hipLaunchKernelGGL((panel_kernel<T, false>), dim3(bc), dim3(PANEL_THREADS), 0, stream,
+                               m, n, A, lda, ipiv, strideP, info, j, jb);
+        RSA_LAUNCH_CHECK();
+        if(r0 < n && !wreg)
             for(int64_t b0 = 0; b0 < bc; b0 += MAX_GRID_YZ)
             {
                 const int nb = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);

@@ -1,0 +1,88 @@
+"""GPU parity of the blocked LU's kernels at the edges of their dispatch, against the oracle.
+
+The register-resident panel has one instantiation per range of row counts
+(512 threads, 1 to 16 rows each, 32 to 8 columns wide), so each test runs at
+the last row count of a range and the first of the next.
+"""
+import numpy as np
+import pytest
+
+import oracle
+import rocsolver_amd as ra
+
+pytestmark = pytest.mark.gpu
+EPS = {np.float64: np.finfo(np.float64).eps, np.float32: np.finfo(np.float32).eps}
+PANEL_ROWS = [65, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193]
+
+
+def rel_fro(a, b):
+    return np.linalg.norm((a - b).ravel()) / max(np.linalg.norm(b.ravel()), 1e-300)
+
+
+@pytest.mark.parametrize("m", PANEL_ROWS)
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_one_panel_special_values(torch_gpu, handle, m, dtype):
+    """Eight columns, so one panel of any width: the same operations in the
+    same order as the oracle, bit for bit, with NaN, infinities, a zero
+    column, exact ties and columns that are constant."""
+    print(f"panel m={m} {dtype.__name__}", flush=True)
+    g = np.random.default_rng(m)
+    n, bc = 8, 6
+    A0 = g.uniform(-1, 1, size=(bc, n, m)).astype(dtype)
+    A0[1, 3, m // 2] = np.nan
+    A0[2, 0, 0] = np.nan
+    A0[3, 2, m - 1] = -np.inf
+    A0[4, 5, :] = 0.0
+    A0[4, 1, :] = 0.5
+    A0[5] = np.round(A0[5] * 4) / 4
+    Ao = A0.copy()
+    ip_o, in_o = oracle.getf2(Ao, m)
+    Ad = torch_gpu.from_numpy(A0).cuda()
+    ip, info = ra.getrf(handle, Ad, m=m)
+    torch_gpu.cuda.synchronize()
+    np.testing.assert_array_equal(info.cpu().numpy(), in_o)
+    np.testing.assert_array_equal(ip.cpu().numpy(), ip_o)
+    np.testing.assert_array_equal(Ad.cpu().numpy(), Ao)
+
+
+@pytest.mark.parametrize("m,n", [(m, 40) for m in PANEL_ROWS[1:]] + [(16, 700), (90, 333), (513, 513)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_panels_and_updates(torch_gpu, handle, m, n, dtype):
+    """Several panels with a partial last one, lda > m: pivots equal where the
+    oracle finds them unambiguous, factors within 10 min(m,n) eps there, and
+    P A = L U for every matrix; the padding rows are untouched."""
+    print(f"getrf m={m} n={n} {dtype.__name__}", flush=True)
+    g = np.random.default_rng(m * 31 + n)
+    bc, lda = 3, m + 3
+    A0 = g.uniform(-1, 1, size=(bc, n, lda)).astype(dtype)
+    Ao = np.ascontiguousarray(A0[:, :, :m])
+    ip_o, in_o, gap = oracle.getf2(Ao, m, with_gap=True)
+    Ad = torch_gpu.from_numpy(A0.copy()).cuda()
+    ip, info = ra.getrf(handle, Ad, m=m, batched=True)
+    torch_gpu.cuda.synchronize()
+    Ag, ipg = Ad.cpu().numpy(), ip.cpu().numpy()
+    np.testing.assert_array_equal(Ag[:, :, m:], A0[:, :, m:])
+    Ag = np.ascontiguousarray(Ag[:, :, :m])
+    np.testing.assert_array_equal(info.cpu().numpy(), in_o)
+    unamb = (gap > 1e3 * max(m, n) * EPS[dtype]).all(axis=1)
+    np.testing.assert_array_equal(ipg[unamb], ip_o[unamb])
+    for b in np.nonzero(unamb)[0]:
+        assert rel_fro(Ag[b], Ao[b]) <= 10 * min(m, n) * EPS[dtype]
+    be = oracle.lu_backward_error(A0[:, :, :m].astype(np.float64), Ag.astype(np.float64), ipg, m, n,
+                                  EPS[dtype])
+    assert be.max() < 10.0, be
+
+
+@pytest.mark.parametrize("m,n", [(300, 100), (1100, 70), (2500, 24)])
+def test_panels_without_pivoting(torch_gpu, handle, m, n):
+    g = np.random.default_rng(m)
+    A0 = g.uniform(-1, 1, size=(2, n, m))
+    A0[:, np.arange(n), np.arange(n)] += m
+    Ao = A0.copy()
+    in_o = oracle.getf2_npvt(Ao, m)
+    Ad = torch_gpu.from_numpy(A0).cuda()
+    _, info = ra.getrf(handle, Ad, m=m, pivot=False)
+    torch_gpu.cuda.synchronize()
+    np.testing.assert_array_equal(info.cpu().numpy(), in_o)
+    for b in range(2):
+        assert rel_fro(Ad.cpu().numpy()[b], Ao[b]) <= 10 * n * EPS[np.float64]
