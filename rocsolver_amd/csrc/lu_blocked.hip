@@ -316,30 +316,61 @@ __global__ __launch_bounds__(64) void u12_kernel(int n, Batch<T> AA, int lda, in
 
 // ------------------------------------------------------------------ GEMM
 // C[M x N] -= op(A)[M x K] * B[K x N], column-major, one 64x64 tile per
-// workgroup (4 waves, each 32x32 = 2x2 MFMA 16x16 blocks), K staged through
-// LDS in chunks of 16 (MFMA operand/result layouts: mfma.hpp).
+// workgroup (4 waves, each 32x32 = 2x2 MFMA 16x16 blocks).  K goes through
+// LDS in double-buffered chunks of 16, one barrier a chunk: the next chunk's
+// global loads are in flight during this chunk's matrix instructions.  The
+// operands are swapped (each 16x16 block is formed as its transpose: MFMA
+// operand/result layouts in mfma.hpp), so 16 lanes read and write 16
+// consecutive rows of C.
+//
+// Workgroups go round-robin to the 8 XCDs in launch order.  With 8 matrices
+// or more a matrix's tiles are given to one XCD, so that its A and B panels
+// are read into one L2.
 constexpr int GT = 64; // tile
 constexpr int GK = 16; // k chunk
+constexpr int XCDS = 8;
 
 template <typename T, bool TRANSA>
 __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batch<T> AA,
                                                        int64_t offA, int lda, Batch<T> BB,
                                                        int64_t offB, int ldb, Batch<T> CC,
                                                        int64_t offC, int ldc,
-                                                       const int* __restrict__ skip, int64_t boff)
+                                                       const int* __restrict__ skip, int bc,
+                                                       int tm, int tn)
 {
-    using acc_t = typename mfma16<T>::acc_t;
-    __shared__ T sA[GK][GT]; // sA[k][i]
-    __shared__ T sB[GK][GT]; // sB[k][j]
+    using M_ = mfma16<T>;
+    using acc_t = typename M_::acc_t;
+    // LDS strides that spread an MFMA operand read (16 rows or columns, 2
+    // FP64 or 4 FP32 values of k per 32 or 64 lanes) over the banks
+    constexpr int SR = GT + 16; // [k][i]
+    constexpr int SC = GK + 1; // [j][k]
+    constexpr int PT = GT * GK / 256; // entries of each operand per thread and chunk
+    __shared__ T sA[2][TRANSA ? GT * SC : GK * SR];
+    __shared__ T sB[2][GT * SC];
 
-    const int64_t b = blockIdx.z + boff;
+    const unsigned tiles = unsigned(tm) * unsigned(tn);
+    const unsigned id = blockIdx.x;
+    int64_t b;
+    unsigned tile;
+    if(bc >= XCDS)
+    {
+        b = int64_t(id / (XCDS * tiles)) * XCDS + id % XCDS;
+        tile = (id / XCDS) % tiles;
+        if(b >= bc)
+            return;
+    }
+    else
+    {
+        b = id / tiles;
+        tile = id % tiles;
+    }
     if(skip && skip[b] != 0)
         return;
     const T* A = AA[b] + offA;
     const T* Bm = BB[b] + offB;
     T* C = CC[b] + offC;
-    const int i0 = blockIdx.x * GT;
-    const int j0 = blockIdx.y * GT;
+    const int i0 = int(tile % tm) * GT;
+    const int j0 = int(tile / tm) * GT;
     const int tid = threadIdx.x;
     const int wid = tid / 64;
     const int lane = tid % 64;
@@ -353,68 +384,79 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
         for(int t = 0; t < 2; ++t)
             acc[s][t] = acc_t{0, 0, 0, 0};
 
-    for(int k0 = 0; k0 < K; k0 += GK)
-    {
-        // stage A: GT x GK, B: GK x GT (zero padded)
+    T ra[PT], rb[PT];
+    auto load = [&](int k0) { // zero padded
 #pragma unroll
-        for(int e = tid; e < GT * GK; e += 256)
+        for(int t = 0; t < PT; ++t)
         {
-            int i, k;
-            T v;
+            const int e = tid + 256 * t;
             if(!TRANSA)
             {
-                i = e % GT;
-                k = e / GT;
-                v = (i0 + i < M && k0 + k < K) ? A[(i0 + i) + int64_t(k0 + k) * lda] : T(0);
+                const int i = i0 + e % GT, k = k0 + e / GT;
+                ra[t] = (i < M && k < K) ? A[i + int64_t(k) * lda] : T(0);
             }
             else
             {
-                k = e % GK;
-                i = e / GK;
-                v = (i0 + i < M && k0 + k < K) ? A[(k0 + k) + int64_t(i0 + i) * lda] : T(0);
+                const int k = k0 + e % GK, i = i0 + e / GK;
+                ra[t] = (i < M && k < K) ? A[k + int64_t(i) * lda] : T(0);
             }
-            sA[k][i] = v;
-            const int kb = e % GK, jb = e / GK;
-            sB[kb][jb] = (k0 + kb < K && j0 + jb < N) ? Bm[(k0 + kb) + int64_t(j0 + jb) * ldb]
-                                                      : T(0);
+            const int kb = k0 + e % GK, jb = j0 + e / GK;
+            rb[t] = (kb < K && jb < N) ? Bm[kb + int64_t(jb) * ldb] : T(0);
+        }
+    };
+    load(0);
+    int buf = 0;
+    for(int k0 = 0; k0 < K; k0 += GK, buf ^= 1)
+    {
+#pragma unroll
+        for(int t = 0; t < PT; ++t)
+        {
+            const int e = tid + 256 * t;
+            sA[buf][TRANSA ? (e / GK) * SC + e % GK : (e / GT) * SR + e % GT] = ra[t];
+            sB[buf][(e / GK) * SC + e % GK] = rb[t];
         }
         __syncthreads();
+        if(k0 + GK < K) // uniform
+            load(k0 + GK);
 #pragma unroll
         for(int kk = 0; kk < GK; kk += 4)
         {
             T a[2], bv[2];
+            const int k = kk + lane / 16;
 #pragma unroll
             for(int s = 0; s < 2; ++s)
-                a[s] = sA[kk + lane / 16][wi + s * 16 + lane % 16];
+            {
+                const int i = wi + s * 16 + lane % 16;
+                a[s] = sA[buf][TRANSA ? i * SC + k : k * SR + i];
+            }
 #pragma unroll
             for(int t = 0; t < 2; ++t)
-                bv[t] = sB[kk + lane / 16][wj + t * 16 + lane % 16];
+                bv[t] = sB[buf][(wj + t * 16 + lane % 16) * SC + k];
 #pragma unroll
             for(int s = 0; s < 2; ++s)
 #pragma unroll
                 for(int t = 0; t < 2; ++t)
-                    acc[s][t] = mfma16<T>::run(a[s], bv[t], acc[s][t]);
+                    acc[s][t] = M_::run(bv[t], a[s], acc[s][t]);
         }
-        __syncthreads();
     }
 
 #pragma unroll
     for(int s = 0; s < 2; ++s)
+    {
+        const int i = i0 + wi + s * 16 + lane % 16;
 #pragma unroll
         for(int t = 0; t < 2; ++t)
-        {
-            const int j = j0 + wj + t * 16 + lane % 16;
 #pragma unroll
             for(int r = 0; r < 4; ++r)
             {
-                const int i = i0 + wi + s * 16 + mfma16<T>::row(lane, r);
+                const int j = j0 + wj + t * 16 + M_::row(lane, r);
                 if(i < M && j < N)
                 {
                     T& c = C[i + int64_t(j) * ldc];
                     c = c - acc[s][t][r];
                 }
             }
-        }
+    }
 }
 
 template <typename T>
@@ -424,16 +466,28 @@ static rocblas_status gemm_sub(hipStream_t stream, bool transA, int M, int N, in
 {
     if(M <= 0 || N <= 0 || K <= 0 || bc <= 0)
         return rocblas_status_success;
-    for(int64_t b0 = 0; b0 < bc; b0 += MAX_GRID_YZ)
+    const int tm = ceil_div(M, GT), tn = ceil_div(N, GT);
+    const int64_t tiles = int64_t(tm) * tn;
+    // one launch per 2^30 workgroups at most (whole groups of XCDS matrices)
+    const int64_t most = (int64_t(1) << 30) / tiles / XCDS * XCDS;
+    const int64_t step = most > 0 ? most : 1;
+    for(int64_t b0 = 0; b0 < bc; b0 += step)
     {
-        const int nb = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);
-        dim3 grid(ceil_div(M, GT), ceil_div(N, GT), nb);
+        const int nb = int((bc - b0) < step ? (bc - b0) : step);
+        const int64_t wgs = tiles * (nb >= XCDS ? int64_t(ceil_div(nb, XCDS)) * XCDS : nb);
+        auto from = [&](Batch<T> X) {
+            return X.ptrs ? Batch<T>{nullptr, X.ptrs + b0, 0}
+                          : Batch<T>{X.base + b0 * X.stride, nullptr, X.stride};
+        };
+        const int* sk = skip ? skip + b0 : nullptr;
         if(transA)
-            hipLaunchKernelGGL((gemm_sub_kernel<T, true>), grid, dim3(256), 0, stream, M, N, K, A,
-                               offA, lda, B, offB, ldb, C, offC, ldc, skip, b0);
+            hipLaunchKernelGGL((gemm_sub_kernel<T, true>), dim3(unsigned(wgs)), dim3(256), 0,
+                               stream, M, N, K, from(A), offA, lda, from(B), offB, ldb, from(C),
+                               offC, ldc, sk, nb, tm, tn);
         else
-            hipLaunchKernelGGL((gemm_sub_kernel<T, false>), grid, dim3(256), 0, stream, M, N, K,
-                               A, offA, lda, B, offB, ldb, C, offC, ldc, skip, b0);
+            hipLaunchKernelGGL((gemm_sub_kernel<T, false>), dim3(unsigned(wgs)), dim3(256), 0,
+                               stream, M, N, K, from(A), offA, lda, from(B), offB, ldb, from(C),
+                               offC, ldc, sk, nb, tm, tn);
         RSA_LAUNCH_CHECK();
     }
     return rocblas_status_success;
@@ -448,43 +502,61 @@ rocblas_status getrf_blocked(hipStream_t stream, int m, int n, Batch<T> A, int l
     if(st != rocblas_status_success)
         return st;
     const int kmax = m < n ? m : n;
-    for(int j = 0, jb = 0; j < kmax; j += jb)
+    // C[r0:m, r0:jend] -= A[r0:m, j:r0] A[j:r0, r0:jend]
+    auto update = [&](int j, int r0, int jend) {
+        return gemm_sub<T>(stream, false, m - r0, jend - r0, r0 - j, A, r0 + int64_t(j) * lda, lda,
+                           A, j + int64_t(r0) * lda, lda, A, r0 + int64_t(r0) * lda, lda, bc,
+                           nullptr);
+    };
+    for(int o0 = 0, nb = 0; o0 < kmax; o0 += nb)
     {
-        // panels that fit the registers of one workgroup; taller ones are
-        // factored in global memory
-        const int wreg = panel_reg_width<T>(m - j, lda);
-        const int width = wreg ? wreg : PANEL_NB;
-        jb = (kmax - j) < width ? (kmax - j) : width;
-        const int r0 = j + jb;
-        if(wreg)
+        if(panel_reg_width<T>(m - o0, lda))
         {
-            st = panel_reg<T>(stream, m, A, lda, ipiv, strideP, info, j, jb, 0, n, bc, pivot);
+            // a block column of OUTER_NB columns: its panels in registers,
+            // each applied to the rest of the block only, then the block to
+            // the rest of the matrix, so the trailing matrix is read and
+            // written once per OUTER_NB columns
+            nb = (kmax - o0) < OUTER_NB ? (kmax - o0) : OUTER_NB;
+            const int oend = o0 + nb;
+            for(int j = o0, jb = 0; j < oend; j += jb)
+            {
+                const int w = panel_reg_width<T>(m - j, lda);
+                jb = (oend - j) < w ? (oend - j) : w;
+                st = panel_reg<T>(stream, m, A, lda, ipiv, strideP, info, j, jb, o0, oend, bc,
+                                  pivot);
+                if(st == rocblas_status_success)
+                    st = update(j, j + jb, oend);
+                if(st != rocblas_status_success)
+                    return st;
+            }
+            st = outer_apply<T>(stream, n, A, lda, ipiv, strideP, o0, nb, bc, pivot);
+            if(st == rocblas_status_success)
+                st = update(o0, oend, n);
             if(st != rocblas_status_success)
                 return st;
+            continue;
         }
-        else if(pivot)
+        // panels too tall for the registers, factored in global memory
+        nb = (kmax - o0) < PANEL_NB ? (kmax - o0) : PANEL_NB;
+        const int r0 = o0 + nb;
+        if(pivot)
             hipLaunchKernelGGL((panel_kernel<T, true>), dim3(bc), dim3(PANEL_THREADS), 0, stream, m,
-                               n, A, lda, ipiv, strideP, info, j, jb);
+                               n, A, lda, ipiv, strideP, info, o0, nb);
         else
             hipLaunchKernelGGL((panel_kernel<T, false>), dim3(bc), dim3(PANEL_THREADS), 0, stream,
-                               m, n, A, lda, ipiv, strideP, info, j, jb);
+                               m, n, A, lda, ipiv, strideP, info, o0, nb);
         RSA_LAUNCH_CHECK();
-        if(r0 < n && !wreg)
+        if(r0 < n)
             for(int64_t b0 = 0; b0 < bc; b0 += MAX_GRID_YZ)
             {
-                const int nb = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);
-                hipLaunchKernelGGL((u12_kernel<T>), dim3(ceil_div(n - r0, 64), nb), dim3(64), 0,
-                                   stream, n, A, lda, j, jb, b0);
+                const int cnt = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);
+                hipLaunchKernelGGL((u12_kernel<T>), dim3(ceil_div(n - r0, 64), cnt), dim3(64), 0,
+                                   stream, n, A, lda, o0, nb, b0);
                 RSA_LAUNCH_CHECK();
             }
-        if(r0 < m && r0 < n)
-        {
-            st = gemm_sub<T>(stream, false, m - r0, n - r0, jb, A, r0 + int64_t(j) * lda, lda, A,
-                             j + int64_t(r0) * lda, lda, A, r0 + int64_t(r0) * lda, lda, bc,
-                             nullptr);
-            if(st != rocblas_status_success)
-                return st;
-        }
+        st = update(o0, r0, n);
+        if(st != rocblas_status_success)
+            return st;
     }
     return rocblas_status_success;
 }

@@ -18,6 +18,7 @@
 // barriers, took 303 us for a 32-column FP64 panel of n = 1024 on average
 // (64 matrices); this kernel takes 76 us there.
 #include "internal.hpp"
+#include "mfma.hpp"
 
 #include <climits>
 
@@ -68,6 +69,42 @@ __device__ __forceinline__ int few_argmax(float key, int idx)
     return few_min<NW>((cand && u == mu) ? idx : 0x7fffffff);
 }
 
+// x <- L^-1 x for a unit lower triangular L (N x N, column-major in LDS): four
+// lanes per column, lane q & 3 = s holding rows 4 t + s in x[t].  The solved
+// x_k reaches the other three lanes by a DPP broadcast, so a column takes N
+// steps of at most N/4 fused multiply-adds (a thread per column: up to N - 1).
+template <typename T, int N, int K = 0>
+__device__ __forceinline__ void quad_solve_unit_lower(const T* L, int lane, T (&x)[N / 4])
+{
+    if constexpr(K < N - 1)
+    {
+        if constexpr(K % 4 == 0)
+        {
+            // an empty asm tied to x: the optimiser takes the address of L
+            // as computed from it, so not all of L is loaded ahead (and
+            // spilled)
+            uint32_t lo = 0;
+            asm volatile("" : "+v"(lo) : "v"(x[K / 4]));
+            L += lo;
+        }
+        T xk;
+        if constexpr(sizeof(T) == 8)
+            xk = dpp_mov_d<0x55 * (K % 4)>(x[K / 4]);
+        else
+            xk = __int_as_float(dpp_mov<0x55 * (K % 4)>(__float_as_int(x[K / 4])));
+        const T* col = L + K * N + (lane & 3);
+        if constexpr(K % 4 < 3)
+        {
+            const T y = fma_t(-col[K / 4 * 4], xk, x[K / 4]);
+            x[K / 4] = (lane & 3) > K % 4 ? y : x[K / 4];
+        }
+#pragma unroll
+        for(int t = K / 4 + 1; t < N / 4; ++t)
+            x[t] = fma_t(-col[4 * t], xk, x[t]);
+        quad_solve_unit_lower<T, N, K + 1>(L, lane, x);
+    }
+}
+
 // m - j0 <= R * NT rows, jb <= W columns; W * lda * sizeof(T) below 2^31.
 // Row indices inside the kernel count from j0.
 template <typename T, int W, int R, int NT, bool PIVOT>
@@ -86,9 +123,6 @@ __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, in
     __shared__ int slab[2][NW];
     __shared__ __align__(16) T sL[W * W]; // L11 by columns
     __shared__ int s_swap[W]; // row interchanged with row k (itself: none)
-    __shared__ int s_pos[2 * W]; // rows touched by the interchanges
-    __shared__ int s_src[2 * W]; // row whose entries end at s_pos[q]
-    __shared__ int s_cnt;
 
     const int64_t b = blockIdx.x;
     T* A = AA[b] + j0;
@@ -255,108 +289,221 @@ __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, in
     if(PIVOT)
     {
         // the interchanges composed into one map of at most 2 jb rows: lane q
-        // of the first wavefront keeps slot q (row pos, source src); ballots
-        // find a row's slot, a new row takes the next free one
-        if(wid == 0)
+        // follows row q, lane W + q the row that row q was interchanged with,
+        // back through the interchanges to where its entries are now
+        const int q = lane & (2 * W - 1);
+        const int pos = q < W ? q : (q - W < jb ? s_swap[q - W] : -1);
+        int src = pos;
+        for(int k = jb - 1; k >= 0; --k)
         {
-            int pos = -1, src = -1, cnt = 0;
-            for(int k = 0; k < jb; ++k)
-            {
-                const int r2 = __builtin_amdgcn_readfirstlane(s_swap[k]);
-                if(r2 == k) // uniform
-                    continue;
-                int qs[2];
-#pragma unroll
-                for(int h = 0; h < 2; ++h)
-                {
-                    const int row = h ? r2 : k;
-                    const uint64_t hit = __builtin_amdgcn_ballot_w64(pos == row);
-                    int q = hit ? __builtin_ffsll(hit) - 1 : cnt;
-                    if(!hit)
-                    {
-                        if(lane == q)
-                        {
-                            pos = row;
-                            src = row;
-                        }
-                        ++cnt;
-                    }
-                    qs[h] = q;
-                }
-                const int sa = __builtin_amdgcn_readlane(src, qs[0]);
-                const int sb = __builtin_amdgcn_readlane(src, qs[1]);
-                if(lane == qs[0])
-                    src = sb;
-                if(lane == qs[1])
-                    src = sa;
-            }
-            if(lane < cnt)
-            {
-                s_pos[lane] = pos;
-                s_src[lane] = src;
-            }
-            if(lane == 0)
-                s_cnt = cnt;
+            const int p = s_swap[k];
+            src = src == k ? p : (src == p ? k : src);
         }
-        __syncthreads();
-        // one wavefront per column, lane q moving the entry of slot q; the
-        // loads of four columns in flight
-        const bool mine = lane < s_cnt;
-        const int pos = mine ? s_pos[lane] : 0, src = mine ? s_src[lane] : 0;
-        constexpr int UC = 4;
-        for(int e0 = wid * UC; e0 < nout; e0 += NW * UC)
+        // rows of the second half below jb are in the first; a row met twice
+        // there is moved twice, the same entry to the same place
+        const bool mine = (q < W ? q < jb : pos >= jb) && src != pos;
+        // 64 / (2 W) columns per wavefront, the loads of four such groups in
+        // flight
+        constexpr int UC = 4, CPW = 64 / (2 * W);
+        for(int e0 = wid * UC * CPW + lane / (2 * W); e0 < nout; e0 += NW * UC * CPW)
         {
             T x[UC];
+            auto at = [&](int row, int u) -> T& {
+                const int e = o0 + e0 + u * CPW;
+                return A[row + int64_t(e < j0 ? e : e + jb) * lda];
+            };
 #pragma unroll
             for(int u = 0; u < UC; ++u)
-            {
-                const int j = o0 + e0 + u < j0 ? o0 + e0 + u : o0 + e0 + u + jb;
-                x[u] = (mine && e0 + u < nout) ? A[src + int64_t(j) * lda] : T(0);
-            }
+                x[u] = (mine && e0 + u * CPW < nout) ? at(src, u) : T(0);
 #pragma unroll
             for(int u = 0; u < UC; ++u)
-            {
-                const int j = o0 + e0 + u < j0 ? o0 + e0 + u : o0 + e0 + u + jb;
-                if(mine && e0 + u < nout)
-                    A[pos + int64_t(j) * lda] = x[u];
-            }
+                if(mine && e0 + u * CPW < nout)
+                    at(pos, u) = x[u];
         }
     }
     __syncthreads(); // the interchanged rows are written, L11 is in LDS
 
-    // U12 = L11^-1 A12, one thread per column.  L11 is read through an offset
-    // that the optimiser must take as computed from x[k] every two columns
-    // (an empty asm tied to x[k]), so its entries are not all loaded ahead of
-    // the substitution (and spilled).
-    for(int j = j0 + jb + tid; j < oend; j += NT)
+    // U12 = L11^-1 A12, four lanes per column
+    for(int j = j0 + jb + tid / 4; j < oend; j += NT / 4)
     {
-        T* col = A + int64_t(j) * lda;
-        T x[W];
+        T* col = A + int64_t(j) * lda + (lane & 3);
+        T x[W / 4];
 #pragma unroll
-        for(int i = 0; i < W; ++i)
-            x[i] = i < jb ? col[i] : T(0);
-        const T* L = sL;
+        for(int t = 0; t < W / 4; ++t)
+            x[t] = 4 * t + (lane & 3) < jb ? col[4 * t] : T(0);
+        quad_solve_unit_lower<T, W>(sL, lane, x);
 #pragma unroll
-        for(int k = 0; k < W; ++k)
-        {
-            if(k < jb) // uniform
-            {
-                if((k & 1) == 0)
-                {
-                    uint32_t lo = 0;
-                    asm volatile("" : "+v"(lo) : "v"(x[k]));
-                    L = sL + lo;
-                }
-#pragma unroll
-                for(int i = k + 1; i < W; ++i)
-                    x[i] = fma_t(-L[i + k * W], x[k], x[i]);
-            }
-        }
-#pragma unroll
-        for(int i = 0; i < W; ++i)
-            if(i < jb)
-                col[i] = x[i];
+        for(int t = 0; t < W / 4; ++t)
+            if(4 * t + (lane & 3) < jb)
+                col[4 * t] = x[t];
     }
+}
+
+// ------------------------------------------------------------ outer block
+// The finished block column [o0, o0 + nb), nb <= OUTER_NB, applied to the
+// columns outside it: its interchanges to all of them, and U12 = L11^-1 A12
+// for those right of it.  64 columns per workgroup; the left_chunks first
+// workgroups of a matrix take the columns left of the block.
+//
+// Bound by latency and by the scattered rows of the interchanges (one cache
+// line per row and column), so one block's interchanges are composed into a
+// map and applied once, not panel by panel.  The nb top rows stay in LDS from
+// the interchange to the solve: 32-row diagonal blocks by substitution (four
+// lanes per column), the rows below by matrix-core products.  Each wavefront
+// owns 16 columns from then on, so the solve has no barrier.
+constexpr int OUTER_COLS = 64;
+
+template <typename T, bool PIVOT>
+__global__ __launch_bounds__(256, 1) void outer_apply_kernel(int n, Batch<T> AA, int lda,
+                                                             const int* __restrict__ ipivA,
+                                                             int64_t strideP, int o0, int nb,
+                                                             int left_chunks, int64_t boff)
+{
+    using M = mfma16<T>;
+    constexpr int LS = OUTER_NB + 1; // column stride of the right-hand sides in LDS
+    constexpr int DB = 32; // diagonal block
+    constexpr int UC = 16; // columns in flight
+    __shared__ T sB[OUTER_COLS * LS];
+    __shared__ __align__(16) T sL[OUTER_NB / DB][DB * DB];
+    __shared__ int s_piv[OUTER_NB];
+
+    const int64_t b = blockIdx.y + boff;
+    T* A = AA[b] + o0;
+    const int tid = threadIdx.x;
+    const int wid = tid / 64;
+    const int lane = tid % 64;
+    const int chunk = blockIdx.x;
+    const bool right = chunk >= left_chunks; // uniform
+    const int c0 = right ? o0 + nb + (chunk - left_chunks) * OUTER_COLS : chunk * OUTER_COLS;
+    const int nc = (right ? n : o0) - c0 < OUTER_COLS ? (right ? n : o0) - c0 : OUTER_COLS;
+
+    if(PIVOT && tid < nb)
+        s_piv[tid] = ipivA[b * strideP + o0 + tid] - 1 - o0;
+    if(right)
+    {
+#pragma unroll
+        for(int d = 0; d < OUTER_NB / DB; ++d)
+            for(int e = tid; e < DB * DB; e += 256)
+            {
+                const int i = DB * d + e % DB, k = DB * d + e / DB;
+                sL[d][e] = (i < nb && k < nb) ? A[i + int64_t(o0 + k) * lda] : T(0);
+            }
+    }
+    __syncthreads();
+
+    // threads 0..127 follow the rows of the block, threads 128..255 the rows
+    // they were interchanged with, back to where their entries are now (a row
+    // below the block met twice is moved twice, the same entry to the same
+    // place)
+    int pos = tid < OUTER_NB ? tid : -1, src = pos;
+    if(PIVOT)
+    {
+        if(tid >= OUTER_NB && tid - OUTER_NB < nb)
+            pos = s_piv[tid - OUTER_NB];
+        src = pos;
+        for(int k = nb - 1; k >= 0; --k)
+        {
+            const int p = s_piv[k];
+            src = src == k ? p : (src == p ? k : src);
+        }
+    }
+    const bool top = tid < OUTER_NB;
+    const bool load = top ? (tid < nb && (right || src != pos)) : (pos >= nb && src != pos);
+    for(int cb = 0; cb < nc; cb += UC) // uniform
+    {
+        T x[UC];
+#pragma unroll
+        for(int u = 0; u < UC; ++u)
+            x[u] = (load && cb + u < nc) ? A[src + int64_t(c0 + cb + u) * lda] : T(0);
+        __syncthreads(); // the loads of these columns are done
+        if(right && top)
+        {
+#pragma unroll
+            for(int u = 0; u < UC; ++u)
+                sB[(cb + u) * LS + tid] = x[u];
+        }
+        else if(load)
+        {
+#pragma unroll
+            for(int u = 0; u < UC; ++u)
+                if(cb + u < nc)
+                    A[pos + int64_t(c0 + cb + u) * lda] = x[u];
+        }
+    }
+    if(!right)
+        return;
+    __syncthreads();
+
+    if(16 * wid >= nc) // uniform in the wavefront
+        return;
+    T* colB = sB + 16 * wid * LS; // this wavefront's 16 columns
+#pragma unroll
+    for(int d = 0; d < OUTER_NB / DB; ++d)
+    {
+        if(DB * d < nb) // uniform
+        {
+            {
+                T x[DB / 4];
+                T* xp = colB + (lane >> 2) * LS + DB * d + (lane & 3);
+#pragma unroll
+                for(int t = 0; t < DB / 4; ++t)
+                    x[t] = xp[4 * t];
+                quad_solve_unit_lower<T, DB>(sL[d], lane, x);
+#pragma unroll
+                for(int t = 0; t < DB / 4; ++t)
+                    xp[4 * t] = x[t];
+            }
+            wave_sync();
+            // rows below the diagonal block, 16 at a time
+            T bv[DB / 4];
+#pragma unroll
+            for(int ks = 0; ks < DB / 4; ++ks)
+                bv[ks] = colB[(lane & 15) * LS + DB * d + 4 * ks + (lane >> 4)];
+            for(int i0 = DB * (d + 1); i0 < nb; i0 += 16) // uniform
+            {
+                const int i = i0 + (lane & 15);
+                T av[DB / 4];
+#pragma unroll
+                for(int ks = 0; ks < DB / 4; ++ks)
+                    av[ks] = i < nb ? A[i + int64_t(o0 + DB * d + 4 * ks + (lane >> 4)) * lda]
+                                    : T(0);
+                typename M::acc_t acc = {0, 0, 0, 0};
+#pragma unroll
+                for(int ks = 0; ks < DB / 4; ++ks)
+                    acc = M::run(av[ks], bv[ks], acc);
+#pragma unroll
+                for(int r = 0; r < 4; ++r)
+                    colB[(lane & 15) * LS + i0 + M::row(lane, r)] -= acc[r];
+            }
+            wave_sync();
+        }
+    }
+    for(int c = 0; c < 16; ++c)
+        if(16 * wid + c < nc) // uniform
+            for(int i = lane; i < nb; i += 64)
+                A[i + int64_t(c0 + 16 * wid + c) * lda] = colB[c * LS + i];
+}
+
+template <typename T>
+rocblas_status outer_apply(hipStream_t stream, int n, Batch<T> A, int lda, const int* ipiv,
+                           int64_t strideP, int o0, int nb, int bc, bool pivot)
+{
+    const int left = pivot ? ceil_div(o0, OUTER_COLS) : 0;
+    const int chunks = left + ceil_div(n - o0 - nb, OUTER_COLS);
+    if(chunks <= 0)
+        return rocblas_status_success;
+    for(int64_t b0 = 0; b0 < bc; b0 += 65535)
+    {
+        const int cnt = int((bc - b0) < 65535 ? (bc - b0) : 65535);
+        if(pivot)
+            hipLaunchKernelGGL((outer_apply_kernel<T, true>), dim3(chunks, cnt), dim3(256), 0,
+                               stream, n, A, lda, ipiv, strideP, o0, nb, left, b0);
+        else
+            hipLaunchKernelGGL((outer_apply_kernel<T, false>), dim3(chunks, cnt), dim3(256), 0,
+                               stream, n, A, lda, ipiv, strideP, o0, nb, left, b0);
+        RSA_LAUNCH_CHECK();
+    }
+    return rocblas_status_success;
 }
 
 // Panel width for `rows` rows: the register file of one CU holds 512 threads
@@ -411,6 +558,8 @@ rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ip
 
 #define RSA_PANEL_INST(T)                                                                       \
     template int panel_reg_width<T>(int, int);                                                  \
+    template rocblas_status outer_apply<T>(hipStream_t, int, Batch<T>, int, const int*, int64_t, \
+                                           int, int, int, bool);                                \
     template rocblas_status panel_reg<T>(hipStream_t, int, Batch<T>, int, int*, int64_t, int*,  \
                                          int, int, int, int, int, bool);
 RSA_PANEL_INST(float)

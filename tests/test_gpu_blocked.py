@@ -45,15 +45,21 @@ def test_one_panel_special_values(torch_gpu, handle, m, dtype):
     np.testing.assert_array_equal(Ad.cpu().numpy(), Ao)
 
 
-@pytest.mark.parametrize("m,n", [(m, 40) for m in PANEL_ROWS[1:]] + [(16, 700), (90, 333), (513, 513)])
+# more columns than one outer block of 128: its last partial block, columns left and right of
+# it in whole and partial chunks of 64, matrices dealt to the XCDs in groups of eight
+OUTER = [(16, 700, 3), (90, 333, 9), (128, 129, 8), (513, 513, 3), (640, 640, 2), (1100, 321, 17),
+         (260, 1000, 3)]
+
+
+@pytest.mark.parametrize("m,n,bc", [(m, 40, 3) for m in PANEL_ROWS[1:]] + OUTER)
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-def test_panels_and_updates(torch_gpu, handle, m, n, dtype):
+def test_panels_and_updates(torch_gpu, handle, m, n, bc, dtype):
     """Several panels with a partial last one, lda > m: pivots equal where the
     oracle finds them unambiguous, factors within 10 min(m,n) eps there, and
     P A = L U for every matrix; the padding rows are untouched."""
-    print(f"getrf m={m} n={n} {dtype.__name__}", flush=True)
+    print(f"getrf m={m} n={n} bc={bc} {dtype.__name__}", flush=True)
     g = np.random.default_rng(m * 31 + n)
-    bc, lda = 3, m + 3
+    lda = m + 3
     A0 = g.uniform(-1, 1, size=(bc, n, lda)).astype(dtype)
     Ao = np.ascontiguousarray(A0[:, :, :m])
     ip_o, in_o, gap = oracle.getf2(Ao, m, with_gap=True)
@@ -73,7 +79,7 @@ def test_panels_and_updates(torch_gpu, handle, m, n, dtype):
     assert be.max() < 10.0, be
 
 
-@pytest.mark.parametrize("m,n", [(300, 100), (1100, 70), (2500, 24)])
+@pytest.mark.parametrize("m,n", [(300, 100), (1100, 70), (2500, 24), (530, 530)])
 def test_panels_without_pivoting(torch_gpu, handle, m, n):
     g = np.random.default_rng(m)
     A0 = g.uniform(-1, 1, size=(2, n, m))
