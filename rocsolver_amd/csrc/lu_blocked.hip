@@ -12,10 +12,12 @@
 //      rows), and u12_kernel, one thread per column right of the panel.
 //   2. gemm_sub_kernel: A22 -= L21 * U12 on MFMA (v_mfma_f64_16x16x4f64 /
 //      v_mfma_f32_16x16x4f32), 64x64 tiles.
-// getrs (roclapack_getrs.hpp:117-150): laswp, then for each 64-row diagonal
-// block a substitution kernel followed by an MFMA GEMM update of the rest.
+// getrs (roclapack_getrs.hpp:117-150): the interchanges, then each triangle
+// in 128-row tiles, one launch per tile (update by the tile before, then its
+// own solve).
 #include "internal.hpp"
 #include "mfma.hpp"
+#include "quad_solve.hpp"
 
 #include <climits>
 
@@ -24,7 +26,6 @@ namespace rsa
 
 constexpr int PANEL_NB = 32; // width of the panel in global memory
 constexpr int PANEL_THREADS = 512;
-constexpr int TRSM_NB = 64; // getrs diagonal block
 constexpr int64_t MAX_GRID_YZ = 65535; // grid y/z limit: larger batches are launched in chunks
 
 // ------------------------------------------------------------------ info
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(64) void u12_kernel(int n, Batch<T> AA, int lda, in
 }
 
 // ------------------------------------------------------------------ GEMM
-// C[M x N] -= op(A)[M x K] * B[K x N], column-major, one 64x64 tile per
+// C[M x N] -= A[M x K] * B[K x N], column-major, one 64x64 tile per
 // workgroup (4 waves, each 32x32 = 2x2 MFMA 16x16 blocks).  K goes through
 // LDS in double-buffered chunks of 16, one barrier a chunk: the next chunk's
 // global loads are in flight during this chunk's matrix instructions.  The
@@ -330,7 +331,7 @@ constexpr int GT = 64; // tile
 constexpr int GK = 16; // k chunk
 constexpr int XCDS = 8;
 
-template <typename T, bool TRANSA>
+template <typename T>
 __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batch<T> AA,
                                                        int64_t offA, int lda, Batch<T> BB,
                                                        int64_t offB, int ldb, Batch<T> CC,
@@ -345,7 +346,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
     constexpr int SR = GT + 16; // [k][i]
     constexpr int SC = GK + 1; // [j][k]
     constexpr int PT = GT * GK / 256; // entries of each operand per thread and chunk
-    __shared__ T sA[2][TRANSA ? GT * SC : GK * SR];
+    __shared__ T sA[2][GK * SR];
     __shared__ T sB[2][GT * SC];
 
     const unsigned tiles = unsigned(tm) * unsigned(tn);
@@ -390,16 +391,8 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
         for(int t = 0; t < PT; ++t)
         {
             const int e = tid + 256 * t;
-            if(!TRANSA)
-            {
-                const int i = i0 + e % GT, k = k0 + e / GT;
-                ra[t] = (i < M && k < K) ? A[i + int64_t(k) * lda] : T(0);
-            }
-            else
-            {
-                const int k = k0 + e % GK, i = i0 + e / GK;
-                ra[t] = (i < M && k < K) ? A[k + int64_t(i) * lda] : T(0);
-            }
+            const int i = i0 + e % GT, k = k0 + e / GT;
+            ra[t] = (i < M && k < K) ? A[i + int64_t(k) * lda] : T(0);
             const int kb = k0 + e % GK, jb = j0 + e / GK;
             rb[t] = (kb < K && jb < N) ? Bm[kb + int64_t(jb) * ldb] : T(0);
         }
@@ -412,7 +405,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
         for(int t = 0; t < PT; ++t)
         {
             const int e = tid + 256 * t;
-            sA[buf][TRANSA ? (e / GK) * SC + e % GK : (e / GT) * SR + e % GT] = ra[t];
+            sA[buf][(e / GT) * SR + e % GT] = ra[t];
             sB[buf][(e / GK) * SC + e % GK] = rb[t];
         }
         __syncthreads();
@@ -427,7 +420,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
             for(int s = 0; s < 2; ++s)
             {
                 const int i = wi + s * 16 + lane % 16;
-                a[s] = sA[buf][TRANSA ? i * SC + k : k * SR + i];
+                a[s] = sA[buf][k * SR + i];
             }
 #pragma unroll
             for(int t = 0; t < 2; ++t)
@@ -460,7 +453,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
 }
 
 template <typename T>
-static rocblas_status gemm_sub(hipStream_t stream, bool transA, int M, int N, int K, Batch<T> A,
+static rocblas_status gemm_sub(hipStream_t stream, int M, int N, int K, Batch<T> A,
                                int64_t offA, int lda, Batch<T> B, int64_t offB, int ldb,
                                Batch<T> C, int64_t offC, int ldc, int bc, const int* skip)
 {
@@ -480,14 +473,9 @@ static rocblas_status gemm_sub(hipStream_t stream, bool transA, int M, int N, in
                           : Batch<T>{X.base + b0 * X.stride, nullptr, X.stride};
         };
         const int* sk = skip ? skip + b0 : nullptr;
-        if(transA)
-            hipLaunchKernelGGL((gemm_sub_kernel<T, true>), dim3(unsigned(wgs)), dim3(256), 0,
-                               stream, M, N, K, from(A), offA, lda, from(B), offB, ldb, from(C),
-                               offC, ldc, sk, nb, tm, tn);
-        else
-            hipLaunchKernelGGL((gemm_sub_kernel<T, false>), dim3(unsigned(wgs)), dim3(256), 0,
-                               stream, M, N, K, from(A), offA, lda, from(B), offB, ldb, from(C),
-                               offC, ldc, sk, nb, tm, tn);
+        hipLaunchKernelGGL((gemm_sub_kernel<T>), dim3(unsigned(wgs)), dim3(256), 0, stream, M, N, K,
+                           from(A), offA, lda, from(B), offB, ldb, from(C), offC, ldc, sk, nb, tm,
+                           tn);
         RSA_LAUNCH_CHECK();
     }
     return rocblas_status_success;
@@ -504,7 +492,7 @@ rocblas_status getrf_blocked(hipStream_t stream, int m, int n, Batch<T> A, int l
     const int kmax = m < n ? m : n;
     // C[r0:m, r0:jend] -= A[r0:m, j:r0] A[j:r0, r0:jend]
     auto update = [&](int j, int r0, int jend) {
-        return gemm_sub<T>(stream, false, m - r0, jend - r0, r0 - j, A, r0 + int64_t(j) * lda, lda,
+        return gemm_sub<T>(stream, m - r0, jend - r0, r0 - j, A, r0 + int64_t(j) * lda, lda,
                            A, j + int64_t(r0) * lda, lda, A, r0 + int64_t(r0) * lda, lda, bc,
                            nullptr);
     };
@@ -620,118 +608,343 @@ rocblas_status laswp(hipStream_t stream, int ncols, Batch<T> A, int lda, int k1,
     return rocblas_status_success;
 }
 
-// ------------------------------------------------------------ substitution
-// Solves one diagonal block (rows r0..r0+rb) of the LU against all right-hand
-// sides, one thread per column of B, block in LDS.  kind: 0 = L unit lower
-// (forward), 1 = U non-unit upper (backward), 2 = U^T (forward, non-unit),
-// 3 = L^T (backward, unit).  Column-oriented order with true division, as
-// the reference substitution kernels.
-template <typename T, int KIND>
-__global__ __launch_bounds__(256) void trsm_block_kernel(int r0, int rb, int nrhs, Batch<T> AA,
-                                                         int lda, Batch<T> BB, int ldb,
-                                                         const int* __restrict__ skip,
-                                                         int64_t boff)
+// --------------------------------------------------------------- row order
+// B <- P B (or with inverse, P^T B) for the interchanges of ipiv (1-based,
+// LAPACK order; a pivot outside [1, n] is ignored), n <= 1024 R rows.
+//
+// The interchanges are composed in blocks of 64: a wavefront follows the 64
+// rows of a block and the 64 rows they are interchanged with through the
+// block's steps, and one wavefront then applies the blocks' maps in order to
+// a table of the rows in LDS.  Every column is gathered through the table.
+// (Following every row through all n interchanges took 161 us at n = 2000,
+// and laswp_kernel, two dependent global accesses per row, 154 us; this
+// kernel takes 17 us there.)
+constexpr int PERM_THREADS = 1024;
+constexpr int PERM_COLS = 8; // columns per workgroup
+
+template <typename T, int R>
+__global__ __launch_bounds__(PERM_THREADS) void permute_rows_kernel(
+    int n, int nrhs, Batch<T> BB, int ldb, const int* __restrict__ ipivA, int64_t strideP,
+    int inverse, const int* __restrict__ skip, int64_t boff)
 {
-    __shared__ T sD[TRSM_NB * TRSM_NB];
+    constexpr int ROWS = PERM_THREADS * R;
+    __shared__ unsigned short s_row[ROWS]; // row now at each position
+    __shared__ unsigned short s_pos[ROWS]; // block maps: the rows interchanged with,
+    __shared__ unsigned short s_src[2][ROWS]; // and where both kinds come from
     const int64_t b = blockIdx.y + boff;
+    if(skip && skip[b] != 0)
+        return;
+    T* Bm = BB[b];
+    const int* ipiv = ipivA + b * strideP;
+    const int tid = threadIdx.x;
+    const int lane = tid % 64;
+    const int nblk = (n + 63) / 64;
+    for(int i = tid; i < ROWS; i += PERM_THREADS)
+        s_row[i] = (unsigned short)i;
+    for(int blk = tid / 64; blk < nblk; blk += PERM_THREADS / 64) // one wavefront per block
+    {
+        const int base = 64 * blk, i = base + lane;
+        int p = i < n ? ipiv[i] - 1 : i;
+        p = (p >= 0 && p < n) ? p : i;
+        int s0 = i, s1 = p;
+#pragma unroll 8
+        for(int e = 0; e < 64; ++e)
+        {
+            // back through the block's steps, the last one applied first
+            const int k = inverse ? e : 63 - e;
+            const int row = base + k;
+            const int q = __builtin_amdgcn_readlane(p, k);
+            s0 = s0 == row ? q : (s0 == q ? row : s0);
+            s1 = s1 == row ? q : (s1 == q ? row : s1);
+        }
+        s_src[0][i] = (unsigned short)s0;
+        // a partner inside the block is one of its rows; one met twice is
+        // moved twice, the same row to the same place
+        const bool inside = p >= base && p < base + 64;
+        s_pos[i] = (unsigned short)(inside ? i : p);
+        s_src[1][i] = (unsigned short)(inside ? s0 : s1);
+    }
+    __syncthreads();
+    if(tid < 64)
+        for(int e = 0; e < nblk; ++e)
+        {
+            const int i = 64 * (inverse ? nblk - 1 - e : e) + lane;
+            const int pos = s_pos[i];
+            const unsigned short r0 = s_row[s_src[0][i]], r1 = s_row[s_src[1][i]];
+            wave_sync();
+            s_row[i] = r0;
+            s_row[pos] = r1;
+            wave_sync();
+        }
+    __syncthreads();
+    int src[R];
+#pragma unroll
+    for(int r = 0; r < R; ++r)
+        src[r] = s_row[tid + r * PERM_THREADS];
+    const int c0 = blockIdx.x * PERM_COLS;
+    constexpr int UC = R <= 4 ? 4 : 2; // columns in flight
+    for(int c1 = 0; c1 < PERM_COLS && c0 + c1 < nrhs; c1 += UC) // uniform
+    {
+        T x[UC][R];
+#pragma unroll
+        for(int u = 0; u < UC; ++u)
+#pragma unroll
+            for(int r = 0; r < R; ++r)
+                x[u][r] = (tid + r * PERM_THREADS < n && c0 + c1 + u < nrhs)
+                              ? Bm[src[r] + int64_t(c0 + c1 + u) * ldb]
+                              : T(0);
+        __syncthreads(); // the loads of these columns are done
+#pragma unroll
+        for(int u = 0; u < UC; ++u)
+#pragma unroll
+            for(int r = 0; r < R; ++r)
+                if(tid + r * PERM_THREADS < n && c0 + c1 + u < nrhs)
+                    Bm[tid + r * PERM_THREADS + int64_t(c0 + c1 + u) * ldb] = x[u][r];
+    }
+}
+
+template <typename T>
+static rocblas_status permute_rows(hipStream_t stream, int n, int nrhs, Batch<T> B, int ldb,
+                                   const int* ipiv, int64_t strideP, bool inverse, int bc,
+                                   const int* skip)
+{
+    if(n > 8 * PERM_THREADS)
+        return laswp<T>(stream, nrhs, B, ldb, 1, n, ipiv, strideP, inverse ? -1 : 1, bc, skip);
+    for(int64_t b0 = 0; b0 < bc; b0 += MAX_GRID_YZ)
+    {
+        const int nb = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);
+        auto go = [&](auto r) {
+            hipLaunchKernelGGL((permute_rows_kernel<T, decltype(r)::value>),
+                               dim3(ceil_div(nrhs, PERM_COLS), nb), dim3(PERM_THREADS), 0, stream,
+                               n, nrhs, B, ldb, ipiv, strideP, int(inverse), skip, b0);
+        };
+        if(n <= PERM_THREADS)
+            go(std::integral_constant<int, 1>{});
+        else if(n <= 2 * PERM_THREADS)
+            go(std::integral_constant<int, 2>{});
+        else if(n <= 4 * PERM_THREADS)
+            go(std::integral_constant<int, 4>{});
+        else
+            go(std::integral_constant<int, 8>{});
+        RSA_LAUNCH_CHECK();
+    }
+    return rocblas_status_success;
+}
+
+// ------------------------------------------------------------ substitution
+// One step of a blocked triangular solve of op(A) X = B in place: every
+// 128-row tile of the grid subtracts its block of op(A) times the solved tile
+// `prev` (-1: none), and the workgroups of tile `next` then solve their
+// diagonal block, so a step is one launch and the next step's solve does not
+// wait for a launch of its own.
+// KIND: 0 = L unit lower (forward), 1 = U non-unit upper (backward), 2 = U^T
+// (forward, non-unit), 3 = L^T (backward, unit).
+//
+// COLS right-hand sides per workgroup (8 wavefronts: COLS / 16 groups of
+// columns times the rest as groups of rows).  The products run on the matrix
+// cores straight from memory (operands swapped, so that 16 lanes hold 16
+// consecutive rows), with half of a wavefront's loads or all of them in
+// flight.  The workgroup that solves holds its triangle of op(A) in LDS,
+// loaded before the update: 32-row diagonal blocks are solved by four lanes
+// per column, the rest of the tile updated by matrix-core products; a
+// wavefront owns 16 columns there.
+//
+// Bound by latency: n / 128 dependent steps per triangle.  A thread per
+// column solving 64-row blocks, with the update in a launch of its own, took
+// 1.7 ms for both triangles at n = 1024 x 64, 8 right-hand sides (transposed)
+// and 3.1 ms for one system of n = 2000; this kernel takes 0.69 and 0.80 ms.
+constexpr int ST = 128; // tile rows
+constexpr int SD = 32; // diagonal block rows
+constexpr int STEP_THREADS = 512;
+
+template <typename T, int KIND, int COLS>
+__global__ __launch_bounds__(STEP_THREADS) void trsm_step_kernel(int n, int nrhs, Batch<T> AA,
+                                                                 int lda, Batch<T> BB, int ldb,
+                                                                 const int* __restrict__ skip,
+                                                                 int prev, int next, int tile0,
+                                                                 int64_t boff)
+{
+    using M = mfma16<T>;
+    constexpr bool LOWER = KIND == 0 || KIND == 2;
+    constexpr bool UNIT = KIND == 0 || KIND == 3;
+    constexpr bool TRANS = KIND >= 2;
+    constexpr int CG = COLS / 16, RG = STEP_THREADS / 64 / CG; // groups of columns, of rows
+    constexpr int RT = ST / 16 / RG; // 16-row tiles per wavefront
+    constexpr int LS = ST + 1;
+    constexpr int ND = ST / SD;
+    __shared__ T sB[COLS * LS];
+    // 32x32 blocks (i, k) of the triangle at i (i + 1) / 2 + k (i >= k, by
+    // the block's row and column, exchanged for an upper triangle)
+    __shared__ __align__(16) T sD[ND * (ND + 1) / 2][SD * SD];
+
+    const int64_t b = blockIdx.z + boff;
     if(skip && skip[b] != 0)
         return;
     const T* A = AA[b];
     T* Bm = BB[b];
     const int tid = threadIdx.x;
-    for(int e = tid; e < rb * rb; e += 256)
+    const int wid = tid / 64;
+    const int lane = tid % 64;
+    const int tile = tile0 + blockIdx.x;
+    const int r0 = tile * ST;
+    const int c0 = blockIdx.y * COLS + 16 * (wid % CG); // this wavefront's columns
+    const int wr = 16 * RT * (wid / CG); // and rows of the tile, in the update
+    const bool solve = tile == next; // uniform
+    auto op = [&](int i, int k) -> T {
+        return TRANS ? A[k + int64_t(i) * lda] : A[i + int64_t(k) * lda];
+    };
+    auto block = [](int i, int k) { return i > k ? i * (i + 1) / 2 + k : k * (k + 1) / 2 + i; };
+
+    if(solve) // the triangle of op(A), columns of each block contiguous; past n: the identity
     {
-        const int i = e % rb, k = e / rb;
-        sD[i + k * TRSM_NB] = A[(r0 + i) + int64_t(r0 + k) * lda];
+#pragma unroll
+        for(int bi = 0; bi < ND; ++bi)
+#pragma unroll
+            for(int bk = 0; bk < ND; ++bk)
+                if(LOWER ? bi >= bk : bi <= bk)
+#pragma unroll
+                    for(int h = 0; h < SD * SD / STEP_THREADS; ++h)
+                    {
+                        // memory order along the column of A
+                        const int e = tid + h * STEP_THREADS, x = e % SD, y = e / SD;
+                        const int i = TRANS ? y : x, k = TRANS ? x : y;
+                        const int gi = r0 + SD * bi + i, gk = r0 + SD * bk + k;
+                        sD[block(bi, bk)][k * SD + i]
+                            = (gi < n && gk < n) ? op(gi, gk) : (gi == gk ? T(1) : T(0));
+                    }
     }
-    __syncthreads();
-    const int c = blockIdx.x * 256 + tid;
-    if(c >= nrhs)
+
+    typename M::acc_t acc[RT];
+#pragma unroll
+    for(int t = 0; t < RT; ++t)
+        acc[t] = typename M::acc_t{0, 0, 0, 0};
+    const int col = c0 + (lane & 15);
+    if(prev >= 0)
+    {
+        const int k0 = prev * ST;
+        constexpr int KS = RT == 1 ? 16 : 8; // matrix-core steps whose loads are in flight
+#pragma unroll 1
+        for(int kk = 0; kk < ST; kk += 4 * KS)
+        {
+            T bv[KS], av[KS][RT];
+#pragma unroll
+            for(int q = 0; q < KS; ++q)
+            {
+                const int k = k0 + kk + 4 * q + (lane >> 4);
+                bv[q] = (k < n && col < nrhs) ? Bm[k + int64_t(col) * ldb] : T(0);
+#pragma unroll
+                for(int t = 0; t < RT; ++t)
+                {
+                    const int i = r0 + wr + 16 * t + (lane & 15);
+                    av[q][t] = (i < n && k < n) ? op(i, k) : T(0);
+                }
+            }
+#pragma unroll
+            for(int q = 0; q < KS; ++q)
+#pragma unroll
+                for(int t = 0; t < RT; ++t)
+                    acc[t] = M::run(bv[q], av[q][t], acc[t]);
+        }
+    }
+#pragma unroll
+    for(int t = 0; t < RT; ++t)
+    {
+        const int li = wr + 16 * t + (lane & 15);
+        const int i = r0 + li;
+#pragma unroll
+        for(int r = 0; r < 4; ++r)
+        {
+            const int c = c0 + M::row(lane, r);
+            const bool in = i < n && c < nrhs;
+            T* p = Bm + i + int64_t(c) * ldb;
+            const T v = in ? *p - acc[t][r] : T(0);
+            if(solve)
+                sB[(16 * (wid % CG) + M::row(lane, r)) * LS + li] = v;
+            else if(in)
+                *p = v;
+        }
+    }
+    if(!solve)
         return;
-    T x[TRSM_NB];
+    __syncthreads();
+    if(wid >= CG || c0 >= nrhs) // one wavefront per 16 columns from here on
+        return;
+    T* colB = sB + 16 * wid * LS;
 #pragma unroll
-    for(int i = 0; i < TRSM_NB; ++i)
-        x[i] = i < rb ? Bm[(r0 + i) + int64_t(c) * ldb] : T(0);
-    auto D = [&](int i, int k) { return sD[i + k * TRSM_NB]; };
-    if(KIND == 0)
+    for(int step = 0; step < ND; ++step)
     {
-        // the block read through an offset tied to x[k] every two columns
-        // (an empty asm), so its entries are not all loaded ahead and spilled
-        const T* Dp = sD;
-#pragma unroll
-        for(int k = 0; k < TRSM_NB; ++k)
+        const int d = LOWER ? step : ND - 1 - step;
+        if(r0 + SD * d < n) // uniform
         {
-            if((k & 1) == 0)
             {
-                uint32_t lo = 0;
-                asm volatile("" : "+v"(lo) : "v"(x[k]));
-                Dp = sD + lo;
-            }
+                T x[SD / 4];
+                T* xp = colB + (lane >> 2) * LS + SD * d + (lane & 3);
 #pragma unroll
-            for(int i = k + 1; i < TRSM_NB; ++i)
-                if(i < rb)
-                    x[i] = fma_t(-Dp[i + k * TRSM_NB], x[k], x[i]);
+                for(int t = 0; t < SD / 4; ++t)
+                    x[t] = xp[4 * t];
+                quad_solve<T, SD, LOWER, UNIT>(sD[block(d, d)], lane, x);
+#pragma unroll
+                for(int t = 0; t < SD / 4; ++t)
+                    xp[4 * t] = x[t];
+            }
+            wave_sync();
+            T bv[SD / 4];
+#pragma unroll
+            for(int ks = 0; ks < SD / 4; ++ks)
+                bv[ks] = colB[(lane & 15) * LS + SD * d + 4 * ks + (lane >> 4)];
+#pragma unroll
+            for(int t = 0; t < ST / 16; ++t)
+            {
+                const int e = t / 2; // the 32-row block of these 16 rows
+                if(LOWER ? e > d : e < d)
+                {
+                    typename M::acc_t u = {0, 0, 0, 0};
+#pragma unroll
+                    for(int ks = 0; ks < SD / 4; ++ks)
+                        u = M::run(sD[block(e, d)][(4 * ks + (lane >> 4)) * SD + 16 * (t & 1)
+                                                   + (lane & 15)],
+                                   bv[ks], u);
+#pragma unroll
+                    for(int r = 0; r < 4; ++r)
+                        colB[(lane & 15) * LS + 16 * t + M::row(lane, r)] -= u[r];
+                }
+            }
+            wave_sync();
         }
     }
-    else if(KIND == 1)
-    {
-#pragma unroll
-        for(int k = TRSM_NB - 1; k >= 0; --k)
-        {
-            if(k < rb)
-            {
-                x[k] = x[k] / D(k, k);
-#pragma unroll
-                for(int i = 0; i < k; ++i)
-                    x[i] = fma_t(-D(i, k), x[k], x[i]);
-            }
-        }
-    }
-    else if(KIND == 2)
-    {
-#pragma unroll
-        for(int k = 0; k < TRSM_NB; ++k)
-        {
-            if(k < rb)
-            {
-                x[k] = x[k] / D(k, k);
-#pragma unroll
-                for(int i = k + 1; i < TRSM_NB; ++i)
-                    if(i < rb)
-                        x[i] = fma_t(-D(k, i), x[k], x[i]);
-            }
-        }
-    }
-    else
-    {
-#pragma unroll
-        for(int k = TRSM_NB - 1; k > 0; --k)
-        {
-            if(k < rb)
-            {
-#pragma unroll
-                for(int i = 0; i < k; ++i)
-                    x[i] = fma_t(-D(k, i), x[k], x[i]);
-            }
-        }
-    }
-#pragma unroll
-    for(int i = 0; i < TRSM_NB; ++i)
-        if(i < rb)
-            Bm[(r0 + i) + int64_t(c) * ldb] = x[i];
+    for(int c = 0; c < 16; ++c)
+        if(c0 + c < nrhs) // uniform
+            for(int i = lane; i < ST && r0 + i < n; i += 64)
+                Bm[r0 + i + int64_t(c0 + c) * ldb] = colB[c * LS + i];
 }
 
+// One triangle of A (KIND as above) against all right-hand sides.
 template <typename T, int KIND>
-static rocblas_status trsm_block(hipStream_t stream, int r0, int rb, int nrhs, Batch<T> A, int lda,
-                                 Batch<T> B, int ldb, int bc, const int* skip)
+static rocblas_status trsm_blocked(hipStream_t stream, int n, int nrhs, Batch<T> A, int lda,
+                                   Batch<T> B, int ldb, int bc, const int* skip)
 {
+    constexpr bool LOWER = KIND == 0 || KIND == 2;
+    const int tiles = ceil_div(n, ST);
+    const int cols = nrhs <= 16 ? 16 : 32;
     for(int64_t b0 = 0; b0 < bc; b0 += MAX_GRID_YZ)
     {
         const int nb = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);
-        dim3 grid(ceil_div(nrhs, 256), nb);
-        hipLaunchKernelGGL((trsm_block_kernel<T, KIND>), grid, dim3(256), 0, stream, r0, rb, nrhs,
-                           A, lda, B, ldb, skip, b0);
-        RSA_LAUNCH_CHECK();
+        for(int s = 0; s < tiles; ++s)
+        {
+            // step s solves tile `next` after the update by the tile before
+            const int next = LOWER ? s : tiles - 1 - s;
+            const int prev = s == 0 ? -1 : (LOWER ? s - 1 : next + 1);
+            const int cnt = s == 0 ? 1 : tiles - s; // tiles not solved yet
+            const int tile0 = LOWER || s == 0 ? next : 0;
+            const dim3 grid(cnt, ceil_div(nrhs, cols), nb);
+            if(cols == 16)
+                hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 16>), grid, dim3(STEP_THREADS), 0,
+                                   stream, n, nrhs, A, lda, B, ldb, skip, prev, next, tile0, b0);
+            else
+                hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 32>), grid, dim3(STEP_THREADS), 0,
+                                   stream, n, nrhs, A, lda, B, ldb, skip, prev, next, tile0, b0);
+            RSA_LAUNCH_CHECK();
+        }
     }
     return rocblas_status_success;
 }
@@ -741,61 +954,20 @@ rocblas_status getrs_blocked(hipStream_t stream, bool trans, int n, int nrhs, Ba
                              const int* ipiv, int64_t strideP, Batch<T> B, int ldb, int bc,
                              bool pivot, const int* skip)
 {
+    if(n <= 0 || nrhs <= 0 || bc <= 0)
+        return rocblas_status_success;
     rocblas_status st = rocblas_status_success;
-#define RSA_TRY(x)                            \
-    do                                        \
-    {                                         \
-        st = (x);                             \
-        if(st != rocblas_status_success)      \
-            return st;                        \
-    } while(0)
-    const int nb = TRSM_NB;
-    if(!trans)
-    {
-        if(pivot)
-            RSA_TRY(laswp<T>(stream, nrhs, B, ldb, 1, n, ipiv, strideP, 1, bc, skip));
-        for(int r0 = 0; r0 < n; r0 += nb)
-        {
-            const int rb = (n - r0) < nb ? (n - r0) : nb;
-            RSA_TRY((trsm_block<T, 0>(stream, r0, rb, nrhs, A, lda, B, ldb, bc, skip)));
-            const int r1 = r0 + rb;
-            RSA_TRY(gemm_sub<T>(stream, false, n - r1, nrhs, rb, A, r1 + int64_t(r0) * lda, lda, B,
-                                r0, ldb, B, r1, ldb, bc, skip));
-        }
-        const int last = ((n - 1) / nb) * nb;
-        for(int r0 = last; r0 >= 0; r0 -= nb)
-        {
-            const int rb = (n - r0) < nb ? (n - r0) : nb;
-            RSA_TRY((trsm_block<T, 1>(stream, r0, rb, nrhs, A, lda, B, ldb, bc, skip)));
-            RSA_TRY(gemm_sub<T>(stream, false, r0, nrhs, rb, A, int64_t(r0) * lda, lda, B, r0,
-                                ldb, B, 0, ldb, bc, skip));
-        }
-    }
-    else
-    {
-        for(int r0 = 0; r0 < n; r0 += nb)
-        {
-            const int rb = (n - r0) < nb ? (n - r0) : nb;
-            RSA_TRY((trsm_block<T, 2>(stream, r0, rb, nrhs, A, lda, B, ldb, bc, skip)));
-            const int r1 = r0 + rb;
-            // B[r1:n] -= (U[r0:r1, r1:n])^T B[r0:r1]
-            RSA_TRY(gemm_sub<T>(stream, true, n - r1, nrhs, rb, A, r0 + int64_t(r1) * lda, lda, B,
-                                r0, ldb, B, r1, ldb, bc, skip));
-        }
-        const int last = ((n - 1) / nb) * nb;
-        for(int r0 = last; r0 >= 0; r0 -= nb)
-        {
-            const int rb = (n - r0) < nb ? (n - r0) : nb;
-            RSA_TRY((trsm_block<T, 3>(stream, r0, rb, nrhs, A, lda, B, ldb, bc, skip)));
-            // B[0:r0] -= (L[r0:r1, 0:r0])^T B[r0:r1]
-            RSA_TRY(gemm_sub<T>(stream, true, r0, nrhs, rb, A, r0, lda, B, r0, ldb, B, 0, ldb, bc,
-                                skip));
-        }
-        if(pivot)
-            RSA_TRY(laswp<T>(stream, nrhs, B, ldb, 1, n, ipiv, strideP, -1, bc, skip));
-    }
-#undef RSA_TRY
-    return rocblas_status_success;
+    if(!trans && pivot)
+        st = permute_rows<T>(stream, n, nrhs, B, ldb, ipiv, strideP, false, bc, skip);
+    if(st == rocblas_status_success)
+        st = trans ? trsm_blocked<T, 2>(stream, n, nrhs, A, lda, B, ldb, bc, skip)
+                   : trsm_blocked<T, 0>(stream, n, nrhs, A, lda, B, ldb, bc, skip);
+    if(st == rocblas_status_success)
+        st = trans ? trsm_blocked<T, 3>(stream, n, nrhs, A, lda, B, ldb, bc, skip)
+                   : trsm_blocked<T, 1>(stream, n, nrhs, A, lda, B, ldb, bc, skip);
+    if(st == rocblas_status_success && trans && pivot)
+        st = permute_rows<T>(stream, n, nrhs, B, ldb, ipiv, strideP, true, bc, skip);
+    return st;
 }
 
 #define RSA_INST(T)                                                                              \

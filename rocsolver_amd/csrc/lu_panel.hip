@@ -19,6 +19,7 @@
 // (64 matrices); this kernel takes 76 us there.
 #include "internal.hpp"
 #include "mfma.hpp"
+#include "quad_solve.hpp"
 
 #include <climits>
 
@@ -67,42 +68,6 @@ __device__ __forceinline__ int few_argmax(float key, int idx)
     const int u = cand ? __float_as_int(key) : 0;
     const int mu = few_max<NW>(u);
     return few_min<NW>((cand && u == mu) ? idx : 0x7fffffff);
-}
-
-// x <- L^-1 x for a unit lower triangular L (N x N, column-major in LDS): four
-// lanes per column, lane q & 3 = s holding rows 4 t + s in x[t].  The solved
-// x_k reaches the other three lanes by a DPP broadcast, so a column takes N
-// steps of at most N/4 fused multiply-adds (a thread per column: up to N - 1).
-template <typename T, int N, int K = 0>
-__device__ __forceinline__ void quad_solve_unit_lower(const T* L, int lane, T (&x)[N / 4])
-{
-    if constexpr(K < N - 1)
-    {
-        if constexpr(K % 4 == 0)
-        {
-            // an empty asm tied to x: the optimiser takes the address of L
-            // as computed from it, so not all of L is loaded ahead (and
-            // spilled)
-            uint32_t lo = 0;
-            asm volatile("" : "+v"(lo) : "v"(x[K / 4]));
-            L += lo;
-        }
-        T xk;
-        if constexpr(sizeof(T) == 8)
-            xk = dpp_mov_d<0x55 * (K % 4)>(x[K / 4]);
-        else
-            xk = __int_as_float(dpp_mov<0x55 * (K % 4)>(__float_as_int(x[K / 4])));
-        const T* col = L + K * N + (lane & 3);
-        if constexpr(K % 4 < 3)
-        {
-            const T y = fma_t(-col[K / 4 * 4], xk, x[K / 4]);
-            x[K / 4] = (lane & 3) > K % 4 ? y : x[K / 4];
-        }
-#pragma unroll
-        for(int t = K / 4 + 1; t < N / 4; ++t)
-            x[t] = fma_t(-col[4 * t], xk, x[t]);
-        quad_solve_unit_lower<T, N, K + 1>(L, lane, x);
-    }
 }
 
 // m - j0 <= R * NT rows, jb <= W columns; W * lda * sizeof(T) below 2^31.
@@ -331,7 +296,7 @@ __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, in
 #pragma unroll
         for(int t = 0; t < W / 4; ++t)
             x[t] = 4 * t + (lane & 3) < jb ? col[4 * t] : T(0);
-        quad_solve_unit_lower<T, W>(sL, lane, x);
+        quad_solve<T, W, true, true>(sL, lane, x);
 #pragma unroll
         for(int t = 0; t < W / 4; ++t)
             if(4 * t + (lane & 3) < jb)
@@ -448,7 +413,7 @@ __global__ __launch_bounds__(256, 1) void outer_apply_kernel(int n, Batch<T> AA,
 #pragma unroll
                 for(int t = 0; t < DB / 4; ++t)
                     x[t] = xp[4 * t];
-                quad_solve_unit_lower<T, DB>(sL[d], lane, x);
+                quad_solve<T, DB, true, true>(sL[d], lane, x);
 #pragma unroll
                 for(int t = 0; t < DB / 4; ++t)
                     xp[4 * t] = x[t];

@@ -92,3 +92,33 @@ def test_panels_without_pivoting(torch_gpu, handle, m, n):
     np.testing.assert_array_equal(info.cpu().numpy(), in_o)
     for b in range(2):
         assert rel_fro(Ad.cpu().numpy()[b], Ao[b]) <= 10 * n * EPS[np.float64]
+
+
+@pytest.mark.parametrize("n,nrhs", [(513, 1), (640, 16), (640, 17), (1000, 33), (1024, 8), (1100, 100),
+                                    (2048, 3), (2049, 2), (4097, 1), (8193, 1)])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_blocked_solve(torch_gpu, handle, n, nrhs, trans, dtype):
+    """getrs beyond the fused orders on well-conditioned factors with
+    arbitrary interchanges: X within n eps (relative infinity norm, the
+    reference threshold) of the oracle; whole and partial tiles of 128 rows
+    and of 16 / 32 right-hand sides, every range of the row permutation; the
+    padding rows of B are untouched."""
+    print(f"getrs n={n} nrhs={nrhs} {trans} {dtype.__name__}", flush=True)
+    g = np.random.default_rng(n * 3 + nrhs)
+    bc, lda, ldb = 2, n + 1, n + 5
+    LU = (g.uniform(-1, 1, size=(bc, n, lda)) / n).astype(dtype)
+    LU[:, np.arange(n), np.arange(n)] = g.uniform(1, 2, size=(bc, n)).astype(dtype)
+    ipiv = np.stack([g.integers(np.arange(1, n + 1), n + 1) for _ in range(bc)]).astype(np.int32)
+    B0 = g.uniform(-1, 1, size=(bc, nrhs, ldb)).astype(dtype)
+    Xo = B0.copy()
+    oracle.getrs(trans, LU, n, ipiv, Xo)
+    Bd = torch_gpu.from_numpy(B0.copy()).cuda()
+    ra.getrs(handle, torch_gpu.from_numpy(LU).cuda(), torch_gpu.from_numpy(ipiv).cuda(), Bd, trans=trans)
+    torch_gpu.cuda.synchronize()
+    Xg = Bd.cpu().numpy()
+    np.testing.assert_array_equal(Xg[:, :, n:], B0[:, :, n:])
+    for b in range(bc):
+        err = np.abs(Xg[b, :, :n] - Xo[b, :, :n]).sum(axis=0).max()
+        assert err <= n * EPS[dtype] * np.abs(Xo[b, :, :n]).sum(axis=0).max()
+
