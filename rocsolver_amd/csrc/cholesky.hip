@@ -2,17 +2,19 @@
 // the factor (potrs) and factor-and-solve (posv), uplo lower (A = L L^T) or
 // upper (A = U^T U).  Only the referenced triangle is read or written.
 //
-// Factorisation: one workgroup of 256 threads per matrix, left-looking over
-// 32-column block columns, the rows of the block column spread one per
-// thread (chunks of 256 rows when n is larger):
+// Factorisation: one workgroup per matrix, left-looking over 32-column block
+// columns:
 //   1. every row of the block column subtracts its products with the finished
-//      columns, 32 at a time (the 32 rows of the diagonal block staged in LDS);
-//   2. the wavefront holding the diagonal block factors it in registers
-//      (right-looking; entries of column k reach the other lanes through
-//      v_readlane);
-//   3. every row below solves its 32 entries against the factored block
-//      (multiplying by the stored reciprocals), and the block column is
-//      written.
+//      columns on the matrix cores, 16 rows x 32 columns per step and
+//      wavefront, operands straight from memory.  v_mfma_*_16x16x4 adds its
+//      four products to the accumulator as a chain of fused multiply-adds
+//      with k increasing (checked bit for bit on gfx950, FP32 and FP64,
+//      denormals included), so accumulators that start at A and take -L as
+//      one operand run the unblocked order of operations;
+//   2. one wavefront factors the diagonal block in registers (right-looking;
+//      column k reaches the other lanes through LDS);
+//   3. the rows below solve against it, four lanes per row, multiplying by
+//      the stored reciprocals, and the block column is written.
 // Per entry the order of operations is that of the reference's unblocked
 // potf2 (library/src/lapack/roclapack_potf2.hpp:160-250): t = a_jj minus the
 // squares of row j's finished entries (one fma each, k increasing); t <= 0 ->
@@ -26,6 +28,8 @@
 // LU path (trsv_rows.hpp) on non-unit triangles: L then L^T, or U^T then U
 // (library/src/lapack/roclapack_potrs.hpp:121-148); larger orders use one
 // thread per (system, right-hand side) substitution.
+#include "mfma.hpp"
+#include "quad_solve.hpp"
 #include "trsv_rows.hpp"
 
 #include <cmath>
@@ -34,149 +38,267 @@ namespace rsa
 {
 
 constexpr int CHB = 32; // block-column width
-constexpr int CHT = 256; // threads per workgroup
+constexpr int CHR = 2; // 16-row groups per wavefront and pass
 
 // Element (i, j), i >= j, of the lower factor L: A[i + j lda] with lower
 // storage, A[j + i lda] with upper storage (which holds U = L^T).
-template <typename T>
+template <typename T, bool UP>
 struct LowerView
 {
     T* a;
-    int lda;
-    bool up;
+    int64_t lda;
     __device__ __forceinline__ T& operator()(int i, int j) const
     {
-        return up ? a[j + int64_t(i) * lda] : a[i + int64_t(j) * lda];
+        return UP ? a[j + i * lda] : a[i + j * lda];
+    }
+    // distance between (i, j) and (i, j + 1)
+    __device__ __forceinline__ int64_t next_col() const
+    {
+        return UP ? 1 : lda;
     }
 };
 
-template <typename T>
-__global__ __launch_bounds__(CHT) void potrf_kernel(int n, Batch<T> AA, int lda, int up,
-                                                    int* __restrict__ info)
+// One row of the block column against the factored diagonal block, four lanes
+// per row: lane s = lane & 3 holds entries 4 t + s in x[t].  x_k times the
+// reciprocal 1 / l_kk, then x_m -= x_k l_mk for m > k.
+template <typename T, int K = 0>
+__device__ __forceinline__ void chol_row_solve(const T* L11, const T* res, int lane,
+                                               T (&x)[CHB / 4])
 {
-    __shared__ T sLd[CHB][CHB + 1]; // rows of the diagonal block, one chunk of finished columns
-    __shared__ T sL11[CHB][CHB + 1]; // the factored diagonal block
+    if constexpr(K < CHB)
+    {
+        if constexpr(K % 4 == 0)
+        {
+            const uint32_t zero = after(x);
+            L11 += zero;
+            res += zero;
+        }
+        const int s = lane & 3;
+        const T y = x[K / 4] * res[K];
+        x[K / 4] = s == K % 4 ? y : x[K / 4];
+        const T xk = quad_broadcast<K % 4>(x[K / 4]);
+        const T* col = L11 + K * CHB;
+        if constexpr(K % 4 < 3)
+        {
+            const T z = fma_t(-xk, col[K / 4 * 4 + s], x[K / 4]);
+            x[K / 4] = s > K % 4 ? z : x[K / 4];
+        }
+#pragma unroll
+        for(int t = K / 4 + 1; t < CHB / 4; ++t)
+            x[t] = fma_t(-xk, col[4 * t + s], x[t]);
+        chol_row_solve<T, K + 1>(L11, res, lane, x);
+    }
+}
+
+// Bound by latency: the chain of n pivots (square root, reciprocal and scaling
+// of one column after the other on one wavefront), the row solves and the
+// operand loads.  So small workgroups and 128 registers: four matrices share
+// a CU, and the matrix-core products of one run under the pivots of another.
+// n = 300 x 1024 FP64: 0.72 ms (three matrices per CU: 0.78); one thread per
+// row with vector fused multiply-adds took 4.14 ms.
+template <typename T, int NT, bool UP>
+__global__ __launch_bounds__(NT, NT == 64 ? 2 : 4) void potrf_kernel(int n, Batch<T> AA, int lda,
+                                                      int* __restrict__ info)
+{
+    using M = mfma16<T>;
+    constexpr int NW = NT / 64;
+    constexpr int TS = CHB + 1; // row stride of the exchange buffers
+    constexpr int KS = 2; // matrix-core steps whose loads are in flight
+    __shared__ T sX[NW > 2 ? NW : 2][16 * TS]; // 16 rows per wavefront; first the diagonal block
+    __shared__ T sL11[CHB * CHB]; // the factored diagonal block, by columns
     __shared__ T sres[CHB]; // 1 / l_jj, or 0 after a non-positive pivot
     __shared__ int sinfo;
 
     const int tid = threadIdx.x;
-    const int lane = tid & 63;
+    const int wid = tid >> 6;
     const int64_t b = blockIdx.x;
-    const LowerView<T> L{AA[b], lda, up != 0};
+    const LowerView<T, UP> L{AA[b], lda};
     if(tid == 0)
         sinfo = 0;
+    for(int e = tid; e < CHB * CHB; e += NT)
+        sL11[e] = T(0); // above the diagonal: read, never used
 
     for(int c0 = 0; c0 < n; c0 += CHB)
     {
         const int jb = n - c0 < CHB ? n - c0 : CHB;
-        for(int r0 = c0; r0 < n; r0 += CHT) // uniform
+        const int groups = (n - c0 + 15) / 16; // the first two hold the diagonal block
+        for(int g0 = 0; g0 < groups; g0 += NW * CHR) // uniform
         {
-            const int i = r0 + tid; // row of this thread
-            const bool act = i < n;
-            T acc[CHB];
+            // group t of this wavefront and pass: rows c0 + 16 (g0 + wid + t NW) ...
+            // lane & 15 is the row, register r the column M::row(lane, r).
+            // Rows past n repeat row n - 1, entries above the diagonal the
+            // diagonal's, and are not stored.  (In every phase the lane comes
+            // from an opaque thread id: addresses and masks formed from it at
+            // entry would stay live through all of them.)
+            const int lane = fresh_tid() & 63;
+            typename M::acc_t acc[CHR][2];
+            const T* pa[CHR];
 #pragma unroll
-            for(int j = 0; j < CHB; ++j)
-                acc[j] = (act && j < jb && c0 + j <= i) ? L(i, c0 + j) : T(0);
-
-            // 1. products with the finished columns 0 .. c0-1, CHB at a time
-            for(int k0 = 0; k0 < c0; k0 += CHB)
+            for(int t = 0; t < CHR; ++t)
             {
-                __syncthreads(); // previous chunk's sLd reads are done
-                for(int e = tid; e < CHB * CHB; e += CHT)
+                const int i = c0 + 16 * (g0 + wid + t * NW) + (lane & 15);
+                const int row = i < n ? i : n - 1;
+                pa[t] = &L(row, lane >> 4);
+#pragma unroll
+                for(int ct = 0; ct < 2; ++ct)
+#pragma unroll
+                    for(int r = 0; r < 4; ++r)
+                    {
+                        const int j = c0 + 16 * ct + M::row(lane, r);
+                        acc[t][ct][r] = L(row, j < row ? j : row);
+                    }
+            }
+            // ---- 1. products with the finished columns 0 .. c0-1
+            const T* pb[2];
+#pragma unroll
+            for(int ct = 0; ct < 2; ++ct)
+            {
+                const int j = c0 + 16 * ct + (lane & 15);
+                pb[ct] = &L(j < n ? j : n - 1, lane >> 4);
+            }
+            const int64_t step = 4 * L.next_col();
+            T av[2][KS][CHR], bv[2][KS][2];
+            auto load = [&](int h) {
+#pragma unroll
+                for(int q = 0; q < KS; ++q)
                 {
-                    const int j = e % CHB, kk = e / CHB;
-                    sLd[j][kk] = j < jb ? L(c0 + j, k0 + kk) : T(0);
+#pragma unroll
+                    for(int ct = 0; ct < 2; ++ct)
+                    {
+                        bv[h][q][ct] = *pb[ct];
+                        pb[ct] += step;
+                    }
+#pragma unroll
+                    for(int t = 0; t < CHR; ++t)
+                    {
+                        av[h][q][t] = *pa[t];
+                        pa[t] += step;
+                    }
                 }
-                __syncthreads();
-                if(act)
+            };
+            // one stage's loads in flight under the other's products (c0 is a
+            // multiple of two stages)
+            static_assert(CHB % (8 * KS) == 0, "whole pairs of stages");
+            if(c0 > 0) // uniform
+                load(0);
+#pragma unroll 1
+            for(int k0 = 0; k0 < c0; k0 += 8 * KS)
+            {
+#pragma unroll
+                for(int h = 0; h < 2; ++h)
                 {
-                    T li[CHB];
+                    if(h == 0 || k0 + 8 * KS < c0) // uniform
+                        load(h ^ 1);
 #pragma unroll
-                    for(int kk = 0; kk < CHB; ++kk)
-                        li[kk] = L(i, k0 + kk);
+                    for(int q = 0; q < KS; ++q)
 #pragma unroll
-                    for(int j = 0; j < CHB; ++j)
-                        if(c0 + j <= i) // the lower triangle only (diagonal-block rows)
+                        for(int t = 0; t < CHR; ++t)
 #pragma unroll
-                            for(int kk = 0; kk < CHB; ++kk)
-                                acc[j] = fma_t(-li[kk], sLd[j][kk], acc[j]);
+                            for(int ct = 0; ct < 2; ++ct)
+                                acc[t][ct] = M::run(bv[h][q][ct], -av[h][q][t], acc[t][ct]);
                 }
             }
 
-            // 2. the diagonal block: lanes 0 .. jb-1 of wavefront 0 (rows c0 + lane)
-            if(r0 == c0) // uniform
+            // ---- 2. the diagonal block (rows c0 .. c0+31): to LDS, factored
+            // by the first wavefront, row c0 + lane in its lanes 0 .. jb-1
+            if(g0 == 0) // uniform
             {
-                if(tid < 64)
+                const int wl = fresh_tid() & 63;
+#pragma unroll
+                for(int t = 0; t < (NW == 1 ? 2 : 1); ++t)
+                    if(wid + t * NW < 2)
+#pragma unroll
+                        for(int ct = 0; ct < 2; ++ct)
+#pragma unroll
+                            for(int r = 0; r < 4; ++r)
+                                sX[wid + t * NW][(wl & 15) * TS + 16 * ct + M::row(wl, r)]
+                                    = acc[t][ct][r];
+                __syncthreads();
+                if(wid == 0)
                 {
+                    // lane = row + 32 h holds columns 2 q + h of its row; the
+                    // finished column k reaches the lanes through LDS.
+                    // Entries above the diagonal and past jb are never used.
+                    const int fl = fresh_tid() & 63;
+                    const int i = fl & (CHB - 1), h = fl >> 5;
+                    T d[CHB / 2];
+#pragma unroll
+                    for(int q = 0; q < CHB / 2; ++q)
+                        d[q] = sX[i >> 4][(i & 15) * TS + 2 * q + h];
 #pragma unroll
                     for(int k = 0; k < CHB; ++k)
                     {
-                        if(k < jb) // uniform
+                        int ik = i; // one column's masks at a time
+                        asm volatile("" : "+v"(ik));
+                        const T t = readlane_t(d[k / 2], k + CHB * (k & 1)); // updated a_kk
+                        // columns past jb hold copies: factored, never stored
+                        const bool bad = t <= T(0); // uniform
+                        if(bad && k < jb && fl == 0 && sinfo == 0)
+                            sinfo = c0 + k + 1;
+                        const T root = sqrt_t(t);
+                        const T piv = bad ? t : root;
+                        const T r = bad ? T(0) : T(1) / root;
+                        const T l = ik == k ? piv : d[k / 2] * r;
+                        if(h == (k & 1) && ik >= k)
                         {
-                            const T t = readlane_t(acc[k], k); // updated a_kk
-                            T piv, r;
-                            if(t <= T(0))
-                            {
-                                if(lane == 0 && sinfo == 0)
-                                    sinfo = c0 + k + 1;
-                                piv = t;
-                                r = T(0);
-                            }
-                            else
-                            {
-                                piv = sqrt_t(t);
-                                r = T(1) / piv;
-                            }
-                            if(lane == k)
-                                acc[k] = piv;
-                            else if(lane > k && lane < jb)
-                                acc[k] *= r;
-                            if(lane == 0)
-                                sres[k] = r;
-                            // trailing entries of the block: a_jm -= l_jk l_mk, m in (k, j]
-#pragma unroll
-                            for(int m = 0; m < CHB; ++m)
-                                if(m > k && m < jb) // uniform
-                                {
-                                    const T lmk = readlane_t(acc[k], m);
-                                    if(lane >= m && lane < jb)
-                                        acc[m] = fma_t(-acc[k], lmk, acc[m]);
-                                }
+                            d[k / 2] = l;
+                            sL11[k * CHB + ik] = l;
                         }
-                    }
-                    if(lane < jb)
-                    {
+                        if(fl == 0)
+                            sres[k] = r;
+                        wave_sync();
+                        // trailing entries: a_jm -= l_jk l_mk, m in (k, j]
+                        const T* col = sL11 + k * CHB + after(d);
+                        const T lik = col[ik];
 #pragma unroll
-                        for(int j = 0; j < CHB; ++j)
-                            if(j <= lane)
+                        for(int q = k / 2; q < CHB / 2; ++q)
+                            if(2 * q + 1 > k)
                             {
-                                sL11[lane][j] = acc[j];
-                                L(c0 + lane, c0 + j) = acc[j];
+                                const T z = fma_t(-lik, col[2 * q + h], d[q]);
+                                if(2 * q > k)
+                                    d[q] = z;
+                                else
+                                    d[q] = h ? z : d[q];
                             }
                     }
+#pragma unroll
+                    for(int q = 0; q < CHB / 2; ++q)
+                        if(2 * q + h <= i && i < jb)
+                            L(c0 + i, c0 + 2 * q + h) = d[q];
                 }
                 __syncthreads();
             }
 
-            // 3. rows below the diagonal block
-            if(act && i >= c0 + jb)
+            // ---- 3. rows below the diagonal block, 16 at a time through LDS
+            // to four lanes per row
+            T* sx = sX[wid];
+#pragma unroll
+            for(int t = 0; t < CHR; ++t)
             {
-#pragma unroll
-                for(int k = 0; k < CHB; ++k)
+                const int lane = fresh_tid() & 63;
+                const int i0 = c0 + 16 * (g0 + wid + t * NW);
+                if(i0 >= c0 + CHB && i0 < n) // uniform in the wavefront
                 {
-                    if(k < jb) // uniform
-                    {
-                        acc[k] *= sres[k];
+                    wave_sync();
 #pragma unroll
-                        for(int m = 0; m < CHB; ++m)
-                            if(m > k && m < jb)
-                                acc[m] = fma_t(-acc[k], sL11[m][k], acc[m]);
+                    for(int ct = 0; ct < 2; ++ct)
+#pragma unroll
+                        for(int r = 0; r < 4; ++r)
+                            sx[(lane & 15) * TS + 16 * ct + M::row(lane, r)] = acc[t][ct][r];
+                    wave_sync();
+                    T x[CHB / 4];
+#pragma unroll
+                    for(int q = 0; q < CHB / 4; ++q)
+                        x[q] = sx[(lane >> 2) * TS + 4 * q + (lane & 3)];
+                    chol_row_solve<T>(sL11, sres, lane, x);
+                    const int i = i0 + (lane >> 2);
+                    if(i < n)
+                    {
+#pragma unroll
+                        for(int q = 0; q < CHB / 4; ++q)
+                            L(i, c0 + 4 * q + (lane & 3)) = x[q];
                     }
                 }
-#pragma unroll
-                for(int j = 0; j < CHB; ++j)
-                    if(j < jb)
-                        L(i, c0 + j) = acc[j];
             }
         }
         __syncthreads(); // the block column is written before the next one reads it
@@ -248,7 +370,8 @@ __global__ __launch_bounds__(64) void potrs_serial_kernel(int n, int nrhs, Batch
     const int c = int(g % nrhs);
     if(skip && skip[b] != 0)
         return;
-    const LowerView<T> L{AA[b], lda, up != 0};
+    const T* A = AA[b];
+    auto L = [&](int i, int j) { return up ? A[j + int64_t(i) * lda] : A[i + int64_t(j) * lda]; };
     T* x = BB[b] + int64_t(c) * ldb;
     for(int k = 0; k < n; ++k)
     {
@@ -276,8 +399,22 @@ rocblas_status potrf(hipStream_t stream, bool up, int n, Batch<T> A, int lda, in
         const int cnt = int((bc - b0) < (1 << 30) ? (bc - b0) : (1 << 30));
         Batch<T> Ab = A.ptrs ? Batch<T>{nullptr, A.ptrs + b0, 0}
                              : Batch<T>{A.base + b0 * A.stride, nullptr, A.stride};
-        hipLaunchKernelGGL((potrf_kernel<T>), dim3(cnt), dim3(CHT), 0, stream, n, Ab, lda,
-                           int(up), info + b0);
+        auto go = [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
+            if(up)
+                hipLaunchKernelGGL((potrf_kernel<T, NT, true>), dim3(cnt), dim3(NT), 0, stream, n,
+                                   Ab, lda, info + b0);
+            else
+                hipLaunchKernelGGL((potrf_kernel<T, NT, false>), dim3(cnt), dim3(NT), 0, stream, n,
+                                   Ab, lda, info + b0);
+        };
+        // as many wavefronts as the first block column gives 16-row groups
+        if(n <= 64)
+            go(std::integral_constant<int, 64>{});
+        else if(n <= 128)
+            go(std::integral_constant<int, 128>{});
+        else
+            go(std::integral_constant<int, 256>{});
         RSA_LAUNCH_CHECK();
     }
     return rocblas_status_success;

@@ -23,6 +23,21 @@ __device__ __forceinline__ double quad_broadcast(double v)
     return dpp_mov_d<0x55 * S>(v);
 }
 
+// 0, which the optimiser must take as computed from every x (an empty asm):
+// an address it is added to is known only then, so the reads of a triangle
+// that the solve of x walks through are not all issued ahead, nor the updates
+// of its later rows put off with their operands kept, in registers (which
+// spills).
+template <typename T, int N>
+__device__ __forceinline__ uint32_t after(const T (&x)[N])
+{
+    uint32_t zero = 0;
+#pragma unroll
+    for(int t = 0; t < N; ++t)
+        asm volatile("" : "+v"(zero) : "v"(x[t]));
+    return zero;
+}
+
 // x <- T^-1 x, T the lower (forward) or upper (backward) triangle of an N x N
 // block, column-major in LDS; UNIT: its diagonal is taken as 1.  STEP counts
 // the columns done.
@@ -34,12 +49,7 @@ __device__ __forceinline__ void quad_solve(const T* L, int lane, T (&x)[N / 4])
         constexpr int K = LOWER ? STEP : N - 1 - STEP;
         if constexpr(STEP % 4 == 0)
         {
-            // an empty asm tied to x: the optimiser takes the address of L
-            // as computed from it, so not all of L is loaded ahead (and
-            // spilled)
-            uint32_t lo = 0;
-            asm volatile("" : "+v"(lo) : "v"(x[K / 4]));
-            L += lo;
+            L += after(x);
         }
         const int s = lane & 3;
         const T* col = L + K * N;
