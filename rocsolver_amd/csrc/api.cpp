@@ -116,8 +116,8 @@ rocblas_status getrs_impl(rocblas_handle handle, rocblas_operation trans, int n,
     if(n <= FUSED_MAX && fits_buffer<T>(lda, n) && fits_buffer<T>(ldb, nrhs))
     {
         RSA_LOG_STAGE(handle, "getrs_fused", "n", n, "nrhs", nrhs, "trans", trans, "bc", bc);
-        return getrs_fused<T, T>(stream, tr, n, nrhs, A, lda, ipiv, strideP, B, ldb, B, ldb, bc,
-                                 nullptr, false);
+        return getrs_fused<T>(stream, tr, n, nrhs, A, lda, ipiv, strideP, B, ldb, B, ldb, bc,
+                              nullptr);
     }
     RSA_LOG_STAGE(handle, "getrs_blocked", "n", n, "nrhs", nrhs, "trans", trans, "bc", bc);
     return getrs_blocked<T>(stream, tr, n, nrhs, A, lda, ipiv, strideP, B, ldb, bc, true,
@@ -163,8 +163,8 @@ rocblas_status gesv_impl(rocblas_handle handle, int n, int nrhs, Batch<T> A, boo
                                      lu_fused_inv_elems(n)));
         if(st != rocblas_status_success)
             return st;
-        return getrs_fused<T, T>(stream, false, n, nrhs, A, lda, ipiv, strideP, B, ldb, B, ldb,
-                                 bc, info, false);
+        return getrs_fused<T>(stream, false, n, nrhs, A, lda, ipiv, strideP, B, ldb, B, ldb,
+                                 bc, info);
     }
     rocblas_status st = getrf_blocked<T>(stream, n, n, A, lda, ipiv, strideP, info, bc, true);
     if(st != rocblas_status_success)

@@ -24,13 +24,13 @@
 // 1 / a_jj.  So the factor equals the oracle's restatement bit for bit; the
 // reference's own dot/gemv reductions differ from it by rounding only.
 //
-// Solve: for n <= 512 one workgroup per system with the row solvers of the
-// LU path (trsv_rows.hpp) on non-unit triangles: L then L^T, or U^T then U
+// Solve: for n <= 512 one workgroup per system with the tile solver of the LU
+// path (tile_solve.hpp) on non-unit triangles: L then L^T, or U^T then U
 // (library/src/lapack/roclapack_potrs.hpp:121-148); larger orders use one
 // thread per (system, right-hand side) substitution.
 #include "mfma.hpp"
 #include "quad_solve.hpp"
-#include "trsv_rows.hpp"
+#include "tile_solve.hpp"
 
 #include <cmath>
 
@@ -307,53 +307,22 @@ __global__ __launch_bounds__(NT, NT == 64 ? 2 : 4) void potrf_kernel(int n, Batc
         info[b] = sinfo;
 }
 
-// One system per workgroup (n <= NMAX): the two non-unit triangular solves
-// with the factor, through the LU path's row solvers.  skip[b] != 0: B of
-// system b is left unchanged (posv after a failed factorisation).
-template <typename T, int NMAX, int NR>
-__global__ __launch_bounds__(NMAX) void potrs_fused_kernel(int n, int nrhs, Batch<T> AA, int lda,
-                                                           int up, Batch<T> BB, int ldb,
-                                                           const int* __restrict__ skip)
+// One system and 16 right-hand sides per workgroup (n <= NMAX): the two
+// non-unit triangular solves with the factor.  skip[b] != 0: B of system b is
+// left unchanged (posv after a failed factorisation).
+template <typename T, int NMAX, int NT, bool UP>
+__global__ __launch_bounds__(NT, sizeof(T) == 4 ? 4 : NMAX == 64 ? 3 : NMAX < NT ? 4 : 2) void potrs_fused_kernel(
+    int n, int nrhs, Batch<T> AA, int lda, Batch<T> BB, int ldb, int bc, unsigned chunks,
+    const int* __restrict__ skip)
 {
-    __shared__ T sx[2][GBS][NR];
-    __shared__ T sL[GBS][GBS + 1];
-    const int64_t b = blockIdx.x;
-    if(skip && skip[b] != 0)
+    unsigned chunk;
+    const int64_t b = tile_solve_system(blockIdx.x, chunks, chunk);
+    if(b >= bc || (skip && skip[b] != 0))
         return;
-    const int tid = threadIdx.x;
-    const MatrixBuffer<T> A(AA[b], lda, n);
-    T* Bm = BB[b];
-    const MatrixBuffer<T> Bbuf(Bm, ldb, nrhs);
-    for(int c0 = 0; c0 < nrhs; c0 += NR)
-    {
-        T x[NR];
-#pragma unroll
-        for(int q = 0; q < NR; ++q)
-        {
-            const uint32_t off = (tid < n && c0 + q < nrhs)
-                                     ? Bbuf.row_offset(tid) + Bbuf.col_offset(c0 + q)
-                                     : MatrixBuffer<T>::OUT_OF_RANGE;
-            x[q] = Bbuf.load(off, 0);
-        }
-        if(up)
-        {
-            solve_lower_rows<T, NR, true>(n, A, x, sx, sL); // U^T y = b
-            solve_upper_rows<T, NR, false>(n, A, x, sx, sL); // U x = y
-        }
-        else
-        {
-            solve_lower_rows<T, NR, false, false, 1>(n, A, x, sx, sL); // L y = b
-            solve_upper_rows<T, NR, true, false, 1>(n, A, x, sx, sL); // L^T x = y
-        }
-        if(tid < n)
-        {
-#pragma unroll
-            for(int q = 0; q < NR; ++q)
-                if(c0 + q < nrhs)
-                    Bm[tid + int64_t(c0 + q) * ldb] = x[q];
-        }
-        __syncthreads();
-    }
+    const int c0 = int(chunk) * TSC;
+    const int cend = nrhs - c0 < TSC ? nrhs : c0 + TSC;
+    tile_solve_body<T, NMAX, NT, UP ? TILE_CHOL_U : TILE_CHOL_L, false>(
+        n, c0, cend, AA[b], lda, nullptr, BB[b], ldb, BB[b], ldb);
 }
 
 // Any order: one thread per (system, right-hand side), column-oriented
@@ -428,29 +397,43 @@ rocblas_status potrs(hipStream_t stream, bool up, int n, int nrhs, Batch<T> A, i
         return rocblas_status_success;
     if(n <= FUSED_MAX && fits_buffer<T>(lda, n) && fits_buffer<T>(ldb, nrhs))
     {
-        auto go = [&](auto nmax, auto nr) {
-            constexpr int NMAX = decltype(nmax)::value;
-            constexpr int NR = decltype(nr)::value;
-            hipLaunchKernelGGL((potrs_fused_kernel<T, NMAX, NR>), dim3(bc), dim3(NMAX), 0, stream,
-                               n, nrhs, A, lda, int(up), B, ldb, skip);
-        };
-        auto by_nrhs = [&](auto nmax) {
-            if(nrhs <= 1)
-                go(nmax, std::integral_constant<int, 1>{});
-            else if(nrhs <= 4)
-                go(nmax, std::integral_constant<int, 4>{});
+        const int chunks = ceil_div(nrhs, TSC);
+        // one launch per 2^30 workgroups at most
+        const int64_t most = (int64_t(1) << 30) / chunks / TILE_XCDS * TILE_XCDS;
+        const int64_t step = most > 0 ? most : TILE_XCDS;
+        for(int64_t b0 = 0; b0 < bc; b0 += step)
+        {
+            const int nb = int((bc - b0) < step ? (bc - b0) : step);
+            auto from = [&](Batch<T> V) {
+                return V.ptrs ? Batch<T>{nullptr, V.ptrs + b0, 0}
+                              : Batch<T>{V.base + b0 * V.stride, nullptr, V.stride};
+            };
+            auto go = [&](auto nmax, auto nt) {
+                constexpr int NMAX = decltype(nmax)::value;
+                constexpr int NT = decltype(nt)::value;
+                const dim3 grid(unsigned(tile_solve_grid(nb, chunks)));
+                const int* sk = skip ? skip + b0 : nullptr;
+                if(up)
+                    hipLaunchKernelGGL((potrs_fused_kernel<T, NMAX, NT, true>), grid, dim3(NT), 0,
+                                       stream, n, nrhs, from(A), lda, from(B), ldb, nb,
+                                       unsigned(chunks), sk);
+                else
+                    hipLaunchKernelGGL((potrs_fused_kernel<T, NMAX, NT, false>), grid, dim3(NT), 0,
+                                       stream, n, nrhs, from(A), lda, from(B), ldb, nb,
+                                       unsigned(chunks), sk);
+            };
+            using std::integral_constant;
+            constexpr int F = sizeof(T) == 8 ? 2 : 1; // as getrs_fused_launch
+            if(n <= 64)
+                go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{});
+            else if(n <= 128)
+                go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{});
+            else if(n <= 256)
+                go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});
             else
-                go(nmax, std::integral_constant<int, 8>{});
-        };
-        if(n <= 64)
-            by_nrhs(std::integral_constant<int, 64>{});
-        else if(n <= 128)
-            by_nrhs(std::integral_constant<int, 128>{});
-        else if(n <= 256)
-            by_nrhs(std::integral_constant<int, 256>{});
-        else
-            by_nrhs(std::integral_constant<int, 512>{});
-        RSA_LAUNCH_CHECK();
+                go(integral_constant<int, 512>{}, integral_constant<int, 512>{});
+            RSA_LAUNCH_CHECK();
+        }
         return rocblas_status_success;
     }
     const int64_t threads = int64_t(bc) * nrhs;

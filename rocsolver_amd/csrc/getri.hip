@@ -99,8 +99,8 @@ rocblas_status getri_solve(hipStream_t stream, int n, Batch<T> LU, int ldlu, con
     if(n <= SMALL_MAX)
         return getrs_small<T>(stream, false, n, n, LU, ldlu, ipiv, strideP, X, ldx, bc, pivot);
     if(pivot && n <= FUSED_MAX && fits_buffer<T>(ldlu, n) && fits_buffer<T>(ldx, n))
-        return getrs_fused<T, T>(stream, false, n, n, LU, ldlu, ipiv, strideP, X, ldx, X, ldx, bc,
-                                 nullptr, false);
+        return getrs_fused<T>(stream, false, n, n, LU, ldlu, ipiv, strideP, X, ldx, X, ldx, bc,
+                                 nullptr);
     return getrs_blocked<T>(stream, false, n, n, LU, ldlu, ipiv, strideP, X, ldx, bc, pivot,
                             nullptr);
 }

@@ -1,21 +1,19 @@
 // getrs_fused.hpp -- one-workgroup-per-system triangular solves with the LU
 // of getrf, for SMALL_MAX < n <= FUSED_MAX (reference order of operations:
 // library/src/lapack/roclapack_getrs.hpp:117-150 -- laswp, then L, then U for
-// op = N; U^T, L^T, then the reverse interchanges for op = T).
+// op = N; U^T, L^T, then the reverse interchanges for op = T).  The factors
+// are read through a buffer resource: lda * n * sizeof(T) must be below 2^31
+// (fits_buffer).  Systems with skip[b] != 0 are left untouched.
 //
-// Thread i owns row i of NR right-hand sides in registers; the triangles are
-// walked by the row solvers of trsv_rows.hpp (32-row diagonal blocks, loads
-// one block ahead, one barrier per block).  The factors are read through a
-// buffer resource: lda * n * sizeof(TL) must be below 2^31 (fits_buffer).
-//
-// Types: TL is the LU precision and the arithmetic precision; TB is the
-// precision of the right-hand side read from BB and of the solution written
-// to XX (XX may alias BB).  ACCUM adds the result to XX instead of storing it
-// (the correction step of iterative refinement).  Systems with skip[b] != 0
-// are left untouched.
+// Two kernels with the same operations per row, so bit-identical results:
+//   * the tile solver of tile_solve.hpp, 16 right-hand sides per workgroup;
+//   * the row solver of trsv_rows.hpp, thread i owning row i of up to four
+//     right-hand sides, for large batches with few of them: there the read
+//     of the factors bounds the call, and its smaller workgroups keep twice
+//     the systems in flight.
 #pragma once
 
-#include "internal.hpp"
+#include "tile_solve.hpp"
 #include "trsv_rows.hpp"
 
 #include <type_traits>
@@ -23,103 +21,161 @@
 namespace rsa
 {
 
-// Solves one system with the whole workgroup (blockDim.x == NMAX, n <= NMAX).
-template <typename TL, typename TB, int NMAX, int NR, bool ACCUM, bool TRANS>
-__device__ __forceinline__ void getrs_fused_body(int n, int nrhs, const TL* __restrict__ Ap,
-                                                 int lda, const int* __restrict__ ipiv,
-                                                 const TB* Bm, int ldb, TB* X, int ldx)
+// Wavefronts per SIMD that the registers are cut for: two tiles a wavefront
+// fit four, four tiles two in FP64.
+template <typename T, int NMAX, int NT, bool TRANS>
+__global__ __launch_bounds__(NT, sizeof(T) == 4 || NMAX < NT ? 4 : 2) void getrs_tile_kernel(
+    int n, int nrhs, Batch<T> AA, int lda, const int* __restrict__ ipivA, int64_t strideP,
+    Batch<T> BB, int ldb, Batch<T> XX, int ldx, int bc, unsigned chunks,
+    const int* __restrict__ skip)
 {
-    __shared__ TL sx[2][GBS][NR];
-    __shared__ TL sL[GBS][GBS + 1];
+    unsigned chunk;
+    const int64_t b = tile_solve_system(blockIdx.x, chunks, chunk);
+    if(b >= bc || (skip && skip[b] != 0))
+        return;
+    const int c0 = int(chunk) * TSC;
+    const int cend = nrhs - c0 < TSC ? nrhs : c0 + TSC;
+    tile_solve_body<T, NMAX, NT, TILE_LU, TRANS>(n, c0, cend, AA[b], lda, ipivA + b * strideP,
+                                                 BB[b], ldb, XX[b], ldx);
+}
+
+// One system per workgroup (blockDim.x == NMAX, n <= NMAX), nrhs <= NR.
+template <typename T, int NMAX, int NR, bool TRANS>
+__global__ __launch_bounds__(NMAX) void getrs_rows_kernel(int n, int nrhs, Batch<T> AA, int lda,
+                                                          const int* __restrict__ ipivA,
+                                                          int64_t strideP, Batch<T> BB, int ldb,
+                                                          Batch<T> XX, int ldx,
+                                                          const int* __restrict__ skip)
+{
+    __shared__ T sx[2][GBS][NR];
+    __shared__ T sL[GBS][GBS + 1];
     __shared__ int sipiv[NMAX];
     __shared__ int ssrc[NMAX];
 
-    const int tid = threadIdx.x;
-    const MatrixBuffer<TL> A(Ap, lda, n);
-    const MatrixBuffer<TB> Bbuf(Bm, ldb, nrhs);
-    const int pos = pivot_position(n, ipiv, TRANS, sipiv, ssrc);
-    const int src = TRANS ? tid : ssrc[tid];
-    const int dst = TRANS ? pos : tid;
-
-    for(int c0 = 0; c0 < nrhs; c0 += NR)
-    {
-        // all NR loads issued back to back (out-of-range offsets read 0)
-        TL x[NR];
-#pragma unroll
-        for(int q = 0; q < NR; ++q)
-        {
-            const uint32_t off = (tid < n && c0 + q < nrhs)
-                                     ? Bbuf.row_offset(src) + Bbuf.col_offset(c0 + q)
-                                     : MatrixBuffer<TB>::OUT_OF_RANGE;
-            x[q] = TL(Bbuf.load(off, 0));
-        }
-        solve_lower_rows<TL, NR, TRANS>(n, A, x, sx, sL);
-        solve_upper_rows<TL, NR, TRANS>(n, A, x, sx, sL);
-        // every thread has read its right-hand side before any row is stored
-        // (X may alias B and op = T stores at the permuted row)
-        __syncthreads();
-        if(tid < n)
-        {
-#pragma unroll
-            for(int q = 0; q < NR; ++q)
-                if(c0 + q < nrhs)
-                {
-                    TB& o = X[dst + int64_t(c0 + q) * ldx];
-                    o = ACCUM ? TB(o + TB(x[q])) : TB(x[q]);
-                }
-        }
-    }
-}
-
-template <typename TL, typename TB, int NMAX, int NR, bool ACCUM, bool TRANS>
-__global__ __launch_bounds__(NMAX) void getrs_fused_kernel(int n, int nrhs, Batch<TL> AA, int lda,
-                                                           const int* __restrict__ ipivA,
-                                                           int64_t strideP, Batch<TB> BB, int ldb,
-                                                           Batch<TB> XX, int ldx,
-                                                           const int* __restrict__ skip)
-{
     const int64_t b = blockIdx.x;
     if(skip && skip[b] != 0)
         return;
-    getrs_fused_body<TL, TB, NMAX, NR, ACCUM, TRANS>(n, nrhs, AA[b], lda, ipivA + b * strideP,
-                                                     BB[b], ldb, XX[b], ldx);
+    const int tid = threadIdx.x;
+    const MatrixBuffer<T> A(AA[b], lda, n);
+    const MatrixBuffer<T> Bbuf(BB[b], ldb, nrhs);
+    T* X = XX[b];
+    const int pos = pivot_position(n, ipivA + b * strideP, TRANS, sipiv, ssrc);
+    const int src = TRANS ? tid : ssrc[tid];
+    const int dst = TRANS ? pos : tid;
+
+    // all loads issued back to back (out-of-range offsets read 0)
+    T x[NR];
+#pragma unroll
+    for(int q = 0; q < NR; ++q)
+    {
+        const uint32_t off = (tid < n && q < nrhs) ? Bbuf.row_offset(src) + Bbuf.col_offset(q)
+                                                   : MatrixBuffer<T>::OUT_OF_RANGE;
+        x[q] = Bbuf.load(off, 0);
+    }
+    solve_lower_rows<T, NR, TRANS>(n, A, x, sx, sL);
+    solve_upper_rows<T, NR, TRANS>(n, A, x, sx, sL);
+    // every thread has read its right-hand side before any row is stored
+    // (X may alias B and op = T stores at the permuted row)
+    __syncthreads();
+    if(tid < n)
+    {
+#pragma unroll
+        for(int q = 0; q < NR; ++q)
+            if(q < nrhs)
+                X[dst + int64_t(q) * ldx] = x[q];
+    }
 }
 
-template <typename TL, typename TB, bool ACCUM>
-rocblas_status getrs_fused_launch(hipStream_t stream, bool trans, int n, int nrhs, Batch<TL> A,
-                                  int lda, const int* ipiv, int64_t strideP, Batch<TB> B, int ldb,
-                                  Batch<TB> X, int ldx, int bc, const int* skip)
+// Which kernel: rows for at most four right-hand sides of 1024 systems or
+// more (four per CU; two beyond n = 256), where it was the faster one:
+//   op N, FP64: n = 96 x 2048, 4 right-hand sides 69 against 75 us; n = 128 x
+//   16384 676 against 800; n = 256 x 4096 598 against 662; n = 300 x 1024
+//   329 against 376; n = 512 x 512 316 against 328 (with fewer systems tiles:
+//   n = 96 x 512 31 against 40 us, n = 128 x 64 33 against 44);
+//   op N, FP32, n <= 256: n = 128 x 16384 401 against 418 us; beyond, tiles
+//   (n = 512 x 512 216 against 175);
+//   op T: FP64, n <= 96: n = 72 x 2048 69 against 85 us; beyond, tiles (n =
+//   128 x 16384 952 against 858, its loads being uncoalesced by rows).
+template <typename T>
+inline bool getrs_by_rows(bool trans, int n, int nrhs, int bc)
 {
+    if(nrhs > 4 || bc < (n > 256 ? 512 : 1024))
+        return false;
+    return trans ? sizeof(T) == 8 && n <= 96 : sizeof(T) == 8 || n <= 256;
+}
+
+template <typename T>
+rocblas_status getrs_fused_launch(hipStream_t stream, bool trans, int n, int nrhs, Batch<T> A,
+                                  int lda, const int* ipiv, int64_t strideP, Batch<T> B, int ldb,
+                                  Batch<T> X, int ldx, int bc, const int* skip)
+{
+    using std::integral_constant;
     if(bc <= 0 || n <= 0 || nrhs <= 0)
         return rocblas_status_success;
-    auto go = [&](auto nmax, auto nr, auto tr) {
-        constexpr int NMAX = decltype(nmax)::value;
-        constexpr int NR = decltype(nr)::value;
-        constexpr bool TR = decltype(tr)::value;
-        hipLaunchKernelGGL((getrs_fused_kernel<TL, TB, NMAX, NR, ACCUM, TR>), dim3(bc), dim3(NMAX),
-                           0, stream, n, nrhs, A, lda, ipiv, strideP, B, ldb, X, ldx, skip);
-    };
-    auto by_trans = [&](auto nmax, auto nr) {
+    if(getrs_by_rows<T>(trans, n, nrhs, bc))
+    {
+        auto go = [&](auto nmax, auto nr, auto tr) {
+            constexpr int NMAX = decltype(nmax)::value;
+            constexpr int NR = decltype(nr)::value;
+            constexpr bool TR = decltype(tr)::value;
+            hipLaunchKernelGGL((getrs_rows_kernel<T, NMAX, NR, TR>), dim3(bc), dim3(NMAX), 0,
+                               stream, n, nrhs, A, lda, ipiv, strideP, B, ldb, X, ldx, skip);
+        };
+        auto by_nrhs = [&](auto nmax, auto tr) {
+            if(nrhs == 1)
+                go(nmax, integral_constant<int, 1>{}, tr);
+            else
+                go(nmax, integral_constant<int, 4>{}, tr);
+        };
         if(trans)
-            go(nmax, nr, std::true_type{});
+            by_nrhs(integral_constant<int, 128>{}, std::true_type{});
+        else if(n <= 128)
+            by_nrhs(integral_constant<int, 128>{}, std::false_type{});
+        else if(n <= 256)
+            by_nrhs(integral_constant<int, 256>{}, std::false_type{});
+        else if constexpr(sizeof(T) == 8)
+            by_nrhs(integral_constant<int, 512>{}, std::false_type{});
+        RSA_LAUNCH_CHECK();
+        return rocblas_status_success;
+    }
+    const int chunks = ceil_div(nrhs, TSC);
+    // one launch per 2^30 workgroups at most
+    const int64_t most = (int64_t(1) << 30) / chunks / TILE_XCDS * TILE_XCDS;
+    const int64_t step = most > 0 ? most : TILE_XCDS;
+    for(int64_t b0 = 0; b0 < bc; b0 += step)
+    {
+        const int nb = int((bc - b0) < step ? (bc - b0) : step);
+        auto from = [&](Batch<T> V) {
+            return V.ptrs ? Batch<T>{nullptr, V.ptrs + b0, 0}
+                          : Batch<T>{V.base + b0 * V.stride, nullptr, V.stride};
+        };
+        auto go = [&](auto nmax, auto nt) {
+            constexpr int NMAX = decltype(nmax)::value;
+            constexpr int NT = decltype(nt)::value;
+            const dim3 grid(unsigned(tile_solve_grid(nb, chunks)));
+            if(trans)
+                hipLaunchKernelGGL((getrs_tile_kernel<T, NMAX, NT, true>), grid, dim3(NT), 0,
+                                   stream, n, nrhs, from(A), lda, ipiv + b0 * strideP, strideP,
+                                   from(B), ldb, from(X), ldx, nb, unsigned(chunks),
+                                   skip ? skip + b0 : nullptr);
+            else
+                hipLaunchKernelGGL((getrs_tile_kernel<T, NMAX, NT, false>), grid, dim3(NT), 0,
+                                   stream, n, nrhs, from(A), lda, ipiv + b0 * strideP, strideP,
+                                   from(B), ldb, from(X), ldx, nb, unsigned(chunks),
+                                   skip ? skip + b0 : nullptr);
+        };
+        // FP64: two tiles a wavefront up to n = 256 (n = 96 x 2048 78 us
+        // against 91 with four, n = 256 x 4096 681 against 713); FP32: four
+        // (49 against 58 us, 367 against 493)
+        constexpr int F = sizeof(T) == 8 ? 2 : 1;
+        if(n <= 128)
+            go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{});
+        else if(n <= 256)
+            go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});
         else
-            go(nmax, nr, std::false_type{});
-    };
-    auto by_nrhs = [&](auto nmax) {
-        if(nrhs <= 1)
-            by_trans(nmax, std::integral_constant<int, 1>{});
-        else if(nrhs <= 4)
-            by_trans(nmax, std::integral_constant<int, 4>{});
-        else
-            by_trans(nmax, std::integral_constant<int, 8>{});
-    };
-    if(n <= 128)
-        by_nrhs(std::integral_constant<int, 128>{});
-    else if(n <= 256)
-        by_nrhs(std::integral_constant<int, 256>{});
-    else
-        by_nrhs(std::integral_constant<int, 512>{});
-    RSA_LAUNCH_CHECK();
+            go(integral_constant<int, 512>{}, integral_constant<int, 512>{});
+        RSA_LAUNCH_CHECK();
+    }
     return rocblas_status_success;
 }
 

@@ -63,13 +63,12 @@ rocblas_status lu_fused_invdiag(hipStream_t stream, int n, Batch<double> AI, int
                                 int bc);
 
 // One-workgroup-per-system solve with the LU of getrf for SMALL_MAX < n <=
-// FUSED_MAX, arithmetic in TL; reads the right-hand sides from B (type TB),
-// writes (or with accum, adds) the solution to X (may alias B).  Entries with
-// skip[b] != 0 are not touched.
-template <typename TL, typename TB>
-rocblas_status getrs_fused(hipStream_t stream, bool trans, int n, int nrhs, Batch<TL> A, int lda,
-                           const int* ipiv, int64_t strideP, Batch<TB> B, int ldb, Batch<TB> X,
-                           int ldx, int bc, const int* skip, bool accum);
+// FUSED_MAX; reads the right-hand sides from B, writes the solution to X (may
+// be B).  Entries with skip[b] != 0 are not touched.
+template <typename T>
+rocblas_status getrs_fused(hipStream_t stream, bool trans, int n, int nrhs, Batch<T> A, int lda,
+                           const int* ipiv, int64_t strideP, Batch<T> B, int ldb, Batch<T> X,
+                           int ldx, int bc, const int* skip);
 
 // -------------------------------------------------------------- blocked path
 // Register-resident panel A[j0:m, j0:j0+jb], jb <= panel_reg_width(m - j0)

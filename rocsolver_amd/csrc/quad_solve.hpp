@@ -39,36 +39,71 @@ __device__ __forceinline__ uint32_t after(const T (&x)[N])
 }
 
 // x <- T^-1 x, T the lower (forward) or upper (backward) triangle of an N x N
-// block, column-major in LDS; UNIT: its diagonal is taken as 1.  STEP counts
-// the columns done.
-template <typename T, int N, bool LOWER, bool UNIT, int STEP = 0>
-__device__ __forceinline__ void quad_solve(const T* L, int lane, T (&x)[N / 4])
+// block, column-major in LDS; UNIT: its diagonal is taken as 1.  The columns
+// are read in groups of G, one group ahead of the one being applied.
+template <typename T, int N, bool LOWER, bool UNIT, int STEP, int G>
+__device__ __forceinline__ void quad_solve_group(const T* L, int lane, T (&x)[N / 4],
+                                                 const T (&cur)[G][N / 4])
 {
-    if constexpr(STEP < N)
+    const int s = lane & 3;
+    T next[G][N / 4];
+    if constexpr(STEP + G < N)
     {
-        constexpr int K = LOWER ? STEP : N - 1 - STEP;
-        if constexpr(STEP % 4 == 0)
+        const T* at = L + after(x) + s;
+#pragma unroll
+        for(int g = 0; g < G; ++g)
         {
-            L += after(x);
+            const int K = LOWER ? STEP + G + g : N - 1 - (STEP + G + g);
+#pragma unroll
+            for(int t = 0; t < N / 4; ++t)
+                if(LOWER ? t >= K / 4 : t <= K / 4)
+                    next[g][t] = at[K * N + 4 * t];
         }
-        const int s = lane & 3;
-        const T* col = L + K * N;
+    }
+#pragma unroll
+    for(int g = 0; g < G; ++g)
+    {
+        const int K = LOWER ? STEP + g : N - 1 - (STEP + g);
+        const int o = K % 4, q = K / 4; // row K: lane o of the four, x[q]
         if constexpr(!UNIT)
         {
-            const T y = x[K / 4] / col[K];
-            x[K / 4] = s == K % 4 ? y : x[K / 4];
+            // in lane o cur[g][q] is the diagonal entry
+            const T y = x[q] / cur[g][q];
+            x[q] = s == o ? y : x[q];
         }
-        const T xk = quad_broadcast<K % 4>(x[K / 4]);
-        if constexpr(LOWER ? K % 4 < 3 : K % 4 > 0)
+        const T xk = o == 0   ? quad_broadcast<0>(x[q])
+                     : o == 1 ? quad_broadcast<1>(x[q])
+                     : o == 2 ? quad_broadcast<2>(x[q])
+                              : quad_broadcast<3>(x[q]);
+        if(LOWER ? o < 3 : o > 0)
         {
-            const T y = fma_t(-col[K / 4 * 4 + s], xk, x[K / 4]);
-            x[K / 4] = (LOWER ? s > K % 4 : s < K % 4) ? y : x[K / 4];
+            const T y = fma_t(-cur[g][q], xk, x[q]);
+            x[q] = (LOWER ? s > o : s < o) ? y : x[q];
         }
 #pragma unroll
-        for(int t = LOWER ? K / 4 + 1 : 0; t < (LOWER ? N / 4 : K / 4); ++t)
-            x[t] = fma_t(-col[4 * t + s], xk, x[t]);
-        quad_solve<T, N, LOWER, UNIT, STEP + 1>(L, lane, x);
+        for(int t = 0; t < N / 4; ++t)
+            if(LOWER ? t > q : t < q)
+                x[t] = fma_t(-cur[g][t], xk, x[t]);
     }
+    if constexpr(STEP + G < N)
+        quad_solve_group<T, N, LOWER, UNIT, STEP + G, G>(L, lane, x, next);
+}
+
+template <typename T, int N, bool LOWER, bool UNIT, int G = (sizeof(T) == 8 ? 2 : 4)>
+__device__ __forceinline__ void quad_solve(const T* L, int lane, T (&x)[N / 4])
+{
+    static_assert(N % G == 0, "whole groups");
+    T first[G][N / 4];
+#pragma unroll
+    for(int g = 0; g < G; ++g)
+    {
+        const int K = LOWER ? g : N - 1 - g;
+#pragma unroll
+        for(int t = 0; t < N / 4; ++t)
+            if(LOWER ? t >= K / 4 : t <= K / 4)
+                first[g][t] = L[K * N + 4 * t + (lane & 3)];
+    }
+    quad_solve_group<T, N, LOWER, UNIT, 0, G>(L, lane, x, first);
 }
 
 } // namespace rsa

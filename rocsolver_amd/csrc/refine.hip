@@ -675,8 +675,8 @@ rocblas_status dsgesv_refine(hipStream_t stream, int factor, int n, int nrhs, Ba
     hipLaunchKernelGGL(ir_mark_singular_kernel, dim3(ceil_div(bc, 256)), dim3(256), 0, stream,
                        info, fskip, bc);
     RSA_LAUNCH_CHECK();
-    RSA_TRY((getrs_fused<double, double>(stream, false, n, nrhs, LU64, n, ipiv, n, B, ldb, X, ldx,
-                                         bc, fskip, false)));
+    RSA_TRY((getrs_fused<double>(stream, false, n, nrhs, LU64, n, ipiv, n, B, ldb, X, ldx,
+                                         bc, fskip)));
 #undef RSA_TRY
     return rocblas_status_success;
 }

@@ -1,7 +1,7 @@
 // vbatched.hpp -- variable-size batched getrf / getrs / gesv (orders 0..512
 // mixed in one batch) in one persistent launch.  No counterpart in the
 // reference; the per-matrix algorithms are the fixed-size ones (lu_small.hpp
-// for n <= 64, lu_fused.hpp + getrs_fused.hpp above), so every matrix gets
+// for n <= 64, lu_fused.hpp + tile_solve.hpp above), so every matrix gets
 // bit-for-bit the result the fixed-size routines give it.
 //
 // Two launches, no host synchronisation (graph-capturable):
@@ -20,10 +20,10 @@
 // autotuner (rocsolver_amd/autotune.py) and installed through the C ABI.
 #pragma once
 
-#include "getrs_fused.hpp"
 #include "internal.hpp"
 #include "lu_fused.hpp"
 #include "lu_small.hpp"
+#include "tile_solve.hpp"
 
 namespace rsa
 {
@@ -140,13 +140,11 @@ __device__ __forceinline__ void vb_big(const VbArgs<T>& a, int b)
     if(OP == VB_GETRS)
     {
         if(a.trans)
-            getrs_fused_body<T, T, VB_THREADS, VB_NR, false, true>(nb, a.nrhs[b], Ab, ldab, ipb,
-                                                                   a.B[b], a.ldb[b], a.B[b],
-                                                                   a.ldb[b]);
+            tile_solve_body<T, VB_THREADS, VB_THREADS, TILE_LU, true>(
+                nb, 0, a.nrhs[b], Ab, ldab, ipb, a.B[b], a.ldb[b], a.B[b], a.ldb[b]);
         else
-            getrs_fused_body<T, T, VB_THREADS, VB_NR, false, false>(nb, a.nrhs[b], Ab, ldab, ipb,
-                                                                    a.B[b], a.ldb[b], a.B[b],
-                                                                    a.ldb[b]);
+            tile_solve_body<T, VB_THREADS, VB_THREADS, TILE_LU, false>(
+                nb, 0, a.nrhs[b], Ab, ldab, ipb, a.B[b], a.ldb[b], a.B[b], a.ldb[b]);
         return;
     }
     const int z = lu_fused_body<T, T, VB_THREADS>(nb, Ab, ldab, Ab, ldab, ipb);
@@ -155,9 +153,8 @@ __device__ __forceinline__ void vb_big(const VbArgs<T>& a, int b)
     if(OP == VB_GESV && z == 0) // uniform; a singular system leaves B untouched
     {
         __syncthreads(); // the factors written by every wave are visible
-        getrs_fused_body<T, T, VB_THREADS, VB_NR, false, false>(nb, a.nrhs[b], Ab, ldab, ipb,
-                                                                a.B[b], a.ldb[b], a.B[b],
-                                                                a.ldb[b]);
+        tile_solve_body<T, VB_THREADS, VB_THREADS, TILE_LU, false>(
+            nb, 0, a.nrhs[b], Ab, ldab, ipb, a.B[b], a.ldb[b], a.B[b], a.ldb[b]);
     }
 }
 

@@ -1,0 +1,61 @@
+"""The two one-workgroup solvers of getrs (orders 65..512) agree bit for bit.
+
+A batch of 1024 systems or more with at most four right-hand sides may take the row solver, a
+small batch or more right-hand sides the tile solver; both run the same operations per row, so a
+system's solution must not depend on the batch it came in or on the other right-hand sides.
+"""
+import numpy as np
+import pytest
+
+import oracle
+import rocsolver_amd as ra
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [65, 80, 96, 97, 127, 128, 129, 160, 255, 257, 300, 511, 512])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_same_bits_for_any_batch_and_rhs_count(torch_gpu, handle, n, trans, dtype):
+    print(f"getrs n={n} {trans} {dtype.__name__}", flush=True)
+    g = np.random.default_rng(n)
+    small, nrhs = 2, 19
+    LU = g.uniform(-1, 1, size=(small, n, n)).astype(dtype) / np.sqrt(n)
+    LU[:, np.arange(n), np.arange(n)] += np.asarray(2, dtype)
+    LU = LU.astype(dtype)
+    ipiv = np.stack([g.integers(np.arange(1, n + 1), n + 1) for _ in range(small)]).astype(np.int32)
+    B = g.uniform(-1, 1, size=(small, nrhs, n)).astype(dtype)
+    Ld, ip = torch_gpu.from_numpy(LU).cuda(), torch_gpu.from_numpy(ipiv).cuda()
+    Bd = torch_gpu.from_numpy(B).cuda()
+    want = Bd.clone()
+    ra.getrs(handle, Ld, ip, want, trans=trans)  # 16 + 3 right-hand sides
+    for r in (1, 3):  # the same systems, few right-hand sides, in a large batch
+        rep = 512
+        X = Bd[:, :r].contiguous().repeat(rep, 1, 1)
+        ra.getrs(handle, Ld.repeat(rep, 1, 1), ip.repeat(rep, 1), X, trans=trans)
+        assert torch_gpu.equal(X.view(rep, small, r, n), want[:, :r].expand(rep, small, r, n))
+    Xo = B.copy()
+    oracle.getrs(trans, LU, n, ipiv, Xo)
+    err = np.abs(want.cpu().numpy() - Xo).max() / np.abs(Xo).max()
+    assert err <= n * np.finfo(dtype).eps
+
+
+@pytest.mark.parametrize("trans", ["N", "T"])
+def test_singular_factor_stays_in_its_column(torch_gpu, handle, trans):
+    """A zero on U's diagonal gives infinities and NaN where the oracle has
+    them, in a partial last block too, and leaves the other systems alone."""
+    g = np.random.default_rng(5)
+    n = 75
+    LU = g.uniform(-1, 1, size=(3, n, n)) / n
+    LU[:, np.arange(n), np.arange(n)] = 1.5
+    LU[1, 70, 70] = 0.0
+    ipiv = np.tile(np.arange(1, n + 1, dtype=np.int32), (3, 1))
+    B = g.uniform(-1, 1, size=(3, 6, n))
+    B[1, 3, 70:] = 0.0
+    Xo = B.copy()
+    oracle.getrs(trans, LU, n, ipiv, Xo)
+    X = torch_gpu.from_numpy(B.copy()).cuda()
+    ra.getrs(handle, torch_gpu.from_numpy(LU).cuda(), torch_gpu.from_numpy(ipiv).cuda(), X, trans=trans)
+    X = X.cpu().numpy()
+    np.testing.assert_array_equal(np.isfinite(X), np.isfinite(Xo))
+    np.testing.assert_allclose(X[[0, 2]], Xo[[0, 2]], rtol=0, atol=n * np.finfo(float).eps * np.abs(Xo[[0, 2]]).max())
