@@ -14,10 +14,10 @@
 //                                         16-column stages prefetched one stage
 //                                         ahead into registers)
 //   3. panel: the accumulators are transposed through LDS to one logical row
-//      per thread and factored with partial pivoting, one barrier per column:
-//      every wave publishes its best candidate row (arg-max, ties to the
-//      lower row -- the reference rule, see pivot_key) and all threads pick
-//      the winner;
+//      per thread and factored with partial pivoting (pivot_step.hpp: every
+//      wave publishes its best candidate -- arg-max, ties to the lower row,
+//      the reference rule, see pivot_key -- all threads pick the winner, whose
+//      row then goes to LDS);
 //   4. the finished block column is written to the output in the logical
 //      order of that moment.
 // Row interchanges never touch memory.  Rows of L21_t are left where step t
@@ -31,6 +31,7 @@
 
 #include "internal.hpp"
 #include "mfma.hpp"
+#include "pivot_step.hpp"
 
 #include <type_traits>
 
@@ -97,10 +98,8 @@ __device__ __forceinline__ int lu_fused_body(int n, const TI* __restrict__ Ai, i
     __shared__ TC sLtt[FNB * UB];
     __shared__ int spi[NMAX]; // logical row -> original row
     __shared__ short ssig[SMAX * NMAX]; // block t: logical row -> storage row
-    __shared__ __align__(16) TC scand[2 * NW * FNB];
-    __shared__ TC skey[2 * NW];
-    __shared__ TC spv[2 * NW];
-    __shared__ int slab[2 * NW];
+    __shared__ __align__(16) TC srow[2][FNB]; // pivot row
+    __shared__ PivotRecord srec[2][NW];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -454,60 +453,30 @@ __device__ __forceinline__ int lu_fused_body(int n, const TI* __restrict__ Ai, i
             {
                 const int c = c0 + k;
                 const int par = k & 1;
-                TC key = (label >= c && label < n) ? pivot_key(rowv[k], label == c) : TC(-1);
-                int lab = label;
-                wave_argmax(key, lab);
-                if(label == lab)
+                const TC key = (label >= c && label < n) ? pivot_key(rowv[k], label == c) : TC(-1);
+                publish_candidate(key, rowv[k], label, &srec[par][w]);
+                __syncthreads();
+                int bl, wb;
+                TC pv, rp;
+                select_candidate<TC, NW>(srec[par], bl, wb, pv, rp);
+                // the pivot row to LDS (whole 16-byte groups from the one
+                // holding column k) by the one thread that holds it, after
+                // the choice: every wavefront's candidate row before it, with
+                // one barrier fewer, filled the LDS pipeline, which takes a
+                // one-lane 16-byte store as a full one
+                if(label == bl)
                 {
-                    // whole 16-byte groups from the one holding column k
-                    // (aligned 16-byte stores; entries left of k are unused),
-                    // and the candidate's key, row and pivot value
                     constexpr int G = 16 / int(sizeof(TC));
 #pragma unroll
                     for(int j = 0; j < FNB; ++j)
                         if(j / G >= k / G)
-                            scand[(par * NW + w) * FNB + j] = rowv[j];
-                    skey[par * NW + w] = key;
-                    slab[par * NW + w] = lab;
-                    spv[par * NW + w] = rowv[k];
+                            srow[par][j] = rowv[j];
                 }
                 __syncthreads();
-                // every wavefront's candidate read first, then a branch-free
-                // selection (ties to the lower row; bitwise operators, so no
-                // short-circuit branches)
-                TC kws[NW], pvs[NW];
-                int lws[NW];
-#pragma unroll
-                for(int ww = 0; ww < NW; ++ww)
-                {
-                    kws[ww] = skey[par * NW + ww];
-                    lws[ww] = slab[par * NW + ww];
-                    pvs[ww] = spv[par * NW + ww];
-                }
-                int wb = 0;
-                TC bk = kws[0];
-                int bl = lws[0];
-                TC pv = pvs[0];
-#pragma unroll
-                for(int ww = 1; ww < NW; ++ww)
-                {
-                    const bool better = (kws[ww] > bk) | ((kws[ww] == bk) & (lws[ww] < bl));
-                    bk = better ? kws[ww] : bk;
-                    bl = better ? lws[ww] : bl;
-                    pv = better ? pvs[ww] : pv;
-                    wb = better ? ww : wb;
-                }
-                // the winner's row (its index held in a vector register: as a
-                // scalar, every read of it waits for the previous one; the
-                // row offset stays a visible multiple of FNB, so the reads
-                // are 16-byte ds_read_b128 with immediate offsets); the
-                // reciprocal of the pivot is formed while those reads are in
-                // flight
-                uint32_t wbv = uint32_t(wb);
-                opaque(wbv);
-                const TC* prow = scand + (par * NW) * FNB + wbv * FNB;
+                const TC* prow = srow[par];
+                pv = readlane_t(pv, wb);
+                rp = readlane_t(rp, wb);
                 const bool nz = pv != TC(0);
-                const TC rp = nz ? TC(1) / pv : TC(1);
                 if(!nz && zero_at == 0)
                     zero_at = c + 1;
                 if(tid == 0)
@@ -533,9 +502,7 @@ __device__ __forceinline__ int lu_fused_body(int n, const TI* __restrict__ Ai, i
 #pragma unroll
                     for(int c8 = (k + 1) / CH * CH; c8 < FNB; c8 += CH)
                     {
-                        // whole 16-byte groups (ds_read_b128; the candidate
-                        // row was stored as whole groups from the one
-                        // holding column k, and entries left of k are unused)
+                        // whole 16-byte groups (ds_read_b128)
                         constexpr int G = 16 / int(sizeof(TC));
                         typedef TC g16_t __attribute__((ext_vector_type(G)));
                         TC u[CH];

@@ -1,11 +1,11 @@
 // lu_panel.hip -- register-resident panel of the blocked LU.
 //
 // One workgroup per matrix holds the W columns A[j0:m, j0:j0+jb] of a panel
-// in registers, R rows per thread, and factors them with partial pivoting
-// with one barrier per column, as the panel of the fused LU does: every
-// wavefront publishes its best candidate row with its key, each thread then
-// finds the winner among the wavefronts, and the interchange moves labels
-// (the logical row a register row holds), not data.  The rows are written
+// in registers, R rows per thread, and factors them with partial pivoting, as
+// the panel of the fused LU does (pivot_step.hpp): every wavefront publishes
+// its best candidate, each thread then finds the winner among them, the
+// winner's row goes to LDS, and the interchange moves labels (the logical row
+// a register row holds), not data.  The rows are written
 // back once, to their final positions.  Interchange semantics: the same final
 // rows as roclapack_getf2.hpp:41-99.
 //
@@ -16,59 +16,16 @@
 // workgroup, broadcast of the winning row, rank-1 update of R rows a thread).
 // Reading and writing the panel in global memory at every column, with two
 // barriers, took 303 us for a 32-column FP64 panel of n = 1024 on average
-// (64 matrices); this kernel takes 76 us there.
+// (64 matrices); this kernel takes 40 us there.
 #include "internal.hpp"
 #include "mfma.hpp"
+#include "pivot_step.hpp"
 #include "quad_solve.hpp"
 
 #include <climits>
 
 namespace rsa
 {
-
-// largest / smallest over groups of NW (4 or 8) consecutive lanes
-template <int NW, typename I>
-__device__ __forceinline__ I few_max(I v)
-{
-    auto mx = [](I a, I b) { return a > b ? a : b; };
-    v = mx(v, I(dpp_mov<0xB1>(int(v))));
-    v = mx(v, I(dpp_mov<0x4E>(int(v))));
-    if(NW == 8)
-        v = mx(v, I(dpp_mov<0x141>(int(v))));
-    return v;
-}
-template <int NW>
-__device__ __forceinline__ int few_min(int v)
-{
-    v = min(v, dpp_mov<0xB1>(v));
-    v = min(v, dpp_mov<0x4E>(v));
-    if(NW == 8)
-        v = min(v, dpp_mov<0x141>(v));
-    return v;
-}
-
-// Index of the largest key among NW candidates, one per lane of each group of
-// NW lanes (a negative key: no candidate), ties to the smaller index; at
-// least one is a candidate.  As group_argmax, on the bit patterns.
-template <int NW>
-__device__ __forceinline__ int few_argmax(double key, int idx)
-{
-    const bool cand = key >= 0.0;
-    const uint64_t u = cand ? uint64_t(__double_as_longlong(key)) : 0u;
-    const int hi = int(u >> 32);
-    const unsigned lo = unsigned(u);
-    const int mh = few_max<NW>(hi);
-    const unsigned ml = few_max<NW>(hi == mh ? lo : 0u);
-    return few_min<NW>((cand && hi == mh && lo == ml) ? idx : 0x7fffffff);
-}
-template <int NW>
-__device__ __forceinline__ int few_argmax(float key, int idx)
-{
-    const bool cand = key >= 0.f;
-    const int u = cand ? __float_as_int(key) : 0;
-    const int mu = few_max<NW>(u);
-    return few_min<NW>((cand && u == mu) ? idx : 0x7fffffff);
-}
 
 // m - j0 <= R * NT rows, jb <= W columns; W * lda * sizeof(T) below 2^31.
 // Row indices inside the kernel count from j0.
@@ -83,9 +40,8 @@ __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, in
     constexpr int CH = 8; // columns of the pivot row read at a time
     static_assert((NW == 4 || NW == 8) && W % CH == 0 && 2 * W <= 64, "panel shape");
     typedef T g16_t __attribute__((ext_vector_type(G)));
-    __shared__ __align__(16) T scand[2][NW][W];
-    __shared__ T skey[2][NW];
-    __shared__ int slab[2][NW];
+    __shared__ __align__(16) T srow[2][W]; // pivot row
+    __shared__ PivotRecord srec[2][NW];
     __shared__ __align__(16) T sL[W * W]; // L11 by columns
     __shared__ int s_swap[W]; // row interchanged with row k (itself: none)
 
@@ -123,10 +79,12 @@ __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, in
         if(k < jb) // uniform
         {
             const int par = k & 1;
-            T key = T(-1);
-            int lab = INT_MAX;
+            int bl = k, wave = 0;
+            T pv, rcp;
             if(PIVOT)
             {
+                T key = T(-1), val = T(0);
+                int lab = INT_MAX;
 #pragma unroll
                 for(int r = 0; r < R; ++r)
                 {
@@ -134,47 +92,41 @@ __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, in
                     const bool better = (kk > key) | ((kk == key) & (label[r] < lab) & (kk >= T(0)));
                     key = better ? kk : key;
                     lab = better ? label[r] : lab;
+                    val = better ? v[r][k] : val;
                 }
-                wave_argmax(key, lab);
+                publish_candidate(key, val, lab, &srec[par][wid]);
+                __syncthreads();
+                select_candidate<T, NW>(srec[par], bl, wave, pv, rcp);
             }
-            else
-                lab = k;
-            // the row held by this wavefront that may become the pivot row
-            // (whole 16-byte groups from the one holding column k)
+            // the pivot row to LDS (whole 16-byte groups from the one holding
+            // column k): only by the thread that holds it, after the choice
+            // -- every wavefront's candidate row before it would fill the LDS
+            // pipeline, which takes a one-lane 16-byte store as a full one
 #pragma unroll
             for(int r = 0; r < R; ++r)
-                if(label[r] == lab)
-                {
-                    const int at = PIVOT ? wid : 0;
+                if(label[r] == bl)
 #pragma unroll
                     for(int j = 0; j < W; ++j)
                         if(j / G >= k / G)
-                            scand[par][at][j] = v[r][j];
-                }
-            if(PIVOT && lane == 0)
-            {
-                skey[par][wid] = key;
-                slab[par][wid] = lab;
-            }
+                            srow[par][j] = v[r][j];
             __syncthreads();
-            int bl = k, wb = 0;
+            const T* prow = srow[par];
             if(PIVOT)
             {
-                const int cw = lane & (NW - 1);
-                const T ck = skey[par][cw];
-                const int cl = slab[par][cw];
-                const int best = few_argmax<NW>(ck, (cl << 3) | cw);
-                bl = __builtin_amdgcn_readfirstlane(best >> 3);
-                wb = best & 7;
+                pv = readlane_t(pv, wave);
+                rcp = readlane_t(rcp, wave);
             }
-            const T* prow = &scand[par][0][0] + wb * W;
-            const T pv = prow[k];
+            else
+            {
+                pv = prow[k];
+                rcp = T(1) / pv;
+            }
             const bool nz = pv != T(0);
             // a zero pivot leaves the column alone with pivoting (every
             // candidate is zero) and multiplies it by zero without (the
             // reference npvt kernels keep the scale at 0:
             // roclapack_getf2_specialized_kernels.hpp:185-188,427-430)
-            const T rcp = nz ? T(1) / pv : T(0);
+            rcp = nz ? rcp : T(0);
             if(!nz && zero_at == 0)
                 zero_at = k + 1;
             if(PIVOT && tid == 0)
