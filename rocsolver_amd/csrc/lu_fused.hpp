@@ -32,6 +32,7 @@
 #include "internal.hpp"
 #include "mfma.hpp"
 #include "pivot_step.hpp"
+#include "quad_solve.hpp"
 
 #include <type_traits>
 
@@ -588,77 +589,76 @@ __device__ __forceinline__ int lu_fused_body(int n, const TI* __restrict__ Ai, i
         }
         if constexpr(INVW)
         {
-            // inv(L_ss) for the later block columns' U = inv(L) C: one
-            // wavefront solves L X = I by columns -- lane j (< 32) holds
-            // column j of X and runs the column-oriented forward substitution,
-            // x_i -= L(i, m) x_m for i > m, the L entries read as LDS
-            // broadcasts -- and writes the whole 32x32 X (ones on the
-            // diagonal, zeros above) column-major to block s of winv.
-            if(inv_now && w == s % NW) // one wavefront; the others wait at the next barrier
+            // inv(L_ss) for the later block columns' U = inv(L) C: L X = I by
+            // columns, four lanes per column (quad_solve.hpp), 16 columns a
+            // wavefront, with the operations of a column-oriented forward
+            // substitution; X (ones on the diagonal, zeros above) goes
+            // column-major to block s of winv.  With INVM 2 the U~ columns
+            // (task 2, 3) are solved the same way, dividing by the diagonal.
+            constexpr int TASKS = INVM == 2 ? 4 : 2;
+            constexpr int TPW = (TASKS + NW - 1) / NW; // tasks per wavefront
+            constexpr int CB = FNB + 1;
+            if(inv_now) // uniform
             {
-                // thread id made opaque here: the identity columns would
-                // otherwise be formed once at entry and kept live (spilled)
-                const int ft = fresh_tid();
-                const int j = ft & (FNB - 1);
-                // INVM 2: lanes 32..63 invert U~ the same way, dividing by its
-                // diagonal (x_m /= d_m; d_m = 1 for L, an exact division)
-                const int h = INVM == 2 ? (ft >> 5) & 1 : 0;
-                TC x[FNB];
+                TC x[TPW][FNB / 4];
 #pragma unroll
-                for(int r = 0; r < FNB; ++r)
-                    x[r] = r == j ? TC(1) : TC(0);
-                uint32_t base = uint32_t(h) * uint32_t(FNB * FNB);
-#pragma unroll
-                for(int m = 0; m < FNB; ++m)
+                for(int q = 0; q < TPW; ++q)
                 {
-                    // the column's reads wait for x_m (the empty asm ties
-                    // their address to it), or the unrolled solve hoists
-                    // all 496 reads to its top
-                    asm volatile("" : "+v"(base) : "v"(x[m]));
-                    const TC* col = sbuf + base + m * FNB;
-                    if constexpr(INVM == 2)
+                    const int task = w + q * NW; // uniform in the wavefront
+                    if(task < TASKS)
                     {
-                        const TC dv = col[m];
-                        x[m] = x[m] / (h ? dv : TC(1));
-                    }
+                        // (lane positions from an opaque thread id: formed at
+                        // entry they would be kept live, and spill)
+                        const int ft = fresh_tid() & 63;
+                        const int j = 16 * (task & 1) + (ft >> 2);
 #pragma unroll
-                    for(int r = m + 1; r < FNB; ++r)
-                        x[r] = fma_t(-col[r], x[m], x[r]);
-                }
-                if constexpr(INVM == 1)
-                {
-                    if(lane < FNB)
-                    {
-                        // element stores: winv need not be 16-byte aligned
-                        TC* dst = winv + s * FNB * FNB + j * FNB;
-#pragma unroll
-                        for(int r = 0; r < FNB; ++r)
-                            dst[r] = x[r];
-                    }
-                }
-                else
-                {
-                    // results through LDS (every lane has read its matrix)
-                    // so the block is stored a column at a time: entry (i, k)
-                    // is inv(L)(i, k) below the diagonal, inv(U)(i, k) =
-                    // inv(U~)(31 - i, 31 - k) on and above it
-                    constexpr int CB = FNB + 1;
-                    wave_sync();
-#pragma unroll
-                    for(int r = 0; r < FNB; ++r)
-                    {
-                        if(h == 0)
-                            sbuf[r * CB + j] = x[r];
+                        for(int t = 0; t < FNB / 4; ++t)
+                            x[q][t] = 4 * t + (ft & 3) == j ? TC(1) : TC(0);
+                        if(task < 2)
+                            quad_solve<TC, FNB, true, true, 1>(sbuf, ft, x[q]);
                         else
-                            sbuf[FNB * CB + (FNB - 1 - r) * CB + (FNB - 1 - j)] = x[r];
-                    }
-                    wave_sync();
-                    const int ft2 = fresh_tid(); // opaque: addresses not formed at entry
-                    const int i = ft2 & (FNB - 1);
+                            quad_solve<TC, FNB, true, false, 1>(sbuf + FNB * FNB, ft, x[q]);
+                        if constexpr(INVM == 1)
+                        {
+                            // element stores: winv need not be 16-byte aligned
+                            TC* dst = winv + s * FNB * FNB + j * FNB + (ft & 3);
 #pragma unroll
-                    for(int t2 = 0; t2 < FNB / 2; ++t2)
+                            for(int t = 0; t < FNB / 4; ++t)
+                                dst[4 * t] = x[q][t];
+                        }
+                    }
+                }
+                if constexpr(INVM == 2)
+                {
+                    // results through LDS so the block is stored a column at
+                    // a time: entry (i, k) is inv(L)(i, k) below the diagonal,
+                    // inv(U)(i, k) = inv(U~)(31 - i, 31 - k) on and above it
+                    __syncthreads(); // every wavefront has read its matrix
+#pragma unroll
+                    for(int q = 0; q < TPW; ++q)
                     {
-                        const int k = ((ft2 >> 5) & 1) + 2 * t2;
+                        const int task = w + q * NW;
+                        if(task < TASKS)
+                        {
+                            const int ft = fresh_tid() & 63;
+                            const int j = 16 * (task & 1) + (ft >> 2);
+#pragma unroll
+                            for(int t = 0; t < FNB / 4; ++t)
+                            {
+                                const int r = 4 * t + (ft & 3);
+                                if(task < 2)
+                                    sbuf[r * CB + j] = x[q][t];
+                                else
+                                    sbuf[FNB * CB + (FNB - 1 - r) * CB + (FNB - 1 - j)] = x[q][t];
+                            }
+                        }
+                    }
+                    __syncthreads();
+#pragma unroll
+                    for(int e = 0; e < FNB * FNB / NMAX; ++e)
+                    {
+                        const int idx = fresh_tid() + e * NMAX;
+                        const int i = idx % FNB, k = idx / FNB;
                         const TC v = i > k ? sbuf[i * CB + k] : sbuf[FNB * CB + i * CB + k];
                         Aout.store(v, Aout.offset(i < jb && k < jb, c0 + i, c0 + k), 0);
                     }
