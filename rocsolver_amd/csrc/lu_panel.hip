@@ -424,16 +424,20 @@ rocblas_status outer_apply(hipStream_t stream, int n, Batch<T> A, int lda, const
 }
 
 // Panel width for `rows` rows: the register file of one CU holds 512 threads
-// x 128 (64-bit: 64) values of a panel beside the working set, so the panel
-// narrows as it gets taller; 0: too tall (or too long a leading dimension for
-// the 32-bit offsets), the caller uses its panel in global memory.
+// x 128 values (FP64: 96) of a panel beside the working set, so the panel
+// narrows as it gets taller (32 columns of 1025..1536 FP64 rows on three rows
+// a thread against 16 on four: n = 2000 5.07 -> 4.92 ms); 0: too tall (or too
+// long a leading dimension for the 32-bit offsets), the caller uses its panel
+// in global memory.
 template <typename T>
 int panel_reg_width(int rows, int lda)
 {
     if(!fits_buffer<T>(lda, 32))
         return 0;
-    const int unit = sizeof(T) == 8 ? 1024 : 2048;
-    return rows <= unit ? 32 : rows <= 2 * unit ? 16 : rows <= 4 * unit ? 8 : 0;
+    if constexpr(sizeof(T) == 8)
+        return rows <= 1536 ? 32 : rows <= 2048 ? 16 : rows <= 4096 ? 8 : 0;
+    else
+        return rows <= 2048 ? 32 : rows <= 4096 ? 16 : rows <= 8192 ? 8 : 0;
 }
 
 template <typename T>
@@ -461,6 +465,8 @@ rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ip
         go(integral_constant<int, 32>{}, integral_constant<int, 1>{}, integral_constant<int, 512>{});
     else if(rows <= 1024)
         go(integral_constant<int, 32>{}, integral_constant<int, 2>{}, integral_constant<int, 512>{});
+    else if(rows <= 1536)
+        go(integral_constant<int, 32>{}, integral_constant<int, 3>{}, integral_constant<int, 512>{});
     else if(rows <= 2048)
         go(integral_constant<int, 16 * S>{}, integral_constant<int, 4>{},
            integral_constant<int, 512>{});

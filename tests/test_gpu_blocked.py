@@ -12,7 +12,7 @@ import rocsolver_amd as ra
 
 pytestmark = pytest.mark.gpu
 EPS = {np.float64: np.finfo(np.float64).eps, np.float32: np.finfo(np.float32).eps}
-PANEL_ROWS = [65, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193]
+PANEL_ROWS = [65, 256, 257, 512, 513, 1024, 1025, 1536, 1537, 2048, 2049, 4096, 4097, 8192, 8193]
 
 
 def rel_fro(a, b):
