@@ -73,13 +73,14 @@ rocblas_status getrs_fused(hipStream_t stream, bool trans, int n, int nrhs, Batc
 // -------------------------------------------------------------- blocked path
 // Register-resident panel A[j0:m, j0:j0+jb], jb <= panel_reg_width(m - j0)
 // columns, with its interchanges applied to the other columns of [o0, oend)
-// and U12 solved for those right of it.  Width 0: the panel is too tall.
+// and U12 solved for those right of it up to uend.  Width 0: the panel is too
+// tall.
 template <typename T>
 int panel_reg_width(int rows, int lda);
 template <typename T>
 rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ipiv,
-                         int64_t strideP, int* info, int j0, int jb, int o0, int oend, int bc,
-                         bool pivot);
+                         int64_t strideP, int* info, int j0, int jb, int o0, int oend, int uend,
+                         int bc, bool pivot);
 // The finished block column [o0, o0 + nb), nb <= OUTER_NB, applied to the
 // columns outside it: interchanges, and U12 right of it.
 constexpr int OUTER_NB = 128;

@@ -10,7 +10,8 @@
 // rows as roclapack_getf2.hpp:41-99.
 //
 // The kernel then applies the panel's interchanges to the other columns of
-// [o0, oend) and solves U12 = L11^-1 A12 for those right of the panel.
+// [o0, oend) and solves U12 = L11^-1 A12 for those right of the panel up to
+// uend.
 //
 // What bounds it: the chain of dependent column steps (arg-max across the
 // workgroup, broadcast of the winning row, rank-1 update of R rows a thread).
@@ -33,7 +34,7 @@ template <typename T, int W, int R, int NT, bool PIVOT>
 __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, int lda,
                                                           int* __restrict__ ipivA, int64_t strideP,
                                                           int* __restrict__ info, int j0, int jb,
-                                                          int o0, int oend)
+                                                          int o0, int oend, int uend)
 {
     constexpr int NW = NT / 64;
     constexpr int G = 16 / int(sizeof(T)); // entries per 16-byte group
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, in
     __syncthreads(); // the interchanged rows are written, L11 is in LDS
 
     // U12 = L11^-1 A12, four lanes per column
-    for(int j = j0 + jb + tid / 4; j < oend; j += NT / 4)
+    for(int j = j0 + jb + tid / 4; j < uend; j += NT / 4)
     {
         T* col = A + int64_t(j) * lda + (lane & 3);
         T x[W / 4];
@@ -442,8 +443,8 @@ int panel_reg_width(int rows, int lda)
 
 template <typename T>
 rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ipiv,
-                         int64_t strideP, int* info, int j0, int jb, int o0, int oend, int bc,
-                         bool pivot)
+                         int64_t strideP, int* info, int j0, int jb, int o0, int oend, int uend,
+                         int bc, bool pivot)
 {
     auto go = [&](auto w, auto r, auto nt) {
         constexpr int W = decltype(w)::value;
@@ -451,10 +452,10 @@ rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ip
         constexpr int NT = decltype(nt)::value;
         if(pivot)
             hipLaunchKernelGGL((panel_reg_kernel<T, W, R, NT, true>), dim3(bc), dim3(NT), 0, stream,
-                               m, A, lda, ipiv, strideP, info, j0, jb, o0, oend);
+                               m, A, lda, ipiv, strideP, info, j0, jb, o0, oend, uend);
         else
             hipLaunchKernelGGL((panel_reg_kernel<T, W, R, NT, false>), dim3(bc), dim3(NT), 0,
-                               stream, m, A, lda, ipiv, strideP, info, j0, jb, o0, oend);
+                               stream, m, A, lda, ipiv, strideP, info, j0, jb, o0, oend, uend);
     };
     using std::integral_constant;
     constexpr int S = sizeof(T) == 8 ? 1 : 2;
@@ -484,7 +485,7 @@ rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ip
     template rocblas_status outer_apply<T>(hipStream_t, int, Batch<T>, int, const int*, int64_t, \
                                            int, int, int, bool);                                \
     template rocblas_status panel_reg<T>(hipStream_t, int, Batch<T>, int, int*, int64_t, int*,  \
-                                         int, int, int, int, int, bool);
+                                         int, int, int, int, int, int, bool);
 RSA_PANEL_INST(float)
 RSA_PANEL_INST(double)
 

@@ -48,7 +48,9 @@ def test_one_panel_special_values(torch_gpu, handle, m, dtype):
 # more columns than one outer block of 128: its last partial block, columns left and right of
 # it in whole and partial chunks of 64, matrices dealt to the XCDs in groups of eight
 OUTER = [(16, 700, 3), (90, 333, 9), (128, 129, 8), (513, 513, 3), (640, 640, 2), (1100, 321, 17),
-         (260, 1000, 3)]
+         (260, 1000, 3),
+         # block columns factored by halves (64 MB and more in panels of at most 16 columns)
+         (4096, 128, 33), (2600, 100, 65)]
 
 
 @pytest.mark.parametrize("m,n,bc", [(m, 40, 3) for m in PANEL_ROWS[1:]] + OUTER)
