@@ -47,11 +47,12 @@ constexpr int tile_solve_tpw()
 
 // op(T) X = acc in place, T the lower (forward) or upper (backward) triangle
 // of op(A).  Rows past n are zero in and out.  par: parity of the LDS buffers.
+// A forward solve starts at block `begin` (the rows before it are zero).
 template <typename T, int NT, int TPW, bool LOWER, bool TRANS, bool UNIT>
 __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>& A,
                                                     typename mfma16<T>::acc_t (&acc)[TPW],
                                                     T (*sX)[TSC * TSX], T (*sL)[TSB * TSB],
-                                                    int& par)
+                                                    int& par, int begin = 0)
 {
     using M = mfma16<T>;
     constexpr int NW = NT / 64;
@@ -131,7 +132,8 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
             xp[4 * q] = TSB * d + 4 * q + (lane & 3) < n ? x[q] : T(0);
     };
 
-    const int first = LOWER ? 0 : D - 1, dir = LOWER ? 1 : -1;
+    const int first = LOWER ? begin : D - 1, dir = LOWER ? 1 : -1;
+    const int steps = D - begin;
     load_diag(first);
 #pragma unroll
     for(int t = 0; t < TPW; ++t)
@@ -139,19 +141,19 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
             publish(t, wid + t * NW, sX[par]);
     put_diag(first, sL[par]);
     load_rows(first);
-    if(D > 1) // uniform
+    if(steps > 1) // uniform
         load_diag(first + dir);
     __syncthreads();
     if(wid == 0)
         solve(first, sX[par], sL[par]);
     __syncthreads();
-    for(int s = 0; s < D; ++s)
+    for(int s = 0; s < steps; ++s)
     {
         // block d is solved; its product with the rows of the next block
         // comes first, so that the next block is solved while the other
         // wavefronts update the rows beyond it
         const int d = first + dir * s, next = d + dir;
-        const bool more = s + 1 < D; // uniform
+        const bool more = s + 1 < steps; // uniform
         T* X = sX[par];
         T* Xn = sX[par ^ 1];
         T* Ln = sL[par ^ 1];
@@ -204,7 +206,7 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
                 update(t);
         }
         load_rows(next);
-        if(s + 2 < D) // uniform
+        if(s + 2 < steps) // uniform
             load_diag(next + dir);
         __syncthreads();
     }
@@ -338,6 +340,58 @@ __device__ __forceinline__ void tile_solve_body(int n, int c0, int cend, const T
             for(int r = 0; r < 4; ++r)
                 X.store(acc[t][r], offset(X, t, r, TRANS), 0);
     }
+}
+
+// Columns c0 .. c0+15 of U^-1 L^-1 into X, the inverse of A = P^T L U with its
+// columns in the order of the interchanges: X = (U^-1 L^-1) P, so column k of
+// the product is column s_row[k] of X (ipiv null: no interchanges).  The
+// right-hand sides are columns of the identity, formed here; their rows before
+// block c0 / 32 are zero through the forward solve, which starts there.
+template <typename T, int NMAX, int NT>
+__device__ __forceinline__ void tile_inverse_body(int n, int c0, const T* __restrict__ Ap, int lda,
+                                                  const int* __restrict__ ipiv, T* Xm, int ldx)
+{
+    using M = mfma16<T>;
+    constexpr int NW = NT / 64;
+    constexpr int TPW = tile_solve_tpw<NMAX, NT>();
+    __shared__ T sX[2][TSC * TSX];
+    __shared__ __align__(16) T sL[2][TSB * TSB];
+    __shared__ unsigned short s_row[NMAX];
+
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const MatrixBuffer<T> A(Ap, lda, n), X(Xm, ldx, n);
+    if(ipiv) // uniform
+        pivot_rows<NMAX, NT>(n, ipiv, s_row, reinterpret_cast<unsigned short*>(sL));
+    else
+    {
+        for(int i = threadIdx.x; i < NMAX; i += NT)
+            s_row[i] = (unsigned short)i;
+        __syncthreads();
+    }
+    typename M::acc_t acc[TPW];
+#pragma unroll
+    for(int t = 0; t < TPW; ++t)
+#pragma unroll
+        for(int r = 0; r < 4; ++r)
+        {
+            const int lane = fresh_tid() & 63;
+            const int i = 16 * (wid + t * NW) + (lane & 15);
+            acc[t][r] = i < n && i == c0 + M::row(lane, r) ? T(1) : T(0);
+        }
+    int par = 0;
+    tile_solve_triangle<T, NT, TPW, true, false, true>(n, A, acc, sX, sL, par, c0 / TSB);
+    tile_solve_triangle<T, NT, TPW, false, false, false>(n, A, acc, sX, sL, par);
+#pragma unroll
+    for(int t = 0; t < TPW; ++t)
+#pragma unroll
+        for(int r = 0; r < 4; ++r)
+        {
+            const int lane = fresh_tid() & 63;
+            const int i = 16 * (wid + t * NW) + (lane & 15);
+            const int k = c0 + M::row(lane, r);
+            const bool in = i < n && k < n;
+            X.store(acc[t][r], X.offset(in, i, in ? int(s_row[k]) : 0), 0);
+        }
 }
 
 // System and group of 16 right-hand sides of a workgroup.  Workgroups go
