@@ -88,12 +88,12 @@ static dim3 square_grid(int n, int bc)
     return dim3(unsigned(tiles < 64 ? tiles : 64), unsigned(bc < 65535 ? bc : 65535));
 }
 
-// One system and 16 columns of its inverse per workgroup.  Bound by the
+// One system and 16 CT columns of its inverse per workgroup.  Bound by the
 // latency of the solves; against writing I and solving for it, the forward
 // solve skips the blocks that the identity leaves zero (on average half), and
 // no right-hand side is written or read: dgetri n = 100 x 2000 0.81 -> 0.68
 // ms with its two copies.
-template <typename T, int NMAX, int NT>
+template <typename T, int NMAX, int NT, int CT>
 __global__ __launch_bounds__(NT, sizeof(T) == 4 || NMAX < NT ? 4 : 2) void inverse_tile_kernel(
     int n, Batch<T> AA, int lda, const int* __restrict__ ipivA, int64_t strideP, Batch<T> XX,
     int ldx, int bc, unsigned chunks)
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(NT, sizeof(T) == 4 || NMAX < NT ? 4 : 2) void inver
     const int64_t b = tile_solve_system(blockIdx.x, chunks, chunk);
     if(b >= bc)
         return;
-    tile_inverse_body<T, NMAX, NT>(n, int(chunk) * TSC, AA[b], lda,
+    tile_inverse_body<T, NMAX, NT, CT>(n, int(chunk) * CT * TSC, AA[b], lda,
                                    ipivA ? ipivA + b * strideP : nullptr, XX[b], ldx);
 }
 
@@ -111,7 +111,10 @@ static rocblas_status inverse_tiles(hipStream_t stream, int n, Batch<T> LU, int 
                                     const int* ipiv, int64_t strideP, Batch<T> X, int ldx, int bc)
 {
     using std::integral_constant;
-    const int chunks = ceil_div(n, TSC);
+    // 32 columns a workgroup beyond n = 128: n = 400 x 200 2.02 -> 1.35 ms, n =
+    // 200 x 800 1.31 -> 1.13; no gain at n = 100 (0.68), 0.96 at n = 128 x 100
+    const int cols = n <= 128 ? TSC : 2 * TSC;
+    const int chunks = ceil_div(n, cols);
     // one launch per 2^30 workgroups at most
     const int64_t step = (int64_t(1) << 30) / chunks / TILE_XCDS * TILE_XCDS;
     for(int64_t b0 = 0; b0 < bc; b0 += step)
@@ -121,21 +124,25 @@ static rocblas_status inverse_tiles(hipStream_t stream, int n, Batch<T> LU, int 
             return V.ptrs ? Batch<T>{nullptr, V.ptrs + b0, 0}
                           : Batch<T>{V.base + b0 * V.stride, nullptr, V.stride};
         };
-        auto go = [&](auto nmax, auto nt) {
+        auto go = [&](auto nmax, auto nt, auto ct) {
             constexpr int NMAX = decltype(nmax)::value;
             constexpr int NT = decltype(nt)::value;
-            hipLaunchKernelGGL((inverse_tile_kernel<T, NMAX, NT>),
+            constexpr int CT = decltype(ct)::value;
+            hipLaunchKernelGGL((inverse_tile_kernel<T, NMAX, NT, CT>),
                                dim3(unsigned(tile_solve_grid(nb, chunks))), dim3(NT), 0, stream, n,
                                from(LU), ldlu, ipiv ? ipiv + b0 * strideP : nullptr, strideP,
                                from(X), ldx, nb, unsigned(chunks));
         };
         constexpr int F = sizeof(T) == 8 ? 2 : 1; // as getrs_fused_launch
         if(n <= 128)
-            go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{});
+            go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{},
+               integral_constant<int, 1>{});
         else if(n <= 256)
-            go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});
+            go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{},
+               integral_constant<int, 2>{});
         else
-            go(integral_constant<int, 512>{}, integral_constant<int, 512>{});
+            go(integral_constant<int, 512>{}, integral_constant<int, 512>{},
+               integral_constant<int, 2>{});
         RSA_LAUNCH_CHECK();
     }
     return rocblas_status_success;

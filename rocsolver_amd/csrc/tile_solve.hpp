@@ -47,15 +47,19 @@ constexpr int tile_solve_tpw()
 
 // op(T) X = acc in place, T the lower (forward) or upper (backward) triangle
 // of op(A).  Rows past n are zero in and out.  par: parity of the LDS buffers.
-// A forward solve starts at block `begin` (the rows before it are zero).
-template <typename T, int NT, int TPW, bool LOWER, bool TRANS, bool UNIT>
+// A forward solve starts at block `begin` (the rows before it are zero).  CT
+// groups of 16 right-hand sides share the factor's entries and the barriers;
+// each has its own solving wavefront.
+template <typename T, int NT, int TPW, int CT, bool LOWER, bool TRANS, bool UNIT>
 __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>& A,
-                                                    typename mfma16<T>::acc_t (&acc)[TPW],
-                                                    T (*sX)[TSC * TSX], T (*sL)[TSB * TSB],
+                                                    typename mfma16<T>::acc_t (&acc)[TPW][CT],
+                                                    T (*sX)[CT * TSC * TSX],
+                                                    T (*sL)[TSB * TSB],
                                                     int& par, int begin = 0)
 {
     using M = mfma16<T>;
     constexpr int NW = NT / 64;
+    static_assert(CT <= NW, "a solving wavefront per group");
     constexpr int DL = TSB * TSB / NT; // entries of the diagonal block per thread
     constexpr int KS = TSB / 4;
     const int D = (n + TSB - 1) / TSB;
@@ -112,13 +116,16 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
     auto publish = [&](int t, int tile, T* X) {
         const int lane = fresh_tid() & 63;
 #pragma unroll
-        for(int r = 0; r < 4; ++r)
-            X[M::row(lane, r) * TSX + 16 * (tile & 1) + (lane & 15)] = acc[t][r];
+        for(int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for(int r = 0; r < 4; ++r)
+                X[(16 * ct + M::row(lane, r)) * TSX + 16 * (tile & 1) + (lane & 15)]
+                    = acc[t][ct][r];
     };
-    auto solve = [&](int d, T* X, const T* L) { // by one wavefront
+    auto solve = [&](int ct, int d, T* X, const T* L) { // group ct, by one wavefront
         const int lane = fresh_tid() & 63;
         T x[TSB / 4];
-        T* xp = X + (lane >> 2) * TSX + (lane & 3);
+        T* xp = X + (16 * ct + (lane >> 2)) * TSX + (lane & 3);
 #pragma unroll
         for(int q = 0; q < TSB / 4; ++q)
             x[q] = xp[4 * q];
@@ -144,8 +151,8 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
     if(steps > 1) // uniform
         load_diag(first + dir);
     __syncthreads();
-    if(wid == 0)
-        solve(first, sX[par], sL[par]);
+    if(wid < CT)
+        solve(wid, first, sX[par], sL[par]);
     __syncthreads();
     for(int s = 0; s < steps; ++s)
     {
@@ -158,20 +165,24 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
         T* Xn = sX[par ^ 1];
         T* Ln = sL[par ^ 1];
         par ^= 1;
-        T bv[KS];
+        T bv[CT][KS];
         {
             const int lane = fresh_tid() & 63;
             const int g = LOWER ? lane >> 4 : 3 - (lane >> 4);
 #pragma unroll
-            for(int ks = 0; ks < KS; ++ks)
-                bv[ks] = -X[(lane & 15) * TSX + 4 * ks + g];
+            for(int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for(int ks = 0; ks < KS; ++ks)
+                    bv[ct][ks] = -X[(16 * ct + (lane & 15)) * TSX + 4 * ks + g];
         }
         auto update = [&](int t) {
 #pragma unroll
             for(int q = 0; q < KS; ++q)
             {
                 const int ks = LOWER ? q : KS - 1 - q;
-                acc[t] = M::run(bv[ks], av[t][ks], acc[t]);
+#pragma unroll
+                for(int ct = 0; ct < CT; ++ct)
+                    acc[t][ct] = M::run(bv[ct][ks], av[t][ks], acc[t][ct]);
             }
         };
 #pragma unroll
@@ -182,8 +193,11 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
             {
                 const int lane = fresh_tid() & 63;
 #pragma unroll
-                for(int r = 0; r < 4; ++r)
-                    acc[t][r] = X[M::row(lane, r) * TSX + 16 * (tile & 1) + (lane & 15)];
+                for(int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for(int r = 0; r < 4; ++r)
+                        acc[t][ct][r]
+                            = X[(16 * ct + M::row(lane, r)) * TSX + 16 * (tile & 1) + (lane & 15)];
             }
             else if(more && (tile >> 1) == next) // uniform
             {
@@ -196,8 +210,9 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
             break;
         put_diag(next, Ln);
         __syncthreads();
-        if(wid == (2 * next) % NW) // uniform: an owner of the next block's rows
-            solve(next, Xn, Ln);
+        const int ct = (wid + NW - (2 * next) % NW) % NW; // uniform
+        if(ct < CT) // first the owners of the next block's rows
+            solve(ct, next, Xn, Ln);
 #pragma unroll
         for(int t = 0; t < TPW; ++t)
         {
@@ -310,27 +325,27 @@ __device__ __forceinline__ void tile_solve_body(int n, int c0, int cend, const T
     int par = 0;
     for(; c0 < cend; c0 += TSC) // uniform
     {
-        typename M::acc_t acc[TPW];
+        typename M::acc_t acc[TPW][1];
 #pragma unroll
         for(int t = 0; t < TPW; ++t)
 #pragma unroll
             for(int r = 0; r < 4; ++r)
-                acc[t][r] = B.load(offset(B, t, r, !TRANS), 0);
+                acc[t][0][r] = B.load(offset(B, t, r, !TRANS), 0);
         if constexpr(FACTOR == TILE_LU && !TRANS)
         {
-            tile_solve_triangle<T, NT, TPW, true, false, true>(n, A, acc, sX, sL, par);
-            tile_solve_triangle<T, NT, TPW, false, false, false>(n, A, acc, sX, sL, par);
+            tile_solve_triangle<T, NT, TPW, 1, true, false, true>(n, A, acc, sX, sL, par);
+            tile_solve_triangle<T, NT, TPW, 1, false, false, false>(n, A, acc, sX, sL, par);
         }
         else if constexpr(FACTOR == TILE_LU)
         {
-            tile_solve_triangle<T, NT, TPW, true, true, false>(n, A, acc, sX, sL, par); // U^T
-            tile_solve_triangle<T, NT, TPW, false, true, true>(n, A, acc, sX, sL, par); // L^T
+            tile_solve_triangle<T, NT, TPW, 1, true, true, false>(n, A, acc, sX, sL, par); // U^T
+            tile_solve_triangle<T, NT, TPW, 1, false, true, true>(n, A, acc, sX, sL, par); // L^T
         }
         else
         {
             constexpr bool UP = FACTOR == TILE_CHOL_U;
-            tile_solve_triangle<T, NT, TPW, true, UP, false>(n, A, acc, sX, sL, par);
-            tile_solve_triangle<T, NT, TPW, false, !UP, false>(n, A, acc, sX, sL, par);
+            tile_solve_triangle<T, NT, TPW, 1, true, UP, false>(n, A, acc, sX, sL, par);
+            tile_solve_triangle<T, NT, TPW, 1, false, !UP, false>(n, A, acc, sX, sL, par);
         }
         // every right-hand side was read before the solves' barriers, so the
         // permuted rows of op T may overwrite them
@@ -338,23 +353,23 @@ __device__ __forceinline__ void tile_solve_body(int n, int c0, int cend, const T
         for(int t = 0; t < TPW; ++t)
 #pragma unroll
             for(int r = 0; r < 4; ++r)
-                X.store(acc[t][r], offset(X, t, r, TRANS), 0);
+                X.store(acc[t][0][r], offset(X, t, r, TRANS), 0);
     }
 }
 
-// Columns c0 .. c0+15 of U^-1 L^-1 into X, the inverse of A = P^T L U with its
+// Columns c0 .. c0 + 16 CT - 1 of U^-1 L^-1 into X, the inverse of A = P^T L U with its
 // columns in the order of the interchanges: X = (U^-1 L^-1) P, so column k of
 // the product is column s_row[k] of X (ipiv null: no interchanges).  The
 // right-hand sides are columns of the identity, formed here; their rows before
 // block c0 / 32 are zero through the forward solve, which starts there.
-template <typename T, int NMAX, int NT>
+template <typename T, int NMAX, int NT, int CT>
 __device__ __forceinline__ void tile_inverse_body(int n, int c0, const T* __restrict__ Ap, int lda,
                                                   const int* __restrict__ ipiv, T* Xm, int ldx)
 {
     using M = mfma16<T>;
     constexpr int NW = NT / 64;
     constexpr int TPW = tile_solve_tpw<NMAX, NT>();
-    __shared__ T sX[2][TSC * TSX];
+    __shared__ T sX[2][CT * TSC * TSX];
     __shared__ __align__(16) T sL[2][TSB * TSB];
     __shared__ unsigned short s_row[NMAX];
 
@@ -368,29 +383,30 @@ __device__ __forceinline__ void tile_inverse_body(int n, int c0, const T* __rest
             s_row[i] = (unsigned short)i;
         __syncthreads();
     }
-    typename M::acc_t acc[TPW];
+    typename M::acc_t acc[TPW][CT];
 #pragma unroll
     for(int t = 0; t < TPW; ++t)
 #pragma unroll
-        for(int r = 0; r < 4; ++r)
+        for(int r = 0; r < 4 * CT; ++r)
         {
             const int lane = fresh_tid() & 63;
             const int i = 16 * (wid + t * NW) + (lane & 15);
-            acc[t][r] = i < n && i == c0 + M::row(lane, r) ? T(1) : T(0);
+            const int k = c0 + 16 * (r / 4) + M::row(lane, r % 4);
+            acc[t][r / 4][r % 4] = i < n && i == k ? T(1) : T(0);
         }
     int par = 0;
-    tile_solve_triangle<T, NT, TPW, true, false, true>(n, A, acc, sX, sL, par, c0 / TSB);
-    tile_solve_triangle<T, NT, TPW, false, false, false>(n, A, acc, sX, sL, par);
+    tile_solve_triangle<T, NT, TPW, CT, true, false, true>(n, A, acc, sX, sL, par, c0 / TSB);
+    tile_solve_triangle<T, NT, TPW, CT, false, false, false>(n, A, acc, sX, sL, par);
 #pragma unroll
     for(int t = 0; t < TPW; ++t)
 #pragma unroll
-        for(int r = 0; r < 4; ++r)
+        for(int r = 0; r < 4 * CT; ++r)
         {
             const int lane = fresh_tid() & 63;
             const int i = 16 * (wid + t * NW) + (lane & 15);
-            const int k = c0 + M::row(lane, r);
+            const int k = c0 + 16 * (r / 4) + M::row(lane, r % 4);
             const bool in = i < n && k < n;
-            X.store(acc[t][r], X.offset(in, i, in ? int(s_row[k]) : 0), 0);
+            X.store(acc[t][r / 4][r % 4], X.offset(in, i, in ? int(s_row[k]) : 0), 0);
         }
 }
 
