@@ -258,8 +258,11 @@ def getrf(handle: Handle, A, m: int | None = None, pivot: bool = True, batched: 
     m = lda if m is None else m
     k = min(m, n)
     dev = A.device
-    ipiv = torch.zeros((bc, max(k, 1)), dtype=torch.int32, device=dev)
-    info = torch.zeros(bc, dtype=torch.int32, device=dev)
+    # every entry is written by the call where there are pivots (info always):
+    # no clearing launches before it
+    ipiv = (torch.empty if pivot and k else torch.zeros)((bc, max(k, 1)), dtype=torch.int32,
+                                                         device=dev)
+    info = torch.empty(bc, dtype=torch.int32, device=dev)
     p = _prefix(A)
     if batched:
         ptrs = pointer_array(A)
@@ -303,7 +306,7 @@ def getri(handle: Handle, LU, ipiv=None, C=None, form: str = "strided"):
     import torch
     bc, n, lda = LU.shape
     p = _prefix(LU)
-    info = torch.zeros(bc, dtype=torch.int32, device=LU.device)
+    info = torch.empty(bc, dtype=torch.int32, device=LU.device)
     npvt = ipiv is None
     name = f"rocsolver_{p}getri" + ("_npvt" if npvt else "") + ("_outofplace" if C is not None else "")
     piv = [] if npvt else [ipiv.data_ptr()]
@@ -339,7 +342,7 @@ def potrf(handle: Handle, A, uplo: str = "L", form: str = "strided", unblocked: 
     bc, n, lda = A.shape
     p = _prefix(A)
     u = FILL_UPPER if uplo.upper() == "U" else FILL_LOWER
-    info = torch.zeros(bc, dtype=torch.int32, device=A.device)
+    info = torch.empty(bc, dtype=torch.int32, device=A.device)
     name = f"rocsolver_{p}" + ("potf2" if unblocked else "potrf")
     if form == "plain":
         assert bc == 1
@@ -362,7 +365,7 @@ def potrs(handle: Handle, F, B, uplo: str = "L", form: str = "strided", posv: bo
     p = _prefix(F)
     u = FILL_UPPER if uplo.upper() == "U" else FILL_LOWER
     name = f"rocsolver_{p}" + ("posv" if posv else "potrs")
-    info = torch.zeros(bc, dtype=torch.int32, device=F.device) if posv else None
+    info = torch.empty(bc, dtype=torch.int32, device=F.device) if posv else None
     tail = [info.data_ptr()] if posv else []
     if form == "plain":
         assert bc == 1
@@ -383,8 +386,10 @@ def gesv(handle: Handle, A, B, batched: bool = False):
     bc, n, lda = A.shape
     _, nrhs, ldb = B.shape
     dev = A.device
-    ipiv = torch.zeros((bc, max(n, 1)), dtype=torch.int32, device=dev)
-    info = torch.zeros(bc, dtype=torch.int32, device=dev)
+    # written whole by the call (no pivots when there is nothing to solve)
+    ipiv = (torch.empty if n and nrhs else torch.zeros)((bc, max(n, 1)), dtype=torch.int32,
+                                                        device=dev)
+    info = torch.empty(bc, dtype=torch.int32, device=dev)
     p = _prefix(A)
     if batched:
         pa, pb = pointer_array(A), pointer_array(B)
