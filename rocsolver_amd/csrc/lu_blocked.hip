@@ -839,9 +839,9 @@ __global__ __launch_bounds__(STEP_THREADS) void trsm_step_kernel(int n, int nrhs
     const int tid = threadIdx.x;
     const int wid = tid / 64;
     const int lane = tid % 64;
-    const int tile = tile0 + blockIdx.x;
+    const int tile = tile0 + blockIdx.y;
     const int r0 = tile * ST;
-    const int c0 = blockIdx.y * COLS + 16 * (wid % CG); // this wavefront's columns
+    const int c0 = blockIdx.x * COLS + 16 * (wid % CG); // this wavefront's columns
     const int wr = 16 * RT * (wid / CG); // and rows of the tile, in the update
     const bool solve = tile == next; // uniform
     auto op = [&](int i, int k) -> T {
@@ -990,7 +990,8 @@ static rocblas_status trsm_blocked(hipStream_t stream, int n, int nrhs, Batch<T>
             const int prev = s == 0 ? -1 : (LOWER ? s - 1 : next + 1);
             const int cnt = s == 0 ? 1 : tiles - s; // tiles not solved yet
             const int tile0 = LOWER || s == 0 ? next : 0;
-            const dim3 grid(cnt, ceil_div(nrhs, cols), nb);
+            // right-hand sides in x: more than 65535 groups of them are allowed
+            const dim3 grid(ceil_div(nrhs, cols), cnt, nb);
             if(cols == 16)
                 hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 16>), grid, dim3(STEP_THREADS), 0,
                                    stream, n, nrhs, A, lda, B, ldb, skip, prev, next, tile0, b0);

@@ -124,3 +124,22 @@ def test_blocked_solve(torch_gpu, handle, n, nrhs, trans, dtype):
         err = np.abs(Xg[b, :, :n] - Xo[b, :, :n]).sum(axis=0).max()
         assert err <= n * EPS[dtype] * np.abs(Xo[b, :, :n]).sum(axis=0).max()
 
+
+
+def test_blocked_solve_many_right_hand_sides(torch_gpu, handle):
+    """More groups of right-hand sides than a grid's second dimension holds: the same 33
+    columns over and over, so every copy has the solution of the first, bit for bit, and that
+    one is the solution of a call with 33 columns."""
+    n, copies, w = 513, 63551, 33
+    print(f"getrs n={n} nrhs={copies * w}", flush=True)
+    g = np.random.default_rng(7)
+    LU = (g.uniform(-1, 1, size=(1, n, n)) / n).astype(np.float32)
+    LU[:, np.arange(n), np.arange(n)] = g.uniform(1, 2, size=(1, n)).astype(np.float32)
+    ipiv = g.integers(np.arange(1, n + 1), n + 1).astype(np.int32)[None]
+    LUd, ipd = torch_gpu.from_numpy(LU).cuda(), torch_gpu.from_numpy(ipiv).cuda()
+    few = torch_gpu.from_numpy(g.uniform(-1, 1, size=(1, w, n)).astype(np.float32)).cuda()
+    many = few.repeat(1, copies, 1)
+    ra.getrs(handle, LUd, ipd, few)
+    ra.getrs(handle, LUd, ipd, many)
+    torch_gpu.cuda.synchronize()
+    assert torch_gpu.equal(many.view(copies, w, n), few.expand(copies, w, n))
