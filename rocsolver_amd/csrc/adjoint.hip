@@ -7,64 +7,74 @@
 // No counterpart in the reference; the transposed solve follows getrs's
 // op = T order (roclapack_getrs.hpp:134-150).
 #include "internal.hpp"
+#include "mfma.hpp"
 
 namespace rsa
 {
 
-constexpr int OT = 64; // output tile
-constexpr int OK = 16; // right-hand sides per LDS round
+constexpr int OR = 4; // 16-row tiles of an output column group per wavefront
+constexpr int OK = 4; // matrix-core steps (4 right-hand sides each) whose loads are in flight
 
-// dA[i0:i0+64, j0:j0+64] = -sum_c dB[i, c] X[j, c]; one workgroup per tile and
-// matrix, each thread 16 outputs, writes coalesced along columns of dA.
+// dA = -sum_c dB[:, c] X[:, c]^T on the matrix cores: a wavefront forms 64 rows
+// of 16 columns, its operands straight from memory (the operands are swapped,
+// so that 16 lanes write 16 consecutive rows).  The products accumulate from
+// zero as a chain of fused multiply-adds with c increasing.
+//
+// Bound by writing dA.  No LDS and no barrier, and only the 16-column groups
+// and 16-row tiles that hold entries of dA are formed: 64x64 tiles staged in
+// LDS with 16 vector fused multiply-adds per staged value took 73 us at n = 96
+// x 2048, 16 right-hand sides (151 MB of dA); this kernel takes 49 us.
 template <typename T>
 __global__ __launch_bounds__(256) void outer_neg_kernel(int n, int nrhs, Batch<T> DB, int lddb,
                                                         Batch<T> XX, int ldx, Batch<T> DA,
                                                         int ldda, int64_t boff)
 {
-    __shared__ T sB[OK][OT + 1];
-    __shared__ T sX[OK][OT + 1];
-    const int64_t b = blockIdx.z + boff;
-    const T* dB = DB[b];
-    const T* X = XX[b];
-    T* dA = DA[b];
-    const int i0 = blockIdx.x * OT, j0 = blockIdx.y * OT;
-    const int tid = threadIdx.x;
-    const int ti = tid % OT;       // row within the tile
-    const int tj = (tid / OT) * 16; // first of 16 columns
-    T acc[16];
+    using M = mfma16<T>;
+    const int64_t b = blockIdx.y + boff;
+    const int lane = threadIdx.x & 63;
+    const unsigned groups = unsigned(n + 15) / 16;
+    const unsigned unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i0 = int(unit / groups) * 16 * OR;
+    const int j0 = int(unit % groups) * 16;
+    if(i0 >= n)
+        return;
+    const int l16 = lane & 15, g = lane >> 4;
+    const T* dB = DB[b] + i0 + l16 + int64_t(g) * lddb;
+    const T* X = XX[b] + j0 + l16 + int64_t(g) * ldx;
+    const int left = n - i0 - l16; // row 16 t + l16 of the wavefront's rows exists: 16 t < left
+    const bool xin = j0 + l16 < n;
+    typename M::acc_t acc[OR];
 #pragma unroll
-    for(int q = 0; q < 16; ++q)
-        acc[q] = T(0);
-    for(int c0 = 0; c0 < nrhs; c0 += OK)
+    for(int t = 0; t < OR; ++t)
+        acc[t] = typename M::acc_t{0, 0, 0, 0};
+    for(int c0 = 0; c0 < nrhs; c0 += 4 * OK) // uniform
     {
-        __syncthreads();
-        for(int e = tid; e < OK * OT; e += 256)
-        {
-            const int r = e % OT, c = e / OT;
-            const bool okc = c0 + c < nrhs;
-            sB[c][r] = (okc && i0 + r < n) ? dB[(i0 + r) + int64_t(c0 + c) * lddb] : T(0);
-            sX[c][r] = (okc && j0 + r < n) ? X[(j0 + r) + int64_t(c0 + c) * ldx] : T(0);
-        }
-        __syncthreads();
+        T xv[OK], bv[OK][OR];
 #pragma unroll
-        for(int c = 0; c < OK; ++c)
+        for(int q = 0; q < OK; ++q)
         {
-            const T bi = sB[c][ti];
+            const int c = c0 + 4 * q;
+            const bool in = c + g < nrhs;
+            xv[q] = in && xin ? X[int64_t(c) * ldx] : T(0);
 #pragma unroll
-            for(int q = 0; q < 16; ++q)
-                acc[q] = fma_t(bi, sX[c][tj + q], acc[q]);
+            for(int t = 0; t < OR; ++t)
+                bv[q][t] = in && 16 * t < left ? dB[16 * t + int64_t(c) * lddb] : T(0);
         }
+#pragma unroll
+        for(int q = 0; q < OK; ++q)
+#pragma unroll
+            for(int t = 0; t < OR; ++t)
+                acc[t] = M::run(xv[q], bv[q][t], acc[t]);
     }
-    const int i = i0 + ti;
-    if(i < n)
-    {
+    T* dA = DA[b] + i0 + l16;
 #pragma unroll
-        for(int q = 0; q < 16; ++q)
-        {
-            const int j = j0 + tj + q;
-            if(j < n)
-                dA[i + int64_t(j) * ldda] = -acc[q];
-        }
+    for(int r = 0; r < 4; ++r)
+    {
+        const int j = j0 + M::row(lane, r);
+#pragma unroll
+        for(int t = 0; t < OR; ++t)
+            if(j < n && 16 * t < left)
+                dA[16 * t + int64_t(j) * ldda] = -acc[t][r];
     }
 }
 
@@ -93,25 +103,32 @@ rocblas_status gesv_adjoint(hipStream_t stream, int n, int nrhs, Batch<T> LU, in
     constexpr int64_t MAXYZ = 65535;
     if(nrhs > 0)
     {
-        // dB = dX, then dB = A^-T dB
-        for(int64_t b0 = 0; b0 < bc; b0 += MAXYZ)
-        {
-            const int nb = int((bc - b0) < MAXYZ ? (bc - b0) : MAXYZ);
-            const int gx = ceil_div(int64_t(n) * nrhs, 256) < 64 ? ceil_div(int64_t(n) * nrhs, 256)
-                                                                : 64;
-            hipLaunchKernelGGL((copy_cols_kernel<T>), dim3(gx, nb), dim3(256), 0, stream, n, nrhs,
-                               dX, lddx, dB, lddb, b0);
-            RSA_LAUNCH_CHECK();
-        }
+        const bool fused = n > SMALL_MAX && n <= FUSED_MAX && fits_buffer<T>(lda, n)
+                           && fits_buffer<T>(lddx, nrhs) && fits_buffer<T>(lddb, nrhs);
         rocblas_status st;
-        if(n <= SMALL_MAX)
-            st = getrs_small<T>(stream, true, n, nrhs, LU, lda, ipiv, strideP, dB, lddb, bc, true);
-        else if(n <= FUSED_MAX && fits_buffer<T>(lda, n) && fits_buffer<T>(lddb, nrhs))
-            st = getrs_fused<T>(stream, true, n, nrhs, LU, lda, ipiv, strideP, dB, lddb, dB,
-                                   lddb, bc, nullptr);
+        if(fused) // reads dX, writes dB
+            st = getrs_fused<T>(stream, true, n, nrhs, LU, lda, ipiv, strideP, dX, lddx, dB, lddb,
+                                bc, nullptr);
         else
-            st = getrs_blocked<T>(stream, true, n, nrhs, LU, lda, ipiv, strideP, dB, lddb, bc, true,
-                                  nullptr);
+        {
+            // dB = dX, then dB = A^-T dB
+            for(int64_t b0 = 0; b0 < bc; b0 += MAXYZ)
+            {
+                const int nb = int((bc - b0) < MAXYZ ? (bc - b0) : MAXYZ);
+                const int gx = ceil_div(int64_t(n) * nrhs, 256) < 64
+                                   ? ceil_div(int64_t(n) * nrhs, 256)
+                                   : 64;
+                hipLaunchKernelGGL((copy_cols_kernel<T>), dim3(gx, nb), dim3(256), 0, stream, n,
+                                   nrhs, dX, lddx, dB, lddb, b0);
+                RSA_LAUNCH_CHECK();
+            }
+            if(n <= SMALL_MAX)
+                st = getrs_small<T>(stream, true, n, nrhs, LU, lda, ipiv, strideP, dB, lddb, bc,
+                                    true);
+            else
+                st = getrs_blocked<T>(stream, true, n, nrhs, LU, lda, ipiv, strideP, dB, lddb, bc,
+                                      true, nullptr);
+        }
         if(st != rocblas_status_success)
             return st;
     }
@@ -119,7 +136,9 @@ rocblas_status gesv_adjoint(hipStream_t stream, int n, int nrhs, Batch<T> LU, in
     for(int64_t b0 = 0; b0 < bc; b0 += MAXYZ)
     {
         const int nb = int((bc - b0) < MAXYZ ? (bc - b0) : MAXYZ);
-        dim3 grid(ceil_div(n, OT), ceil_div(n, OT), nb);
+        // four wavefronts a workgroup, each 16 OR rows of 16 columns
+        const int64_t units = int64_t(ceil_div(n, 16)) * ceil_div(n, 16 * OR);
+        const dim3 grid(unsigned(ceil_div(units, 4)), nb);
         hipLaunchKernelGGL((outer_neg_kernel<T>), grid, dim3(256), 0, stream, n, nrhs, dB, lddb, X,
                            ldx, dA, ldda, b0);
         RSA_LAUNCH_CHECK();

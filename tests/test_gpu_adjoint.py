@@ -72,3 +72,51 @@ def test_adjoint_central_differences(torch_gpu):
         Bm[b, c, i] -= h
         fd = (loss(A.detach(), Bp) - loss(A.detach(), Bm)) / (2 * h)
         assert abs(fd - float(B.grad[b, c, i])) <= 1e-6 * max(1.0, abs(fd))
+
+
+@pytest.mark.parametrize("n,nrhs", [(1, 1), (15, 3), (16, 4), (17, 5), (63, 15), (64, 16), (65, 17), (80, 33),
+                                    (129, 1), (513, 2)])
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+def test_adjoint_padded_and_in_place(torch_gpu, n, nrhs, dtype):
+    """Through the C ABI with leading dimensions above n, each different, dX apart from dB and
+    the same buffer: dB and dA within the forward-error bound of the FP64 closed form (with the
+    stored X), edges of the outer product's 16-column groups, 64-row blocks and 16-column
+    rounds; padding untouched; both forms bit-identical."""
+    torch = torch_gpu
+    import rocsolver_amd as ra
+    print(f"adjoint padded n={n} nrhs={nrhs} {dtype}", flush=True)
+    dt, bc = getattr(torch, dtype), 3
+    p = "d" if dtype == "float64" else "s"
+    eps = float(np.finfo(getattr(np, dtype)).eps)
+    g = torch.Generator().manual_seed(n)
+    lda, ldx, ldg, ldb, ldda = n + 2, n + 3, n + 1, n + 1, n + 4
+    A = torch.randn(bc, n, lda, dtype=torch.float64, generator=g).to(dt)
+    A[:, torch.arange(n), torch.arange(n)] += 2.0 * n
+    X = torch.randn(bc, nrhs, ldx, dtype=torch.float64, generator=g).to(dt)
+    G = torch.randn(bc, nrhs, ldg, dtype=torch.float64, generator=g).to(dt)
+    M = A[:, :, :n].double()  # the transpose of each matrix
+    dB_ref = torch.linalg.solve(M, G[:, :, :n].double().transpose(1, 2)).transpose(1, 2)
+    dA_ref = -torch.bmm(X[:, :, :n].double().transpose(1, 2).contiguous(), dB_ref.contiguous())
+    got = []
+    with ra.Handle() as h:
+        LU = A.cuda()
+        ipiv, _ = ra.getrf(h, LU, m=n)
+        Xd = X.cuda()
+        for same in (False, True):
+            Gd = G.cuda()
+            dB = Gd if same else torch.full((bc, nrhs, ldb), 7.0, dtype=dt, device="cuda")
+            dA = torch.full((bc, n, ldda), 7.0, dtype=dt, device="cuda")
+            ra.check(f"rocsolver_amd_{p}gesv_adjoint_strided_batched", h.value, n, nrhs,
+                     LU.data_ptr(), lda, n * lda, ipiv.data_ptr(), ipiv.stride(0), Xd.data_ptr(),
+                     ldx, nrhs * ldx, Gd.data_ptr(), ldg, nrhs * ldg, dB.data_ptr(), ldb,
+                     nrhs * ldb, dA.data_ptr(), ldda, n * ldda, bc)
+            torch.cuda.synchronize()
+            if not same:
+                assert torch.equal(Gd.cpu(), G) and bool((dB[:, :, n:] == 7.0).all())
+            assert bool((dA[:, :, n:] == 7.0).all())
+            got.append((dB[:, :, :n].cpu(), dA[:, :, :n].cpu()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    kappa = float(torch.linalg.cond(M).max())
+    for g_, ref in zip(got[0], (dB_ref, dA_ref)):
+        err = (g_.double() - ref).abs().max() / ref.abs().max()
+        assert float(err) < 10 * kappa * n * eps, float(err)
