@@ -103,7 +103,9 @@ rocblas_status gesv_adjoint(hipStream_t stream, int n, int nrhs, Batch<T> LU, in
     constexpr int64_t MAXYZ = 65535;
     if(nrhs > 0)
     {
-        const bool fused = n > SMALL_MAX && n <= FUSED_MAX && fits_buffer<T>(lda, n)
+        const bool fused = n <= FUSED_MAX
+                           && (n > SMALL_MAX || getrs_small_by_tiles<T>(n, nrhs, bc))
+                           && fits_buffer<T>(lda, n)
                            && fits_buffer<T>(lddx, nrhs) && fits_buffer<T>(lddb, nrhs);
         rocblas_status st;
         if(fused) // reads dX, writes dB

@@ -108,12 +108,16 @@ rocblas_status getrs_impl(rocblas_handle handle, rocblas_operation trans, int n,
         return rocblas_status_success;
     hipStream_t stream;
     rocblas_get_stream(handle, &stream);
+    const bool fits = fits_buffer<T>(lda, n) && fits_buffer<T>(ldb, nrhs);
     if(n <= SMALL_MAX)
     {
         RSA_LOG_STAGE(handle, "getrs_small", "n", n, "nrhs", nrhs, "trans", trans, "bc", bc);
+        if(fits && getrs_small_by_tiles<T>(n, nrhs, bc))
+            return getrs_fused<T>(stream, tr, n, nrhs, A, lda, ipiv, strideP, B, ldb, B, ldb, bc,
+                                  nullptr);
         return getrs_small<T>(stream, tr, n, nrhs, A, lda, ipiv, strideP, B, ldb, bc, true);
     }
-    if(n <= FUSED_MAX && fits_buffer<T>(lda, n) && fits_buffer<T>(ldb, nrhs))
+    if(n <= FUSED_MAX && fits)
     {
         RSA_LOG_STAGE(handle, "getrs_fused", "n", n, "nrhs", nrhs, "trans", trans, "bc", bc);
         return getrs_fused<T>(stream, tr, n, nrhs, A, lda, ipiv, strideP, B, ldb, B, ldb, bc,

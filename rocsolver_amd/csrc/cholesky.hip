@@ -311,7 +311,7 @@ __global__ __launch_bounds__(NT, NT == 64 ? 2 : 4) void potrf_kernel(int n, Batc
 // non-unit triangular solves with the factor.  skip[b] != 0: B of system b is
 // left unchanged (posv after a failed factorisation).
 template <typename T, int NMAX, int NT, bool UP>
-__global__ __launch_bounds__(NT, sizeof(T) == 4 ? 4 : NMAX == 64 ? 3 : NMAX < NT ? 4 : 2) void potrs_fused_kernel(
+__global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void potrs_fused_kernel(
     int n, int nrhs, Batch<T> AA, int lda, Batch<T> BB, int ldb, int bc, unsigned chunks,
     const int* __restrict__ skip)
 {

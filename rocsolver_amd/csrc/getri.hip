@@ -3,7 +3,7 @@
 //
 // inv(A) is computed as the solution X of A X = I with the triangular-solve
 // kernels of the LU path (the row interchanges of ipiv applied to I, then the
-// unit-lower and upper solves; for 64 < n <= 512 inverse_tile_kernel forms
+// unit-lower and upper solves; up to n = 512 inverse_tile_kernel mostly forms
 // the columns of I itself), which is how the reference computes its
 // out-of-place inverse (roclapack_getri_outofplace.hpp:100-127).  The in-place
 // form (roclapack_getri.hpp:265-378 solves inv(A) L = inv(U) instead) works
@@ -94,7 +94,7 @@ static dim3 square_grid(int n, int bc)
 // no right-hand side is written or read: dgetri n = 100 x 2000 0.81 -> 0.68
 // ms with its two copies.
 template <typename T, int NMAX, int NT, int CT>
-__global__ __launch_bounds__(NT, sizeof(T) == 4 || NMAX < NT ? 4 : 2) void inverse_tile_kernel(
+__global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void inverse_tile_kernel(
     int n, Batch<T> AA, int lda, const int* __restrict__ ipivA, int64_t strideP, Batch<T> XX,
     int ldx, int bc, unsigned chunks)
 {
@@ -104,6 +104,16 @@ __global__ __launch_bounds__(NT, sizeof(T) == 4 || NMAX < NT ? 4 : 2) void inver
         return;
     tile_inverse_body<T, NMAX, NT, CT>(n, int(chunk) * CT * TSC, AA[b], lda,
                                    ipivA ? ipivA + b * strideP : nullptr, XX[b], ldx);
+}
+
+// Tiles against the team solve of lu_small.hpp (eight columns of the inverse a
+// pass, several systems per wavefront), which is the faster one for small
+// orders in large batches.  Team against tiles, FP64: n = 64 x 8192 1.80
+// against 0.66 ms, n = 32 x 8192 248 against 183 us, n = 24 x 8192 148 against
+// 173 but x 1024 63 against 39, n = 16 x 1024 31 against 19.
+inline bool inverse_by_tiles(int n, int bc)
+{
+    return n > 24 || (n > 8 && bc <= 1024);
 }
 
 template <typename T>
@@ -134,7 +144,10 @@ static rocblas_status inverse_tiles(hipStream_t stream, int n, Batch<T> LU, int 
                                from(X), ldx, nb, unsigned(chunks));
         };
         constexpr int F = sizeof(T) == 8 ? 2 : 1; // as getrs_fused_launch
-        if(n <= 128)
+        if(n <= 64)
+            go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{},
+               integral_constant<int, 1>{});
+        else if(n <= 128)
             go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{},
                integral_constant<int, 1>{});
         else if(n <= 256)
@@ -157,7 +170,7 @@ rocblas_status getri_solve(hipStream_t stream, int n, Batch<T> LU, int ldlu, con
     hipLaunchKernelGGL((diag_zero_kernel<T>), dim3((bc + 3) / 4), dim3(256), 0, stream, n, LU,
                        ldlu, info, bc);
     RSA_LAUNCH_CHECK();
-    if(n > SMALL_MAX && n <= FUSED_MAX && fits_buffer<T>(ldlu, n) && fits_buffer<T>(ldx, n))
+    if(inverse_by_tiles(n, bc) && n <= FUSED_MAX && fits_buffer<T>(ldlu, n) && fits_buffer<T>(ldx, n))
         return inverse_tiles<T>(stream, n, LU, ldlu, pivot ? ipiv : nullptr, strideP, X, ldx, bc);
     hipLaunchKernelGGL((set_identity_kernel<T>), square_grid(n, bc), dim3(256), 0, stream, n, X,
                        ldx, bc);

@@ -1,5 +1,5 @@
 // getrs_fused.hpp -- one-workgroup-per-system triangular solves with the LU
-// of getrf, for SMALL_MAX < n <= FUSED_MAX (reference order of operations:
+// of getrf, for n <= FUSED_MAX (reference order of operations:
 // library/src/lapack/roclapack_getrs.hpp:117-150 -- laswp, then L, then U for
 // op = N; U^T, L^T, then the reverse interchanges for op = T).  The factors
 // are read through a buffer resource: lda * n * sizeof(T) must be below 2^31
@@ -7,10 +7,10 @@
 //
 // Two kernels with the same operations per row, so bit-identical results:
 //   * the tile solver of tile_solve.hpp, 16 right-hand sides per workgroup;
-//   * the row solver of trsv_rows.hpp, thread i owning row i of up to four
-//     right-hand sides, for large batches with few of them: there the read
-//     of the factors bounds the call, and its smaller workgroups keep twice
-//     the systems in flight.
+//   * beyond n = 64, the row solver of trsv_rows.hpp, thread i owning row i of
+//     up to four right-hand sides, for large batches with few of them: there
+//     the read of the factors bounds the call, and its smaller workgroups
+//     keep twice the systems in flight.
 #pragma once
 
 #include "tile_solve.hpp"
@@ -21,10 +21,8 @@
 namespace rsa
 {
 
-// Wavefronts per SIMD that the registers are cut for: two tiles a wavefront
-// fit four, four tiles two in FP64.
 template <typename T, int NMAX, int NT, bool TRANS>
-__global__ __launch_bounds__(NT, sizeof(T) == 4 || NMAX < NT ? 4 : 2) void getrs_tile_kernel(
+__global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void getrs_tile_kernel(
     int n, int nrhs, Batch<T> AA, int lda, const int* __restrict__ ipivA, int64_t strideP,
     Batch<T> BB, int ldb, Batch<T> XX, int ldx, int bc, unsigned chunks,
     const int* __restrict__ skip)
@@ -112,7 +110,7 @@ rocblas_status getrs_fused_launch(hipStream_t stream, bool trans, int n, int nrh
     using std::integral_constant;
     if(bc <= 0 || n <= 0 || nrhs <= 0)
         return rocblas_status_success;
-    if(getrs_by_rows<T>(trans, n, nrhs, bc))
+    if(n > SMALL_MAX && getrs_by_rows<T>(trans, n, nrhs, bc))
     {
         auto go = [&](auto nmax, auto nr, auto tr) {
             constexpr int NMAX = decltype(nmax)::value;
@@ -168,7 +166,9 @@ rocblas_status getrs_fused_launch(hipStream_t stream, bool trans, int n, int nrh
         // against 91 with four, n = 256 x 4096 681 against 713); FP32: four
         // (49 against 58 us, 367 against 493)
         constexpr int F = sizeof(T) == 8 ? 2 : 1;
-        if(n <= 128)
+        if(n <= 64)
+            go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{});
+        else if(n <= 128)
             go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{});
         else if(n <= 256)
             go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});

@@ -62,13 +62,37 @@ rocblas_status lu_fused_invdiag(hipStream_t stream, int n, Batch<double> AI, int
                                 Batch<float> AO, int ldo, int* ipiv, int64_t strideP, int* info,
                                 int bc);
 
-// One-workgroup-per-system solve with the LU of getrf for SMALL_MAX < n <=
-// FUSED_MAX; reads the right-hand sides from B, writes the solution to X (may
+// One-workgroup-per-system solve with the LU of getrf for n <= FUSED_MAX; reads the right-hand sides from B, writes the solution to X (may
 // be B).  Entries with skip[b] != 0 are not touched.
 template <typename T>
 rocblas_status getrs_fused(hipStream_t stream, bool trans, int n, int nrhs, Batch<T> A, int lda,
                            const int* ipiv, int64_t strideP, Batch<T> B, int ldb, Batch<T> X,
                            int ldx, int bc, const int* skip);
+
+// Which solve for n <= SMALL_MAX: the team kernels of lu_small.hpp (eight
+// right-hand sides a pass, several systems per wavefront) or getrs_fused's
+// tiles (16 a pass, a workgroup per system); the same operations in the same
+// order.  The team's pass takes a wavefront per system beyond n = 32 and is a
+// chain of n broadcasts, so tiles are the faster ones for large orders, many
+// right-hand sides or few systems.  Team against tile kernels, op T:
+//   n = 56 x 8192, 8 right-hand sides: FP64 223 against 164 us, FP32 148
+//     against 118 (1 right-hand side: 0.6 to 0.8 of the tiles' time);
+//   n = 40 x 8192, 17 right-hand sides: FP64 405 against 307 us, FP32 241
+//     against 208 (n = 33: FP32 1.05 times slower);
+//   n = 32 x 1024, 8 right-hand sides: FP64 25 against 16 us, FP32 21 against
+//     15 (x 8192: 1.3 times slower).
+template <typename T>
+inline bool getrs_small_by_tiles(int n, int nrhs, int bc)
+{
+    const bool few = bc <= 1024; // four systems per CU
+    if(nrhs <= 1)
+        return false;
+    if(n > 48)
+        return true;
+    if(n > 32)
+        return nrhs > 8 ? few || sizeof(T) == 8 || n >= 40 : few && n >= 40;
+    return few && (n > 24 || (n >= 20 && nrhs > 8));
+}
 
 // -------------------------------------------------------------- blocked path
 // Register-resident panel A[j0:m, j0:j0+jb], jb <= panel_reg_width(m - j0)

@@ -45,6 +45,14 @@ constexpr int tile_solve_tpw()
     return NMAX / 16 / (NT / 64);
 }
 
+// Wavefronts per SIMD that the registers are cut for: two tiles a wavefront
+// fit four, four tiles two in FP64.
+template <typename T, int NMAX, int NT>
+constexpr int tile_waves()
+{
+    return sizeof(T) == 4 ? 4 : NMAX == 64 ? 3 : NMAX < NT ? 4 : 2;
+}
+
 // op(T) X = acc in place, T the lower (forward) or upper (backward) triangle
 // of op(A).  Rows past n are zero in and out.  par: parity of the LDS buffers.
 // A forward solve starts at block `begin` (the rows before it are zero).  CT

@@ -59,3 +59,47 @@ def test_singular_factor_stays_in_its_column(torch_gpu, handle, trans):
     X = X.cpu().numpy()
     np.testing.assert_array_equal(np.isfinite(X), np.isfinite(Xo))
     np.testing.assert_allclose(X[[0, 2]], Xo[[0, 2]], rtol=0, atol=n * np.finfo(float).eps * np.abs(Xo[[0, 2]]).max())
+
+
+# orders up to 64 on both sides of the rule that gives a call to the tile solver (by the order,
+# the right-hand sides and the batch), partial and whole blocks of 32 rows
+@pytest.mark.parametrize("n", [19, 20, 24, 25, 32, 33, 39, 40, 48, 49, 63, 64])
+@pytest.mark.parametrize("nrhs,bc", [(2, 5), (9, 5), (17, 5), (9, 1025)])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_small_orders_equal_the_oracle(torch_gpu, handle, n, nrhs, bc, trans, dtype):
+    """Bit for bit, with lda > n and ldb > n, a singular system (infinities and NaN where the
+    oracle has them) and untouched padding rows, in the strided and the pointer-array form."""
+    print(f"getrs n={n} nrhs={nrhs} bc={bc} {trans} {dtype.__name__}", flush=True)
+    g = np.random.default_rng(n * 7 + nrhs)
+    lda, ldb = n + 3, n + 2
+    LU = (g.uniform(-1, 1, size=(bc, n, lda)) / np.sqrt(n)).astype(dtype)
+    LU[:, np.arange(n), np.arange(n)] += np.asarray(2, dtype)
+    LU[1, n - 2, n - 2] = 0
+    ipiv = np.stack([g.integers(np.arange(1, n + 1), n + 1) for _ in range(bc)]).astype(np.int32)
+    B = g.uniform(-1, 1, size=(bc, nrhs, ldb)).astype(dtype)
+    Xo = B.copy()
+    with np.errstate(all="ignore"):
+        oracle.getrs(trans, LU, n, ipiv, Xo)
+    for batched in (False, True):
+        X = torch_gpu.from_numpy(B.copy()).cuda()
+        ra.getrs(handle, torch_gpu.from_numpy(LU).cuda(), torch_gpu.from_numpy(ipiv).cuda(), X,
+                 trans=trans, batched=batched)
+        np.testing.assert_array_equal(X.cpu().numpy(), Xo)
+
+
+@pytest.mark.parametrize("n", [8, 9, 16, 17, 24, 25, 33, 64])
+@pytest.mark.parametrize("bc", [1, 1024, 1025])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_small_inverses_equal_the_solve_for_the_identity(torch_gpu, handle, n, bc, dtype):
+    print(f"getri n={n} bc={bc} {dtype.__name__}", flush=True)
+    g = np.random.default_rng(n)
+    one = (g.uniform(-1, 1, size=(1, n, n)) / np.sqrt(n)).astype(dtype)
+    one[:, np.arange(n), np.arange(n)] += np.asarray(2, dtype)
+    ipiv = g.integers(np.arange(1, n + 1), n + 1).astype(np.int32)[None]
+    want = np.eye(n, dtype=dtype)[None].copy()
+    oracle.getrs("N", one, n, ipiv, want)
+    inv = torch_gpu.from_numpy(one).cuda().repeat(bc, 1, 1)
+    info = ra.getri(handle, inv, torch_gpu.from_numpy(ipiv).cuda().repeat(bc, 1))
+    assert not bool(info.any())
+    assert torch_gpu.equal(inv, torch_gpu.from_numpy(want).cuda().expand(bc, n, n))
