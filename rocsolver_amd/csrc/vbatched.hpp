@@ -90,8 +90,14 @@ __device__ __forceinline__ void vb_small_pack(const VbArgs<T>& a, const int* __r
                                               int (*perm)[64], int (*spiv)[64])
 {
     constexpr int TPW = 64 / TS;
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
+    // Formed here, not at kernel entry, where the large matrices' body would
+    // keep the lane numbers of every pack alive and spill them (FP64 gesv: 124
+    // bytes of scratch a lane, now 12).  1000 matrices of orders 4..64, 8
+    // right-hand sides, FP64: gesv 245 -> 222 us, getrs 217 -> 139; 8000 of
+    // orders 65..512 gesv 20.5 -> 19.7 ms.
+    const int tid = fresh_tid();
+    const int lane = tid & 63;
+    const int w = tid >> 6;
     const int team = lane / TS;
     const int row = lane % TS;
     // uniform trip count per wavefront; a team past the end idles
