@@ -313,13 +313,13 @@ __global__ __launch_bounds__(NT, NT == 64 ? 2 : 4) void potrf_kernel(int n, Batc
 template <typename T, int NMAX, int NT, bool UP>
 __global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void potrs_fused_kernel(
     int n, int nrhs, Batch<T> AA, int lda, Batch<T> BB, int ldb, int bc, unsigned chunks,
-    const int* __restrict__ skip)
+    unsigned chunk0, const int* __restrict__ skip)
 {
     unsigned chunk;
     const int64_t b = tile_solve_system(blockIdx.x, chunks, chunk);
     if(b >= bc || (skip && skip[b] != 0))
         return;
-    const int c0 = int(chunk) * TSC;
+    const int c0 = int(chunk0 + chunk) * TSC;
     const int cend = nrhs - c0 < TSC ? nrhs : c0 + TSC;
     tile_solve_body<T, NMAX, NT, UP ? TILE_CHOL_U : TILE_CHOL_L, false>(
         n, c0, cend, AA[b], lda, nullptr, BB[b], ldb, BB[b], ldb);
@@ -363,30 +363,26 @@ rocblas_status potrf(hipStream_t stream, bool up, int n, Batch<T> A, int lda, in
         return rocblas_status_success;
     if(n <= 0)
         return reset_info(stream, info, bc);
-    for(int64_t b0 = 0; b0 < bc; b0 += 1 << 30)
-    {
-        const int cnt = int((bc - b0) < (1 << 30) ? (bc - b0) : (1 << 30));
-        Batch<T> Ab = A.ptrs ? Batch<T>{nullptr, A.ptrs + b0, 0}
-                             : Batch<T>{A.base + b0 * A.stride, nullptr, A.stride};
-        auto go = [&](auto nt) {
-            constexpr int NT = decltype(nt)::value;
+    auto go = [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        return launch_split(bc, 1, NT, 1, [&](int64_t b0, int64_t nb, int64_t, int64_t) {
+            const dim3 grid{unsigned(nb)};
             if(up)
-                hipLaunchKernelGGL((potrf_kernel<T, NT, true>), dim3(cnt), dim3(NT), 0, stream, n,
-                                   Ab, lda, info + b0);
+                hipLaunchKernelGGL((potrf_kernel<T, NT, true>), grid, dim3(NT), 0, stream, n,
+                                   batch_from(A, b0), lda, info + b0);
             else
-                hipLaunchKernelGGL((potrf_kernel<T, NT, false>), dim3(cnt), dim3(NT), 0, stream, n,
-                                   Ab, lda, info + b0);
-        };
-        // as many wavefronts as the first block column gives 16-row groups
-        if(n <= 64)
-            go(std::integral_constant<int, 64>{});
-        else if(n <= 128)
-            go(std::integral_constant<int, 128>{});
-        else
-            go(std::integral_constant<int, 256>{});
-        RSA_LAUNCH_CHECK();
-    }
-    return rocblas_status_success;
+                hipLaunchKernelGGL((potrf_kernel<T, NT, false>), grid, dim3(NT), 0, stream, n,
+                                   batch_from(A, b0), lda, info + b0);
+            RSA_LAUNCH_CHECK();
+            return rocblas_status_success;
+        });
+    };
+    // as many wavefronts as the first block column gives 16-row groups
+    if(n <= 64)
+        return go(std::integral_constant<int, 64>{});
+    if(n <= 128)
+        return go(std::integral_constant<int, 128>{});
+    return go(std::integral_constant<int, 256>{});
 }
 
 template <typename T>
@@ -397,44 +393,37 @@ rocblas_status potrs(hipStream_t stream, bool up, int n, int nrhs, Batch<T> A, i
         return rocblas_status_success;
     if(n <= FUSED_MAX && fits_buffer<T>(lda, n) && fits_buffer<T>(ldb, nrhs))
     {
-        const int chunks = ceil_div(nrhs, TSC);
-        // one launch per 2^30 workgroups at most
-        const int64_t most = (int64_t(1) << 30) / chunks / TILE_XCDS * TILE_XCDS;
-        const int64_t step = most > 0 ? most : TILE_XCDS;
-        for(int64_t b0 = 0; b0 < bc; b0 += step)
-        {
-            const int nb = int((bc - b0) < step ? (bc - b0) : step);
-            auto from = [&](Batch<T> V) {
-                return V.ptrs ? Batch<T>{nullptr, V.ptrs + b0, 0}
-                              : Batch<T>{V.base + b0 * V.stride, nullptr, V.stride};
-            };
-            auto go = [&](auto nmax, auto nt) {
-                constexpr int NMAX = decltype(nmax)::value;
-                constexpr int NT = decltype(nt)::value;
-                const dim3 grid(unsigned(tile_solve_grid(nb, chunks)));
-                const int* sk = skip ? skip + b0 : nullptr;
-                if(up)
-                    hipLaunchKernelGGL((potrs_fused_kernel<T, NMAX, NT, true>), grid, dim3(NT), 0,
-                                       stream, n, nrhs, from(A), lda, from(B), ldb, nb,
-                                       unsigned(chunks), sk);
-                else
-                    hipLaunchKernelGGL((potrs_fused_kernel<T, NMAX, NT, false>), grid, dim3(NT), 0,
-                                       stream, n, nrhs, from(A), lda, from(B), ldb, nb,
-                                       unsigned(chunks), sk);
-            };
-            using std::integral_constant;
-            constexpr int F = sizeof(T) == 8 ? 2 : 1; // as getrs_fused_launch
-            if(n <= 64)
-                go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{});
-            else if(n <= 128)
-                go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{});
-            else if(n <= 256)
-                go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});
-            else
-                go(integral_constant<int, 512>{}, integral_constant<int, 512>{});
-            RSA_LAUNCH_CHECK();
-        }
-        return rocblas_status_success;
+        auto go = [&](auto nmax, auto nt) {
+            constexpr int NMAX = decltype(nmax)::value;
+            constexpr int NT = decltype(nt)::value;
+            return launch_split(
+                bc, ceil_div(nrhs, TSC), NT, TILE_XCDS,
+                [&](int64_t b0, int64_t nb, int64_t c0, int64_t nc) {
+                    const dim3 grid{unsigned(tile_solve_grid(int(nb), int(nc)))};
+                    const int* sk = skip ? skip + b0 : nullptr;
+                    if(up)
+                        hipLaunchKernelGGL((potrs_fused_kernel<T, NMAX, NT, true>), grid, dim3(NT),
+                                           0, stream, n, nrhs, batch_from(A, b0), lda,
+                                           batch_from(B, b0), ldb, int(nb), unsigned(nc),
+                                           unsigned(c0), sk);
+                    else
+                        hipLaunchKernelGGL((potrs_fused_kernel<T, NMAX, NT, false>), grid, dim3(NT),
+                                           0, stream, n, nrhs, batch_from(A, b0), lda,
+                                           batch_from(B, b0), ldb, int(nb), unsigned(nc),
+                                           unsigned(c0), sk);
+                    RSA_LAUNCH_CHECK();
+                    return rocblas_status_success;
+                });
+        };
+        using std::integral_constant;
+        constexpr int F = sizeof(T) == 8 ? 2 : 1; // as getrs_fused_launch
+        if(n <= 64)
+            return go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{});
+        if(n <= 128)
+            return go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{});
+        if(n <= 256)
+            return go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});
+        return go(integral_constant<int, 512>{}, integral_constant<int, 512>{});
     }
     const int64_t threads = int64_t(bc) * nrhs;
     hipLaunchKernelGGL((potrs_serial_kernel<T>), dim3(unsigned((threads + 63) / 64)), dim3(64), 0,

@@ -124,41 +124,34 @@ static rocblas_status inverse_tiles(hipStream_t stream, int n, Batch<T> LU, int 
     // 32 columns a workgroup beyond n = 128: n = 400 x 200 2.02 -> 1.35 ms, n =
     // 200 x 800 1.31 -> 1.13; no gain at n = 100 (0.68), 0.96 at n = 128 x 100
     const int cols = n <= 128 ? TSC : 2 * TSC;
-    const int chunks = ceil_div(n, cols);
-    // one launch per 2^30 workgroups at most
-    const int64_t step = (int64_t(1) << 30) / chunks / TILE_XCDS * TILE_XCDS;
-    for(int64_t b0 = 0; b0 < bc; b0 += step)
-    {
-        const int nb = int((bc - b0) < step ? (bc - b0) : step);
-        auto from = [&](Batch<T> V) {
-            return V.ptrs ? Batch<T>{nullptr, V.ptrs + b0, 0}
-                          : Batch<T>{V.base + b0 * V.stride, nullptr, V.stride};
-        };
-        auto go = [&](auto nmax, auto nt, auto ct) {
-            constexpr int NMAX = decltype(nmax)::value;
-            constexpr int NT = decltype(nt)::value;
-            constexpr int CT = decltype(ct)::value;
-            hipLaunchKernelGGL((inverse_tile_kernel<T, NMAX, NT, CT>),
-                               dim3(unsigned(tile_solve_grid(nb, chunks))), dim3(NT), 0, stream, n,
-                               from(LU), ldlu, ipiv ? ipiv + b0 * strideP : nullptr, strideP,
-                               from(X), ldx, nb, unsigned(chunks));
-        };
-        constexpr int F = sizeof(T) == 8 ? 2 : 1; // as getrs_fused_launch
-        if(n <= 64)
-            go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{},
-               integral_constant<int, 1>{});
-        else if(n <= 128)
-            go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{},
-               integral_constant<int, 1>{});
-        else if(n <= 256)
-            go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{},
-               integral_constant<int, 2>{});
-        else
-            go(integral_constant<int, 512>{}, integral_constant<int, 512>{},
-               integral_constant<int, 2>{});
-        RSA_LAUNCH_CHECK();
-    }
-    return rocblas_status_success;
+    const int chunks = ceil_div(n, cols); // at most 16: never split
+    auto go = [&](auto nmax, auto nt, auto ct) {
+        constexpr int NMAX = decltype(nmax)::value;
+        constexpr int NT = decltype(nt)::value;
+        constexpr int CT = decltype(ct)::value;
+        return launch_split(
+            bc, chunks, NT, TILE_XCDS, [&](int64_t b0, int64_t nb, int64_t, int64_t) {
+                hipLaunchKernelGGL((inverse_tile_kernel<T, NMAX, NT, CT>),
+                                   dim3(unsigned(tile_solve_grid(int(nb), chunks))), dim3(NT), 0,
+                                   stream, n, batch_from(LU, b0), ldlu,
+                                   ipiv ? ipiv + b0 * strideP : nullptr, strideP,
+                                   batch_from(X, b0), ldx, int(nb), unsigned(chunks));
+                RSA_LAUNCH_CHECK();
+                return rocblas_status_success;
+            });
+    };
+    constexpr int F = sizeof(T) == 8 ? 2 : 1; // as getrs_fused_launch
+    if(n <= 64)
+        return go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{},
+                  integral_constant<int, 1>{});
+    if(n <= 128)
+        return go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{},
+                  integral_constant<int, 1>{});
+    if(n <= 256)
+        return go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{},
+                  integral_constant<int, 2>{});
+    return go(integral_constant<int, 512>{}, integral_constant<int, 512>{},
+              integral_constant<int, 2>{});
 }
 
 template <typename T>

@@ -24,14 +24,14 @@ namespace rsa
 template <typename T, int NMAX, int NT, bool TRANS>
 __global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void getrs_tile_kernel(
     int n, int nrhs, Batch<T> AA, int lda, const int* __restrict__ ipivA, int64_t strideP,
-    Batch<T> BB, int ldb, Batch<T> XX, int ldx, int bc, unsigned chunks,
+    Batch<T> BB, int ldb, Batch<T> XX, int ldx, int bc, unsigned chunks, unsigned chunk0,
     const int* __restrict__ skip)
 {
     unsigned chunk;
     const int64_t b = tile_solve_system(blockIdx.x, chunks, chunk);
     if(b >= bc || (skip && skip[b] != 0))
         return;
-    const int c0 = int(chunk) * TSC;
+    const int c0 = int(chunk0 + chunk) * TSC;
     const int cend = nrhs - c0 < TSC ? nrhs : c0 + TSC;
     tile_solve_body<T, NMAX, NT, TILE_LU, TRANS>(n, c0, cend, AA[b], lda, ipivA + b * strideP,
                                                  BB[b], ldb, XX[b], ldx);
@@ -116,67 +116,63 @@ rocblas_status getrs_fused_launch(hipStream_t stream, bool trans, int n, int nrh
             constexpr int NMAX = decltype(nmax)::value;
             constexpr int NR = decltype(nr)::value;
             constexpr bool TR = decltype(tr)::value;
-            hipLaunchKernelGGL((getrs_rows_kernel<T, NMAX, NR, TR>), dim3(bc), dim3(NMAX), 0,
-                               stream, n, nrhs, A, lda, ipiv, strideP, B, ldb, X, ldx, skip);
+            return launch_split(bc, 1, NMAX, 1, [&](int64_t b0, int64_t nb, int64_t, int64_t) {
+                hipLaunchKernelGGL((getrs_rows_kernel<T, NMAX, NR, TR>), dim3(unsigned(nb)),
+                                   dim3(NMAX), 0, stream, n, nrhs, batch_from(A, b0), lda,
+                                   ipiv + b0 * strideP, strideP, batch_from(B, b0), ldb,
+                                   batch_from(X, b0), ldx, skip ? skip + b0 : nullptr);
+                RSA_LAUNCH_CHECK();
+                return rocblas_status_success;
+            });
         };
         auto by_nrhs = [&](auto nmax, auto tr) {
-            if(nrhs == 1)
-                go(nmax, integral_constant<int, 1>{}, tr);
-            else
-                go(nmax, integral_constant<int, 4>{}, tr);
+            return nrhs == 1 ? go(nmax, integral_constant<int, 1>{}, tr)
+                             : go(nmax, integral_constant<int, 4>{}, tr);
         };
         if(trans)
-            by_nrhs(integral_constant<int, 128>{}, std::true_type{});
-        else if(n <= 128)
-            by_nrhs(integral_constant<int, 128>{}, std::false_type{});
-        else if(n <= 256)
-            by_nrhs(integral_constant<int, 256>{}, std::false_type{});
-        else if constexpr(sizeof(T) == 8)
-            by_nrhs(integral_constant<int, 512>{}, std::false_type{});
-        RSA_LAUNCH_CHECK();
-        return rocblas_status_success;
+            return by_nrhs(integral_constant<int, 128>{}, std::true_type{});
+        if(n <= 128)
+            return by_nrhs(integral_constant<int, 128>{}, std::false_type{});
+        if(n <= 256)
+            return by_nrhs(integral_constant<int, 256>{}, std::false_type{});
+        if constexpr(sizeof(T) == 8)
+            return by_nrhs(integral_constant<int, 512>{}, std::false_type{});
     }
-    const int chunks = ceil_div(nrhs, TSC);
-    // one launch per 2^30 workgroups at most
-    const int64_t most = (int64_t(1) << 30) / chunks / TILE_XCDS * TILE_XCDS;
-    const int64_t step = most > 0 ? most : TILE_XCDS;
-    for(int64_t b0 = 0; b0 < bc; b0 += step)
-    {
-        const int nb = int((bc - b0) < step ? (bc - b0) : step);
-        auto from = [&](Batch<T> V) {
-            return V.ptrs ? Batch<T>{nullptr, V.ptrs + b0, 0}
-                          : Batch<T>{V.base + b0 * V.stride, nullptr, V.stride};
-        };
-        auto go = [&](auto nmax, auto nt) {
-            constexpr int NMAX = decltype(nmax)::value;
-            constexpr int NT = decltype(nt)::value;
-            const dim3 grid(unsigned(tile_solve_grid(nb, chunks)));
-            if(trans)
-                hipLaunchKernelGGL((getrs_tile_kernel<T, NMAX, NT, true>), grid, dim3(NT), 0,
-                                   stream, n, nrhs, from(A), lda, ipiv + b0 * strideP, strideP,
-                                   from(B), ldb, from(X), ldx, nb, unsigned(chunks),
-                                   skip ? skip + b0 : nullptr);
-            else
-                hipLaunchKernelGGL((getrs_tile_kernel<T, NMAX, NT, false>), grid, dim3(NT), 0,
-                                   stream, n, nrhs, from(A), lda, ipiv + b0 * strideP, strideP,
-                                   from(B), ldb, from(X), ldx, nb, unsigned(chunks),
-                                   skip ? skip + b0 : nullptr);
-        };
-        // FP64: two tiles a wavefront up to n = 256 (n = 96 x 2048 78 us
-        // against 91 with four, n = 256 x 4096 681 against 713); FP32: four
-        // (49 against 58 us, 367 against 493)
-        constexpr int F = sizeof(T) == 8 ? 2 : 1;
-        if(n <= 64)
-            go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{});
-        else if(n <= 128)
-            go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{});
-        else if(n <= 256)
-            go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});
-        else
-            go(integral_constant<int, 512>{}, integral_constant<int, 512>{});
-        RSA_LAUNCH_CHECK();
-    }
-    return rocblas_status_success;
+    auto go = [&](auto nmax, auto nt) {
+        constexpr int NMAX = decltype(nmax)::value;
+        constexpr int NT = decltype(nt)::value;
+        return launch_split(
+            bc, ceil_div(nrhs, TSC), NT, TILE_XCDS,
+            [&](int64_t b0, int64_t nb, int64_t c0, int64_t nc) {
+                const dim3 grid{unsigned(tile_solve_grid(int(nb), int(nc)))};
+                const int* sk = skip ? skip + b0 : nullptr;
+                if(trans)
+                    hipLaunchKernelGGL((getrs_tile_kernel<T, NMAX, NT, true>), grid, dim3(NT), 0,
+                                       stream, n, nrhs, batch_from(A, b0), lda,
+                                       ipiv + b0 * strideP, strideP, batch_from(B, b0), ldb,
+                                       batch_from(X, b0), ldx, int(nb), unsigned(nc), unsigned(c0),
+                                       sk);
+                else
+                    hipLaunchKernelGGL((getrs_tile_kernel<T, NMAX, NT, false>), grid, dim3(NT), 0,
+                                       stream, n, nrhs, batch_from(A, b0), lda,
+                                       ipiv + b0 * strideP, strideP, batch_from(B, b0), ldb,
+                                       batch_from(X, b0), ldx, int(nb), unsigned(nc), unsigned(c0),
+                                       sk);
+                RSA_LAUNCH_CHECK();
+                return rocblas_status_success;
+            });
+    };
+    // FP64: two tiles a wavefront up to n = 256 (n = 96 x 2048 78 us
+    // against 91 with four, n = 256 x 4096 681 against 713); FP32: four
+    // (49 against 58 us, 367 against 493)
+    constexpr int F = sizeof(T) == 8 ? 2 : 1;
+    if(n <= 64)
+        return go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{});
+    if(n <= 128)
+        return go(integral_constant<int, 128>{}, integral_constant<int, 128 * F>{});
+    if(n <= 256)
+        return go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});
+    return go(integral_constant<int, 512>{}, integral_constant<int, 512>{});
 }
 
 } // namespace rsa

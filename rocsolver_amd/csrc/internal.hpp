@@ -4,9 +4,18 @@
 #pragma once
 
 #include "common.hpp"
+#include "launch_split.hpp"
 
 namespace rsa
 {
+
+// The batch from matrix b0 on.
+template <typename T>
+Batch<T> batch_from(Batch<T> V, int64_t b0)
+{
+    return V.ptrs ? Batch<T>{nullptr, V.ptrs + b0, 0}
+                  : Batch<T>{V.base + b0 * V.stride, nullptr, V.stride};
+}
 
 // Largest m, n handled by the register-resident small kernels.
 constexpr int SMALL_MAX = 64;

@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
                                                        int64_t offB, int ldb, Batch<T> CC,
                                                        int64_t offC, int ldc,
                                                        const int* __restrict__ skip, int bc,
-                                                       int tm, int tn)
+                                                       int tm, unsigned tile0, unsigned tiles)
 {
     using M_ = mfma16<T>;
     using acc_t = typename M_::acc_t;
@@ -361,21 +361,20 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
     __shared__ T sA[2][GK * SR];
     __shared__ T sB[2][GT * SC];
 
-    const unsigned tiles = unsigned(tm) * unsigned(tn);
     const unsigned id = blockIdx.x;
     int64_t b;
     unsigned tile;
     if(bc >= XCDS)
     {
         b = int64_t(id / (XCDS * tiles)) * XCDS + id % XCDS;
-        tile = (id / XCDS) % tiles;
+        tile = tile0 + (id / XCDS) % tiles;
         if(b >= bc)
             return;
     }
     else
     {
         b = id / tiles;
-        tile = id % tiles;
+        tile = tile0 + id % tiles;
     }
     if(skip && skip[b] != 0)
         return;
@@ -486,31 +485,25 @@ static rocblas_status gemm_sub(hipStream_t stream, int M, int N, int K, Batch<T>
 {
     if(M <= 0 || N <= 0 || K <= 0 || bc <= 0)
         return rocblas_status_success;
-    const int tm = ceil_div(M, GT), tn = ceil_div(N, GT);
-    const int64_t tiles = int64_t(tm) * tn;
-    // one launch per 2^30 workgroups at most (whole groups of XCDS matrices)
-    const int64_t most = (int64_t(1) << 30) / tiles / XCDS * XCDS;
-    const int64_t step = most > 0 ? most : 1;
-    for(int64_t b0 = 0; b0 < bc; b0 += step)
-    {
-        const int nb = int((bc - b0) < step ? (bc - b0) : step);
-        const int64_t wgs = tiles * (nb >= XCDS ? int64_t(ceil_div(nb, XCDS)) * XCDS : nb);
-        auto from = [&](Batch<T> X) {
-            return X.ptrs ? Batch<T>{nullptr, X.ptrs + b0, 0}
-                          : Batch<T>{X.base + b0 * X.stride, nullptr, X.stride};
-        };
-        const int* sk = skip ? skip + b0 : nullptr;
-        if(K <= 32)
-            hipLaunchKernelGGL((gemm_sub_kernel<T, true>), dim3(unsigned(wgs)), dim3(256), 0,
-                               stream, M, N, K, from(A), offA, lda, from(B), offB, ldb, from(C),
-                               offC, ldc, sk, nb, tm, tn);
-        else
-            hipLaunchKernelGGL((gemm_sub_kernel<T, false>), dim3(unsigned(wgs)), dim3(256), 0,
-                               stream, M, N, K, from(A), offA, lda, from(B), offB, ldb, from(C),
-                               offC, ldc, sk, nb, tm, tn);
-        RSA_LAUNCH_CHECK();
-    }
-    return rocblas_status_success;
+    const int tm = ceil_div(M, GT);
+    return launch_split(
+        bc, int64_t(tm) * ceil_div(N, GT), 256, XCDS,
+        [&](int64_t b0, int64_t nb, int64_t t0, int64_t nt) {
+            const int64_t wgs = nt * (nb >= XCDS ? int64_t(ceil_div(nb, XCDS)) * XCDS : nb);
+            const int* sk = skip ? skip + b0 : nullptr;
+            if(K <= 32)
+                hipLaunchKernelGGL((gemm_sub_kernel<T, true>), dim3(unsigned(wgs)), dim3(256), 0,
+                                   stream, M, N, K, batch_from(A, b0), offA, lda, batch_from(B, b0),
+                                   offB, ldb, batch_from(C, b0), offC, ldc, sk, int(nb), tm,
+                                   unsigned(t0), unsigned(nt));
+            else
+                hipLaunchKernelGGL((gemm_sub_kernel<T, false>), dim3(unsigned(wgs)), dim3(256), 0,
+                                   stream, M, N, K, batch_from(A, b0), offA, lda, batch_from(B, b0),
+                                   offB, ldb, batch_from(C, b0), offC, ldc, sk, int(nb), tm,
+                                   unsigned(t0), unsigned(nt));
+            RSA_LAUNCH_CHECK();
+            return rocblas_status_success;
+        });
 }
 
 // ----------------------------------------------------------------- getrf
@@ -679,7 +672,7 @@ constexpr int PERM_COLS = 8; // columns per workgroup
 template <typename T, int R>
 __global__ __launch_bounds__(PERM_THREADS) void permute_rows_kernel(
     int n, int nrhs, Batch<T> BB, int ldb, const int* __restrict__ ipivA, int64_t strideP,
-    int inverse, const int* __restrict__ skip, int64_t boff)
+    int inverse, const int* __restrict__ skip, unsigned group0, int64_t boff)
 {
     constexpr int ROWS = PERM_THREADS * R;
     __shared__ unsigned short s_row[ROWS]; // row now at each position
@@ -735,7 +728,7 @@ __global__ __launch_bounds__(PERM_THREADS) void permute_rows_kernel(
 #pragma unroll
     for(int r = 0; r < R; ++r)
         src[r] = s_row[tid + r * PERM_THREADS];
-    const int c0 = blockIdx.x * PERM_COLS;
+    const int c0 = int(group0 + blockIdx.x) * PERM_COLS;
     constexpr int UC = R <= 4 ? 4 : 2; // columns in flight
     for(int c1 = 0; c1 < PERM_COLS && c0 + c1 < nrhs; c1 += UC) // uniform
     {
@@ -768,19 +761,23 @@ static rocblas_status permute_rows(hipStream_t stream, int n, int nrhs, Batch<T>
     {
         const int nb = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);
         auto go = [&](auto r) {
-            hipLaunchKernelGGL((permute_rows_kernel<T, decltype(r)::value>),
-                               dim3(ceil_div(nrhs, PERM_COLS), nb), dim3(PERM_THREADS), 0, stream,
-                               n, nrhs, B, ldb, ipiv, strideP, int(inverse), skip, b0);
+            return launch_split(
+                1, ceil_div(nrhs, PERM_COLS), PERM_THREADS, 1,
+                [&](int64_t, int64_t, int64_t g0, int64_t ng) {
+                    hipLaunchKernelGGL((permute_rows_kernel<T, decltype(r)::value>),
+                                       dim3(unsigned(ng), nb), dim3(PERM_THREADS), 0, stream, n,
+                                       nrhs, B, ldb, ipiv, strideP, int(inverse), skip,
+                                       unsigned(g0), b0);
+                    RSA_LAUNCH_CHECK();
+                    return rocblas_status_success;
+                });
         };
-        if(n <= PERM_THREADS)
-            go(std::integral_constant<int, 1>{});
-        else if(n <= 2 * PERM_THREADS)
-            go(std::integral_constant<int, 2>{});
-        else if(n <= 4 * PERM_THREADS)
-            go(std::integral_constant<int, 4>{});
-        else
-            go(std::integral_constant<int, 8>{});
-        RSA_LAUNCH_CHECK();
+        const rocblas_status st = n <= PERM_THREADS       ? go(std::integral_constant<int, 1>{})
+                                  : n <= 2 * PERM_THREADS ? go(std::integral_constant<int, 2>{})
+                                  : n <= 4 * PERM_THREADS ? go(std::integral_constant<int, 4>{})
+                                                          : go(std::integral_constant<int, 8>{});
+        if(st != rocblas_status_success)
+            return st;
     }
     return rocblas_status_success;
 }
@@ -816,7 +813,7 @@ __global__ __launch_bounds__(STEP_THREADS) void trsm_step_kernel(int n, int nrhs
                                                                  int lda, Batch<T> BB, int ldb,
                                                                  const int* __restrict__ skip,
                                                                  int prev, int next, int tile0,
-                                                                 int64_t boff)
+                                                                 unsigned group0, int64_t boff)
 {
     using M = mfma16<T>;
     constexpr bool LOWER = KIND == 0 || KIND == 2;
@@ -841,7 +838,7 @@ __global__ __launch_bounds__(STEP_THREADS) void trsm_step_kernel(int n, int nrhs
     const int lane = tid % 64;
     const int tile = tile0 + blockIdx.y;
     const int r0 = tile * ST;
-    const int c0 = blockIdx.x * COLS + 16 * (wid % CG); // this wavefront's columns
+    const int c0 = int(group0 + blockIdx.x) * COLS + 16 * (wid % CG); // this wavefront's columns
     const int wr = 16 * RT * (wid / CG); // and rows of the tile, in the update
     const bool solve = tile == next; // uniform
     auto op = [&](int i, int k) -> T {
@@ -991,14 +988,23 @@ static rocblas_status trsm_blocked(hipStream_t stream, int n, int nrhs, Batch<T>
             const int cnt = s == 0 ? 1 : tiles - s; // tiles not solved yet
             const int tile0 = LOWER || s == 0 ? next : 0;
             // right-hand sides in x: more than 65535 groups of them are allowed
-            const dim3 grid(ceil_div(nrhs, cols), cnt, nb);
-            if(cols == 16)
-                hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 16>), grid, dim3(STEP_THREADS), 0,
-                                   stream, n, nrhs, A, lda, B, ldb, skip, prev, next, tile0, b0);
-            else
-                hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 32>), grid, dim3(STEP_THREADS), 0,
-                                   stream, n, nrhs, A, lda, B, ldb, skip, prev, next, tile0, b0);
-            RSA_LAUNCH_CHECK();
+            const rocblas_status st = launch_split(
+                1, ceil_div(nrhs, cols), STEP_THREADS, 1,
+                [&](int64_t, int64_t, int64_t g0, int64_t ng) {
+                    const dim3 grid(unsigned(ng), cnt, nb);
+                    if(cols == 16)
+                        hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 16>), grid,
+                                           dim3(STEP_THREADS), 0, stream, n, nrhs, A, lda, B, ldb,
+                                           skip, prev, next, tile0, unsigned(g0), b0);
+                    else
+                        hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 32>), grid,
+                                           dim3(STEP_THREADS), 0, stream, n, nrhs, A, lda, B, ldb,
+                                           skip, prev, next, tile0, unsigned(g0), b0);
+                    RSA_LAUNCH_CHECK();
+                    return rocblas_status_success;
+                });
+            if(st != rocblas_status_success)
+                return st;
         }
     }
     return rocblas_status_success;

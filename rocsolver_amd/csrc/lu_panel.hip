@@ -450,34 +450,42 @@ rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ip
         constexpr int W = decltype(w)::value;
         constexpr int R = decltype(r)::value;
         constexpr int NT = decltype(nt)::value;
-        if(pivot)
-            hipLaunchKernelGGL((panel_reg_kernel<T, W, R, NT, true>), dim3(bc), dim3(NT), 0, stream,
-                               m, A, lda, ipiv, strideP, info, j0, jb, o0, oend, uend);
-        else
-            hipLaunchKernelGGL((panel_reg_kernel<T, W, R, NT, false>), dim3(bc), dim3(NT), 0,
-                               stream, m, A, lda, ipiv, strideP, info, j0, jb, o0, oend, uend);
+        return launch_split(bc, 1, NT, 1, [&](int64_t b0, int64_t cnt, int64_t, int64_t) {
+            const dim3 grid{unsigned(cnt)};
+            int* piv = pivot ? ipiv + b0 * strideP : nullptr;
+            if(pivot)
+                hipLaunchKernelGGL((panel_reg_kernel<T, W, R, NT, true>), grid, dim3(NT), 0, stream,
+                                   m, batch_from(A, b0), lda, piv, strideP, info + b0, j0, jb, o0,
+                                   oend, uend);
+            else
+                hipLaunchKernelGGL((panel_reg_kernel<T, W, R, NT, false>), grid, dim3(NT), 0,
+                                   stream, m, batch_from(A, b0), lda, piv, strideP, info + b0, j0,
+                                   jb, o0, oend, uend);
+            RSA_LAUNCH_CHECK();
+            return rocblas_status_success;
+        });
     };
     using std::integral_constant;
     constexpr int S = sizeof(T) == 8 ? 1 : 2;
     const int rows = m - j0;
+    using i256 = integral_constant<int, 256>;
+    using i512 = integral_constant<int, 512>;
     if(rows <= 256)
-        go(integral_constant<int, 32>{}, integral_constant<int, 1>{}, integral_constant<int, 256>{});
-    else if(rows <= 512)
-        go(integral_constant<int, 32>{}, integral_constant<int, 1>{}, integral_constant<int, 512>{});
-    else if(rows <= 1024)
-        go(integral_constant<int, 32>{}, integral_constant<int, 2>{}, integral_constant<int, 512>{});
-    else if(rows <= 1536)
-        go(integral_constant<int, 32>{}, integral_constant<int, 3>{}, integral_constant<int, 512>{});
-    else if(rows <= 2048)
-        go(integral_constant<int, 16 * S>{}, integral_constant<int, 4>{},
-           integral_constant<int, 512>{});
-    else if(rows <= 4096)
-        go(integral_constant<int, 8 * S>{}, integral_constant<int, 8>{},
-           integral_constant<int, 512>{});
-    else if constexpr(sizeof(T) == 4)
-        go(integral_constant<int, 8>{}, integral_constant<int, 16>{}, integral_constant<int, 512>{});
-    RSA_LAUNCH_CHECK();
-    return rocblas_status_success;
+        return go(integral_constant<int, 32>{}, integral_constant<int, 1>{}, i256{});
+    if(rows <= 512)
+        return go(integral_constant<int, 32>{}, integral_constant<int, 1>{}, i512{});
+    if(rows <= 1024)
+        return go(integral_constant<int, 32>{}, integral_constant<int, 2>{}, i512{});
+    if(rows <= 1536)
+        return go(integral_constant<int, 32>{}, integral_constant<int, 3>{}, i512{});
+    if(rows <= 2048)
+        return go(integral_constant<int, 16 * S>{}, integral_constant<int, 4>{}, i512{});
+    if(rows <= 4096)
+        return go(integral_constant<int, 8 * S>{}, integral_constant<int, 8>{}, i512{});
+    if constexpr(sizeof(T) == 4)
+        return go(integral_constant<int, 8>{}, integral_constant<int, 16>{}, i512{});
+    else
+        return rocblas_status_internal_error; // taller than panel_reg_width allows
 }
 
 #define RSA_PANEL_INST(T)                                                                       \
