@@ -330,9 +330,10 @@ __global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void potrs_fused_k
 template <typename T>
 __global__ __launch_bounds__(64) void potrs_serial_kernel(int n, int nrhs, Batch<T> AA, int lda,
                                                           int up, Batch<T> BB, int ldb, int bc,
+                                                          int64_t block0,
                                                           const int* __restrict__ skip)
 {
-    const int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t g = (block0 + blockIdx.x) * blockDim.x + threadIdx.x;
     if(g >= int64_t(bc) * nrhs)
         return;
     const int64_t b = g / nrhs;
@@ -425,11 +426,13 @@ rocblas_status potrs(hipStream_t stream, bool up, int n, int nrhs, Batch<T> A, i
             return go(integral_constant<int, 256>{}, integral_constant<int, 256 * F>{});
         return go(integral_constant<int, 512>{}, integral_constant<int, 512>{});
     }
-    const int64_t threads = int64_t(bc) * nrhs;
-    hipLaunchKernelGGL((potrs_serial_kernel<T>), dim3(unsigned((threads + 63) / 64)), dim3(64), 0,
-                       stream, n, nrhs, A, lda, int(up), B, ldb, bc, skip);
-    RSA_LAUNCH_CHECK();
-    return rocblas_status_success;
+    return launch_split(
+        (int64_t(bc) * nrhs + 63) / 64, 1, 64, 1, [&](int64_t w0, int64_t nw, int64_t, int64_t) {
+            hipLaunchKernelGGL((potrs_serial_kernel<T>), dim3(unsigned(nw)), dim3(64), 0, stream, n,
+                               nrhs, A, lda, int(up), B, ldb, bc, w0, skip);
+            RSA_LAUNCH_CHECK();
+            return rocblas_status_success;
+        });
 }
 
 #define RSA_CHOL_INST(T)                                                                      \

@@ -160,9 +160,15 @@ rocblas_status getri_solve(hipStream_t stream, int n, Batch<T> LU, int ldlu, con
 {
     if(n <= 0 || bc <= 0)
         return rocblas_status_success;
-    hipLaunchKernelGGL((diag_zero_kernel<T>), dim3((bc + 3) / 4), dim3(256), 0, stream, n, LU,
-                       ldlu, info, bc);
-    RSA_LAUNCH_CHECK();
+    const rocblas_status st
+        = launch_split(bc, 1, 64, 4, [&](int64_t b0, int64_t nb, int64_t, int64_t) {
+              hipLaunchKernelGGL((diag_zero_kernel<T>), dim3(ceil_div(nb, 4)), dim3(256), 0, stream,
+                                 n, batch_from(LU, b0), ldlu, info + b0, int(nb));
+              RSA_LAUNCH_CHECK();
+              return rocblas_status_success;
+          });
+    if(st != rocblas_status_success)
+        return st;
     if(inverse_by_tiles(n, bc) && n <= FUSED_MAX && fits_buffer<T>(ldlu, n) && fits_buffer<T>(ldx, n))
         return inverse_tiles<T>(stream, n, LU, ldlu, pivot ? ipiv : nullptr, strideP, X, ldx, bc);
     hipLaunchKernelGGL((set_identity_kernel<T>), square_grid(n, bc), dim3(256), 0, stream, n, X,

@@ -592,37 +592,54 @@ void nrhs_switch(int nrhs, F&& f)
         f(ic<8>{});
 }
 
+// launch(grid, b0, nb) for the systems of a batch, TPW to a wavefront
+template <int TPW, typename F>
+rocblas_status team_launch(int bc, F&& launch)
+{
+    return launch_split(
+        ceil_div(bc, TPW), 1, 64, 1, [&](int64_t w0, int64_t nw, int64_t, int64_t) {
+            const int64_t b0 = w0 * TPW;
+            launch(dim3(unsigned(nw)), b0, int(bc - b0 < nw * TPW ? bc - b0 : nw * TPW));
+            RSA_LAUNCH_CHECK();
+            return rocblas_status_success;
+        });
+}
+
 template <typename T>
 rocblas_status getrf_small_launch(hipStream_t stream, int m, int n, Batch<T> A, int lda,
                                   int* ipiv, int64_t strideP, int* info, int bc, bool pivot)
 {
+    rocblas_status st = rocblas_status_success;
     team_size_switch(m, [&](auto ts) {
         ncols_switch(n, [&](auto nc) {
             constexpr int TS = decltype(ts)::value;
             constexpr int NC = decltype(nc)::value;
-            dim3 grid(ceil_div(bc, 64 / TS));
             // one buffer per wavefront when its matrices span < 2 GiB
             const bool buf = A.ptrs == nullptr && A.stride >= 0
                              && (uint64_t(64 / TS - 1) * uint64_t(A.stride)
                                  + uint64_t(lda) * uint64_t(n))
                                         * sizeof(T)
                                     < (uint64_t(1) << 31);
-            if(pivot && buf)
-                hipLaunchKernelGGL((getrf_small_kernel<T, NC, TS, true, true>), grid, dim3(64), 0,
-                                   stream, m, n, A, lda, ipiv, strideP, info, bc);
-            else if(pivot)
-                hipLaunchKernelGGL((getrf_small_kernel<T, NC, TS, true, false>), grid, dim3(64),
-                                   0, stream, m, n, A, lda, ipiv, strideP, info, bc);
-            else if(buf)
-                hipLaunchKernelGGL((getrf_small_kernel<T, NC, TS, false, true>), grid, dim3(64),
-                                   0, stream, m, n, A, lda, ipiv, strideP, info, bc);
-            else
-                hipLaunchKernelGGL((getrf_small_kernel<T, NC, TS, false, false>), grid, dim3(64),
-                                   0, stream, m, n, A, lda, ipiv, strideP, info, bc);
+            st = team_launch<64 / TS>(bc, [&](dim3 grid, int64_t b0, int nb) {
+                const Batch<T> Ab = batch_from(A, b0);
+                int* piv = pivot ? ipiv + b0 * strideP : nullptr;
+                if(pivot && buf)
+                    hipLaunchKernelGGL((getrf_small_kernel<T, NC, TS, true, true>), grid, dim3(64),
+                                       0, stream, m, n, Ab, lda, piv, strideP, info + b0, nb);
+                else if(pivot)
+                    hipLaunchKernelGGL((getrf_small_kernel<T, NC, TS, true, false>), grid, dim3(64),
+                                       0, stream, m, n, Ab, lda, piv, strideP, info + b0, nb);
+                else if(buf)
+                    hipLaunchKernelGGL((getrf_small_kernel<T, NC, TS, false, true>), grid, dim3(64),
+                                       0, stream, m, n, Ab, lda, piv, strideP, info + b0, nb);
+                else
+                    hipLaunchKernelGGL((getrf_small_kernel<T, NC, TS, false, false>), grid,
+                                       dim3(64), 0, stream, m, n, Ab, lda, piv, strideP, info + b0,
+                                       nb);
+            });
         });
     });
-    RSA_LAUNCH_CHECK();
-    return rocblas_status_success;
+    return st;
 }
 
 template <typename T>
@@ -630,18 +647,20 @@ rocblas_status gesv_small_launch(hipStream_t stream, int n, int nrhs, Batch<T> A
                                  int* ipiv, int64_t strideP, Batch<T> B, int ldb, int* info,
                                  int bc)
 {
+    rocblas_status st = rocblas_status_success;
     square_switch(n, [&](auto ts, auto nc) {
         nrhs_switch(nrhs, [&](auto nr) {
             constexpr int TS = decltype(ts)::value;
             constexpr int NC = decltype(nc)::value;
             constexpr int NR = decltype(nr)::value;
-            dim3 grid(ceil_div(bc, 64 / TS));
-            hipLaunchKernelGGL((gesv_small_kernel<T, NC, TS, NR>), grid, dim3(64), 0, stream, n,
-                               nrhs, A, lda, ipiv, strideP, B, ldb, info, bc);
+            st = team_launch<64 / TS>(bc, [&](dim3 grid, int64_t b0, int nb) {
+                hipLaunchKernelGGL((gesv_small_kernel<T, NC, TS, NR>), grid, dim3(64), 0, stream, n,
+                                   nrhs, batch_from(A, b0), lda, ipiv + b0 * strideP, strideP,
+                                   batch_from(B, b0), ldb, info + b0, nb);
+            });
         });
     });
-    RSA_LAUNCH_CHECK();
-    return rocblas_status_success;
+    return st;
 }
 
 template <typename T>
@@ -649,18 +668,21 @@ rocblas_status getrs_small_launch(hipStream_t stream, bool trans, int n, int nrh
                                   int lda, const int* ipiv, int64_t strideP, Batch<T> B, int ldb,
                                   int bc, bool pivot)
 {
+    rocblas_status st = rocblas_status_success;
     square_switch(n, [&](auto ts, auto nc) {
         nrhs_switch(nrhs, [&](auto nr) {
             constexpr int TS = decltype(ts)::value;
             constexpr int NC = decltype(nc)::value;
             constexpr int NR = decltype(nr)::value;
-            dim3 grid(ceil_div(bc, 64 / TS));
-            hipLaunchKernelGGL((getrs_small_kernel<T, NC, TS, NR>), grid, dim3(64), 0, stream,
-                               trans, n, nrhs, A, lda, ipiv, strideP, B, ldb, bc, pivot);
+            st = team_launch<64 / TS>(bc, [&](dim3 grid, int64_t b0, int nb) {
+                hipLaunchKernelGGL((getrs_small_kernel<T, NC, TS, NR>), grid, dim3(64), 0, stream,
+                                   trans, n, nrhs, batch_from(A, b0), lda,
+                                   pivot ? ipiv + b0 * strideP : nullptr, strideP,
+                                   batch_from(B, b0), ldb, nb, pivot);
+            });
         });
     });
-    RSA_LAUNCH_CHECK();
-    return rocblas_status_success;
+    return st;
 }
 
 } // namespace rsa

@@ -103,3 +103,36 @@ def test_getrs_shared_factor(room, handle):
     ra.check("rocsolver_sgetrs_strided_batched", handle.value, ra.OP_NONE, n, 1, LU.data_ptr(), n,
              0, ipiv.data_ptr(), 0, B.data_ptr(), n, n, bc)
     assert bool((B[-1] == 2.5).all()) and bool((B[:-1] == 1.5).all())
+
+
+def test_small_systems(room, handle):
+    """Four systems per wavefront: factor, solve, and factor and solve."""
+    import rocsolver_amd as ra
+    torch = room(16)
+    bc = (1 << 28) + 5
+    A = torch.full((bc, 1, 1), 4.0, dtype=torch.float32, device="cuda")
+    A[-1] = 0.0
+    ipiv, info = ra.getrf(handle, A)
+    assert int(info[:-1].abs().max()) == 0 and int(info[-1]) == 1
+    assert bool((ipiv == 1).all())
+    A[-1] = 8.0
+    B = torch.full((bc, 1, 1), 2.0, dtype=torch.float32, device="cuda")
+    ra.getrs(handle, A, ipiv, B)
+    assert bool((B[:-1] == 0.5).all()) and float(B[-1]) == 0.25
+    ipiv.zero_()
+    ipiv, info = ra.gesv(handle, A, B)
+    assert int(info.abs().max()) == 0 and bool((ipiv == 1).all())
+    assert bool((B[:-1] == 0.125).all()) and float(B[-1]) == 0.03125
+
+
+def test_getri_many(room, handle):
+    """A wavefront per matrix looks for zeros on the diagonal."""
+    import rocsolver_amd as ra
+    torch = room(4)
+    bc = (1 << 26) + 3
+    A = torch.full((bc, 1, 1), 4.0, dtype=torch.float32, device="cuda")
+    A[-1] = 0.0
+    ipiv = torch.ones((bc, 1), dtype=torch.int32, device="cuda")
+    info = ra.getri(handle, A, ipiv)
+    assert int(info[:-1].abs().max()) == 0 and int(info[-1]) == 1
+    assert bool((A[:-1] == 0.25).all())
