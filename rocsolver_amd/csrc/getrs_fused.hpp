@@ -8,11 +8,11 @@
 // Two kernels with the same operations per row, so bit-identical results:
 //   * the tile solver of tile_solve.hpp, 16 right-hand sides per workgroup;
 //   * beyond n = 64, the row solver of trsv_rows.hpp, thread i owning row i of
-//     up to four right-hand sides, for large batches with few of them: there
-//     the read of the factors bounds the call, and its smaller workgroups
-//     keep twice the systems in flight.
+//     up to eight right-hand sides, for large batches with few of them
+//     (rows_rule.hpp).
 #pragma once
 
+#include "rows_rule.hpp"
 #include "tile_solve.hpp"
 #include "trsv_rows.hpp"
 
@@ -84,24 +84,6 @@ __global__ __launch_bounds__(NMAX) void getrs_rows_kernel(int n, int nrhs, Batch
     }
 }
 
-// Which kernel: rows for at most four right-hand sides of 1024 systems or
-// more (four per CU; two beyond n = 256), where it was the faster one:
-//   op N, FP64: n = 96 x 2048, 4 right-hand sides 69 against 75 us; n = 128 x
-//   16384 676 against 800; n = 256 x 4096 598 against 662; n = 300 x 1024
-//   329 against 376; n = 512 x 512 316 against 328 (with fewer systems tiles:
-//   n = 96 x 512 31 against 40 us, n = 128 x 64 33 against 44);
-//   op N, FP32, n <= 256: n = 128 x 16384 401 against 418 us; beyond, tiles
-//   (n = 512 x 512 216 against 175);
-//   op T: FP64, n <= 96: n = 72 x 2048 69 against 85 us; beyond, tiles (n =
-//   128 x 16384 952 against 858, its loads being uncoalesced by rows).
-template <typename T>
-inline bool getrs_by_rows(bool trans, int n, int nrhs, int bc)
-{
-    if(nrhs > 4 || bc < (n > 256 ? 512 : 1024))
-        return false;
-    return trans ? sizeof(T) == 8 && n <= 96 : sizeof(T) == 8 || n <= 256;
-}
-
 template <typename T>
 rocblas_status getrs_fused_launch(hipStream_t stream, bool trans, int n, int nrhs, Batch<T> A,
                                   int lda, const int* ipiv, int64_t strideP, Batch<T> B, int ldb,
@@ -129,14 +111,17 @@ rocblas_status getrs_fused_launch(hipStream_t stream, bool trans, int n, int nrh
             return nrhs == 1 ? go(nmax, integral_constant<int, 1>{}, tr)
                              : go(nmax, integral_constant<int, 4>{}, tr);
         };
-        if(trans)
-            return by_nrhs(integral_constant<int, 128>{}, std::true_type{});
+        // the orders and right-hand sides that getrs_by_rows can give
         if(n <= 128)
-            return by_nrhs(integral_constant<int, 128>{}, std::false_type{});
+            return trans ? by_nrhs(integral_constant<int, 128>{}, std::true_type{})
+                         : by_nrhs(integral_constant<int, 128>{}, std::false_type{});
         if(n <= 256)
-            return by_nrhs(integral_constant<int, 256>{}, std::false_type{});
-        if constexpr(sizeof(T) == 8)
-            return by_nrhs(integral_constant<int, 512>{}, std::false_type{});
+            return trans ? by_nrhs(integral_constant<int, 256>{}, std::true_type{})
+                         : by_nrhs(integral_constant<int, 256>{}, std::false_type{});
+        if(nrhs > 4)
+            return go(integral_constant<int, 512>{}, integral_constant<int, 8>{},
+                      std::false_type{});
+        return by_nrhs(integral_constant<int, 512>{}, std::false_type{});
     }
     auto go = [&](auto nmax, auto nt) {
         constexpr int NMAX = decltype(nmax)::value;

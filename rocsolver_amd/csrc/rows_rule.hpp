@@ -1,0 +1,89 @@
+// rows_rule.hpp -- which kernel solves with a factor of order <= 512: the row
+// solver (trsv_rows.hpp) or the tile solver (tile_solve.hpp).  Same operations
+// per row, same bits.  Host code, no HIP.
+//
+// The tile solver works on 16 right-hand sides and whole 32-row blocks whatever
+// the call has; the row solver on what is there, in smaller workgroups that
+// keep more systems in flight, but slower for one system.  So rows win in large
+// batches of few right-hand sides, the earlier the less of the last 32-row
+// block the order fills.
+//
+// The lines come from timing both at about 110 orders and 25 batches per type
+// and op.  Over those the chosen kernel is within 1.15 of the faster one beyond
+// launch noise, and mostly the faster one; the wrong one costs up to 1.8 times.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+namespace rsa
+{
+
+// One line of a table: for orders up to `order`, beyond how many systems per
+// CU rows are taken with 1, 2..4 and 5..8 right-hand sides.
+struct RowsFrom
+{
+    int order;
+    int one, few, more;
+};
+constexpr int NEVER = 1 << 23; // times ROWS_CUS: more than a batch holds
+constexpr int ROWS_CUS = 256;
+
+template <size_t K>
+inline bool rows_win(const RowsFrom (&table)[K], int n, int nrhs, int bc)
+{
+    for(const RowsFrom& l : table)
+        if(n <= l.order)
+        {
+            const int per_cu = nrhs <= 1 ? l.one : nrhs <= 4 ? l.few : nrhs <= 8 ? l.more : NEVER;
+            return bc > int64_t(ROWS_CUS) * per_cu;
+        }
+    return false;
+}
+
+// getrs, 64 < n <= 512.  On both sides of the lines, rows against tiles
+// in us (order x systems, right-hand sides):
+//   op N, FP64: 65 x 2048, 1: 42 against 77; 128 x 8192, 4: 340 against 416;
+//     256 x 1024, 4: 165 against 177; 304 x 2904, 8: 1012 against 1109; but
+//     96 x 512, 4: 44 against 34
+//   op N, FP32: 65 x 512, 1: 28 against 34; 128 x 8192, 4: 203 against 222;
+//     304 x 640, 4: 129 against 163; but 304 x 1024, 4: 229 against 198
+//   op T, FP64: 97 x 8192, 4: 360 against 403; 129 x 1024, 1: 83 against 108;
+//     but 128 x 8192, 4: 498 against 439
+//   op T, FP32: 65 x 8192, 1: 125 against 198; 83 x 8192, 4: 173 against 202;
+//     but 96 x 8192, 4: 256 against 211
+// In op T a row's entries are a column of A, which a thread reads alone: there
+// rows win only where the last 32-row block holds few rows.
+template <typename T>
+inline bool getrs_by_rows(bool trans, int n, int nrhs, int bc)
+{
+    static constexpr RowsFrom N64[]
+        = {{128, 2, 4, NEVER}, {256, 2, 2, NEVER}, {512, 1, 1, 3}};
+    static constexpr RowsFrom T64[] = {{76, 2, 4, NEVER},
+                                       {104, 4, 4, NEVER},
+                                       {128, NEVER, NEVER, NEVER},
+                                       {152, 2, 2, NEVER}};
+    static constexpr RowsFrom N32[] = {{84, 0, 1, NEVER},
+                                       {96, 1, 6, NEVER},
+                                       {108, 1, 1, NEVER},
+                                       {128, 1, 8, NEVER},
+                                       {256, 2, 4, NEVER},
+                                       {512, 2, 2, 8}};
+    static constexpr RowsFrom T32[] = {{70, 0, 1, NEVER},
+                                       {84, 1, 8, NEVER},
+                                       {96, NEVER, NEVER, NEVER},
+                                       {102, 1, 8, NEVER},
+                                       {128, NEVER, NEVER, NEVER},
+                                       {136, 4, 4, NEVER}};
+    if(sizeof(T) == 8)
+        return trans ? rows_win(T64, n, nrhs, bc) : rows_win(N64, n, nrhs, bc);
+    // FP32 beyond n = 256: a CU holds two workgroups of tiles and three of
+    // rows, so rows win between two and three systems per CU for any number of
+    // right-hand sides up to 8, and tiles again up to four, where both take
+    // two rounds
+    if(!trans && n > 256 && nrhs <= 8 && bc > 2 * ROWS_CUS && bc <= 4 * ROWS_CUS)
+        return bc <= 3 * ROWS_CUS;
+    return trans ? rows_win(T32, n, nrhs, bc) : rows_win(N32, n, nrhs, bc);
+}
+
+} // namespace rsa
