@@ -43,9 +43,9 @@ inline bool rows_win(const RowsFrom (&table)[K], int n, int nrhs, int bc)
 
 // getrs, 64 < n <= 512.  On both sides of the lines, rows against tiles
 // in us (order x systems, right-hand sides):
-//   op N, FP64: 65 x 2048, 1: 42 against 77; 128 x 8192, 4: 340 against 416;
-//     256 x 1024, 4: 165 against 177; 304 x 2904, 8: 1012 against 1109; but
-//     96 x 512, 4: 44 against 34
+//   op N, FP64: 65 x 512, 1: 31 against 34; 65 x 2048, 1: 42 against 77; 128 x
+//     8192, 4: 340 against 416; 256 x 1024, 4: 165 against 177; 304 x 2904, 8:
+//     1012 against 1109; but 96 x 512, 4: 44 against 34
 //   op N, FP32: 65 x 512, 1: 28 against 34; 128 x 8192, 4: 203 against 222;
 //     304 x 640, 4: 129 against 163; but 304 x 1024, 4: 229 against 198
 //   op T, FP64: 97 x 8192, 4: 360 against 403; 129 x 1024, 1: 83 against 108;
@@ -57,8 +57,10 @@ inline bool rows_win(const RowsFrom (&table)[K], int n, int nrhs, int bc)
 template <typename T>
 inline bool getrs_by_rows(bool trans, int n, int nrhs, int bc)
 {
-    static constexpr RowsFrom N64[]
-        = {{128, 2, 4, NEVER}, {256, 2, 2, NEVER}, {512, 1, 1, 3}};
+    static constexpr RowsFrom N64[] = {{72, 1, 3, NEVER},
+                                       {128, 2, 4, NEVER},
+                                       {256, 2, 2, NEVER},
+                                       {512, 1, 1, 3}};
     static constexpr RowsFrom T64[] = {{76, 2, 4, NEVER},
                                        {104, 4, 4, NEVER},
                                        {128, NEVER, NEVER, NEVER},

@@ -31,6 +31,7 @@ int main()
 
 # type, op, order, systems, right-hand sides, the faster kernel
 MEASURED = [
+    ("d", "N", 65, 512, 1, "rows"), ("d", "N", 96, 512, 1, "tiles"),
     ("d", "N", 65, 2048, 1, "rows"), ("d", "N", 128, 8192, 4, "rows"),
     ("d", "N", 256, 1024, 4, "rows"), ("d", "N", 304, 2904, 8, "rows"),
     ("d", "N", 96, 512, 4, "tiles"), ("d", "N", 512, 64, 1, "tiles"),
