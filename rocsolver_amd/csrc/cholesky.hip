@@ -25,12 +25,16 @@
 // reference's own dot/gemv reductions differ from it by rounding only.
 //
 // Solve: for n <= 512 one workgroup per system with the tile solver of the LU
-// path (tile_solve.hpp) on non-unit triangles: L then L^T, or U^T then U
-// (library/src/lapack/roclapack_potrs.hpp:121-148); larger orders use one
-// thread per (system, right-hand side) substitution.
+// path (tile_solve.hpp) or, for large batches of few right-hand sides, its row
+// solver (trsv_rows.hpp, rows_rule.hpp), on non-unit triangles: L then L^T, or U^T then U
+// (library/src/lapack/roclapack_potrs.hpp:121-148), with the same operations
+// per row; larger orders use one thread per (system, right-hand side)
+// substitution.
 #include "mfma.hpp"
 #include "quad_solve.hpp"
+#include "rows_rule.hpp"
 #include "tile_solve.hpp"
+#include "trsv_rows.hpp"
 
 #include <cmath>
 
@@ -325,6 +329,38 @@ __global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void potrs_fused_k
         n, c0, cend, AA[b], lda, nullptr, BB[b], ldb, BB[b], ldb);
 }
 
+// The same by rows (blockDim.x == NMAX, n <= NMAX, nrhs <= NR).
+template <typename T, int NMAX, int NR, bool UP>
+__global__ __launch_bounds__(NMAX) void potrs_rows_kernel(int n, int nrhs, Batch<T> AA, int lda,
+                                                          Batch<T> BB, int ldb,
+                                                          const int* __restrict__ skip)
+{
+    __shared__ T sx[2][GBS][NR];
+    __shared__ T sL[GBS][GBS + 1];
+    const int64_t b = blockIdx.x;
+    if(skip && skip[b] != 0)
+        return;
+    const int tid = threadIdx.x;
+    const MatrixBuffer<T> A(AA[b], lda, n);
+    T* Bm = BB[b];
+    const MatrixBuffer<T> Bbuf(Bm, ldb, nrhs);
+    T x[NR];
+#pragma unroll
+    for(int q = 0; q < NR; ++q)
+        x[q] = Bbuf.load(tid < n && q < nrhs ? Bbuf.row_offset(tid) + Bbuf.col_offset(q)
+                                             : MatrixBuffer<T>::OUT_OF_RANGE,
+                         0);
+    solve_lower_rows<T, NR, UP, false, true>(n, A, x, sx, sL); // L or U^T
+    solve_upper_rows<T, NR, !UP, false, true>(n, A, x, sx, sL); // L^T or U
+    if(tid < n)
+    {
+#pragma unroll
+        for(int q = 0; q < NR; ++q)
+            if(q < nrhs)
+                Bm[tid + int64_t(q) * ldb] = x[q];
+    }
+}
+
 // Any order: one thread per (system, right-hand side), column-oriented
 // substitution in the same order of operations.
 template <typename T>
@@ -392,8 +428,44 @@ rocblas_status potrs(hipStream_t stream, bool up, int n, int nrhs, Batch<T> A, i
 {
     if(bc <= 0 || n <= 0 || nrhs <= 0)
         return rocblas_status_success;
+    using std::integral_constant;
     if(n <= FUSED_MAX && fits_buffer<T>(lda, n) && fits_buffer<T>(ldb, nrhs))
     {
+        if(potrs_by_rows<T>(n, nrhs, bc))
+        {
+            auto rows = [&](auto nmax, auto nr) {
+                constexpr int NMAX = decltype(nmax)::value;
+                constexpr int NR = decltype(nr)::value;
+                return launch_split(bc, 1, NMAX, 1, [&](int64_t b0, int64_t nb, int64_t, int64_t) {
+                    const dim3 grid{unsigned(nb)};
+                    const int* sk = skip ? skip + b0 : nullptr;
+                    if(up)
+                        hipLaunchKernelGGL((potrs_rows_kernel<T, NMAX, NR, true>), grid, dim3(NMAX),
+                                           0, stream, n, nrhs, batch_from(A, b0), lda,
+                                           batch_from(B, b0), ldb, sk);
+                    else
+                        hipLaunchKernelGGL((potrs_rows_kernel<T, NMAX, NR, false>), grid,
+                                           dim3(NMAX), 0, stream, n, nrhs, batch_from(A, b0), lda,
+                                           batch_from(B, b0), ldb, sk);
+                    RSA_LAUNCH_CHECK();
+                    return rocblas_status_success;
+                });
+            };
+            auto by_nrhs = [&](auto nmax) {
+                return nrhs == 1 ? rows(nmax, integral_constant<int, 1>{})
+                                 : rows(nmax, integral_constant<int, 4>{});
+            };
+            // the orders and right-hand sides that potrs_by_rows can give
+            if(n <= 64)
+                return nrhs <= 4 ? by_nrhs(integral_constant<int, 64>{})
+                                 : rows(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+            if(n <= 128)
+                return by_nrhs(integral_constant<int, 128>{});
+            if(n <= 256 || sizeof(T) == 4)
+                return by_nrhs(integral_constant<int, 256>{});
+            if constexpr(sizeof(T) == 8)
+                return by_nrhs(integral_constant<int, 512>{});
+        }
         auto go = [&](auto nmax, auto nt) {
             constexpr int NMAX = decltype(nmax)::value;
             constexpr int NT = decltype(nt)::value;
@@ -416,7 +488,6 @@ rocblas_status potrs(hipStream_t stream, bool up, int n, int nrhs, Batch<T> A, i
                     return rocblas_status_success;
                 });
         };
-        using std::integral_constant;
         constexpr int F = sizeof(T) == 8 ? 2 : 1; // as getrs_fused_launch
         if(n <= 64)
             return go(integral_constant<int, 64>{}, integral_constant<int, 64 * F>{});

@@ -10,7 +10,7 @@
 //
 // The lines come from timing both at about 110 orders and 25 batches per type
 // and op.  Over those the chosen kernel is within 1.15 of the faster one beyond
-// launch noise, and mostly the faster one; the wrong one costs up to 1.8 times.
+// launch noise, and mostly the faster one; the wrong one costs up to 3.5 times.
 #pragma once
 
 #include <cstddef>
@@ -86,6 +86,56 @@ inline bool getrs_by_rows(bool trans, int n, int nrhs, int bc)
     if(!trans && n > 256 && nrhs <= 8 && bc > 2 * ROWS_CUS && bc <= 4 * ROWS_CUS)
         return bc <= 3 * ROWS_CUS;
     return trans ? rows_win(T32, n, nrhs, bc) : rows_win(N32, n, nrhs, bc);
+}
+
+// potrs, n <= 512.  On both sides of the lines, rows against tiles in us,
+// lower storage (order x systems, right-hand sides):
+//   FP64: 1 x 65536, 1: 154 against 533; 8 x 4096, 4: 32 against 44; 32 x 2048,
+//     1: 22 against 28; 64 x 4096, 1: 64 against 86; 129 x 4096, 4: 351 against
+//     406; 257 x 1280, 4: 436 against 458; but 32 x 1024, 1: 19 against 16; 64 x
+//     4096, 4: 116 against 86; 512 x 1024, 4: 797 against 748
+//   FP32: 1 x 65536, 1: 100 against 307; 8 x 4096, 4: 19 against 31; 33 x 4096,
+//     4: 42 against 58; 65 x 3072, 4: 63 against 78; 129 x 3072, 1: 137 against
+//     173; but 64 x 1536, 4: 44 against 31; 96 x 1024, 1: 44 against 36; 128 x
+//     2048, 4: 94 against 71
+template <typename T>
+inline bool potrs_by_rows(int n, int nrhs, int bc)
+{
+    static constexpr RowsFrom R64[] = {{4, 0, 1, 6},
+                                       {8, 1, 4, 6},
+                                       {20, 1, 6, NEVER},
+                                       {24, 4, 16, NEVER},
+                                       {32, 6, NEVER, NEVER},
+                                       {47, 3, 6, NEVER},
+                                       {52, 4, 32, NEVER},
+                                       {64, 6, NEVER, NEVER},
+                                       {88, 2, 4, NEVER},
+                                       {96, 4, 16, NEVER},
+                                       {108, 2, 4, NEVER},
+                                       {128, 4, 12, NEVER},
+                                       {151, 2, 2, NEVER},
+                                       {224, 2, 12, NEVER},
+                                       {256, 12, NEVER, NEVER},
+                                       {288, 1, 3, NEVER},
+                                       {384, 1, 6, NEVER},
+                                       {512, 12, NEVER, NEVER}};
+    static constexpr RowsFrom R32[] = {{5, 0, 0, 4},
+                                       {8, 0, 0, 8},
+                                       {12, 0, 4, 12},
+                                       {20, 0, 8, NEVER},
+                                       {26, 4, 12, NEVER},
+                                       {32, 4, NEVER, NEVER},
+                                       {44, 0, 8, NEVER},
+                                       {52, 4, 12, NEVER},
+                                       {64, 12, NEVER, NEVER},
+                                       {68, 1, 4, NEVER},
+                                       {84, 4, 8, NEVER},
+                                       {96, 8, NEVER, NEVER},
+                                       {108, 6, 8, NEVER},
+                                       {128, 32, NEVER, NEVER},
+                                       {136, 4, 4, NEVER},
+                                       {256, 32, NEVER, NEVER}};
+    return sizeof(T) == 8 ? rows_win(R64, n, nrhs, bc) : rows_win(R32, n, nrhs, bc);
 }
 
 } // namespace rsa

@@ -1,4 +1,4 @@
-"""The row and the tile solver behind getrs agree bit for bit.
+"""The row and the tile solver behind potrs and getrs agree bit for bit.
 
 Large batches of few right-hand sides take one workgroup of rows per system,
 small ones the tile solver, by tables over the order (with lines at 32-row
@@ -33,6 +33,28 @@ def _both(torch, call, F, B, rep):
     return one.cpu().numpy()
 
 
+@pytest.mark.parametrize("n", [1, 4, 5, 8, 9, 12, 20, 26, 32, 33, 44, 47, 52, 53, 64, 65, 84, 96, 97,
+                               108, 127, 128, 129, 151, 224, 256, 257, 288, 384, 385, 512])
+@pytest.mark.parametrize("uplo", ["L", "U"])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_potrs(torch_gpu, handle, n, uplo, dtype):
+    torch = torch_gpu
+    g = np.random.default_rng(n)
+    F = _factor(g, n, n + 3, dtype)
+    Fd = torch.from_numpy(F).cuda()
+    for nrhs in (1, 3, 4, 8):
+        print(f"potrs n={n} {uplo} nrhs={nrhs} {dtype.__name__}", flush=True)
+        B = g.uniform(-1, 1, size=(FEW, nrhs, n + 2)).astype(dtype)
+        for rep in (420, 1400) if n <= 256 else (420,):
+            X = _both(torch, lambda f, b: ra.potrs(handle, f, b, uplo=uplo), Fd,
+                      torch.from_numpy(B).cuda(), rep)
+        Xo = B.copy()
+        oracle.potrs(F, n, Xo, uplo)
+        np.testing.assert_array_equal(X[:, :, n:], Xo[:, :, n:])
+        err = np.abs(X - Xo).max() / np.abs(Xo).max()
+        assert err <= n * np.finfo(dtype).eps
+
+
 @pytest.mark.parametrize("n", [65, 76, 84, 96, 97, 104, 108, 128, 129, 136, 152, 200, 256, 257, 384, 512])
 @pytest.mark.parametrize("trans", ["N", "T"])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
@@ -57,3 +79,18 @@ def test_getrs(torch_gpu, handle, n, trans, dtype):
         np.testing.assert_array_equal(X[:, :, n:], Xo[:, :, n:])
         err = np.abs(X - Xo).max() / np.abs(Xo).max()
         assert err <= n * np.finfo(dtype).eps
+
+
+@pytest.mark.parametrize("uplo", ["L", "U"])
+def test_posv_leaves_failed_systems_alone(torch_gpu, handle, uplo):
+    """B of a system whose factorisation failed is not touched by the rows."""
+    torch = torch_gpu
+    bc, n = 1030, 33
+    A = (torch.eye(n, dtype=torch.float64, device="cuda") * 4).repeat(bc, 1, 1)
+    A[500, 20, 20] = -1.0
+    B = torch.ones((bc, 1, n), dtype=torch.float64, device="cuda")
+    info = ra.potrs(handle, A, B, uplo=uplo, posv=True)
+    assert int(info[500]) == 21 and int(info.sum()) == 21
+    want = torch.full_like(B, 0.25)
+    want[500] = 1.0
+    assert torch.equal(B, want)

@@ -22,15 +22,21 @@ int main()
     int n, bc, nrhs;
     while(scanf(" %c %c %d %d %d", &type, &op, &n, &bc, &nrhs) == 5)
     {
-        const bool rows = type == 'd' ? rsa::getrs_by_rows<double>(op == 'T', n, nrhs, bc)
-                                      : rsa::getrs_by_rows<float>(op == 'T', n, nrhs, bc);
+        bool rows;
+        if(op == 'C')
+            rows = type == 'd' ? rsa::potrs_by_rows<double>(n, nrhs, bc)
+                               : rsa::potrs_by_rows<float>(n, nrhs, bc);
+        else
+            rows = type == 'd' ? rsa::getrs_by_rows<double>(op == 'T', n, nrhs, bc)
+                               : rsa::getrs_by_rows<float>(op == 'T', n, nrhs, bc);
         puts(rows ? "rows" : "tiles");
     }
 }
 """
 
-# type, op, order, systems, right-hand sides, the faster kernel
+# type, op (N, T: getrs; C: potrs), order, systems, right-hand sides, the faster kernel
 MEASURED = [
+    # getrs
     ("d", "N", 65, 512, 1, "rows"), ("d", "N", 96, 512, 1, "tiles"),
     ("d", "N", 65, 2048, 1, "rows"), ("d", "N", 128, 8192, 4, "rows"),
     ("d", "N", 256, 1024, 4, "rows"), ("d", "N", 304, 2904, 8, "rows"),
@@ -43,6 +49,16 @@ MEASURED = [
     ("s", "N", 304, 1280, 4, "rows"), ("s", "N", 512, 512, 1, "tiles"),
     ("s", "T", 65, 8192, 1, "rows"), ("s", "T", 83, 8192, 4, "rows"),
     ("s", "T", 96, 8192, 4, "tiles"), ("s", "T", 512, 1024, 1, "tiles"),
+    # potrs
+    ("d", "C", 1, 65536, 1, "rows"), ("d", "C", 8, 4096, 4, "rows"),
+    ("d", "C", 32, 2048, 1, "rows"), ("d", "C", 64, 4096, 1, "rows"),
+    ("d", "C", 129, 4096, 4, "rows"), ("d", "C", 257, 1280, 4, "rows"),
+    ("d", "C", 32, 1024, 1, "tiles"), ("d", "C", 64, 4096, 4, "tiles"),
+    ("d", "C", 512, 1024, 4, "tiles"), ("d", "C", 16, 16384, 8, "tiles"),
+    ("s", "C", 1, 65536, 1, "rows"), ("s", "C", 8, 4096, 4, "rows"),
+    ("s", "C", 33, 4096, 4, "rows"), ("s", "C", 65, 3072, 4, "rows"),
+    ("s", "C", 129, 3072, 1, "rows"), ("s", "C", 64, 1536, 4, "tiles"),
+    ("s", "C", 96, 1024, 1, "tiles"), ("s", "C", 128, 2048, 4, "tiles"),
 ]
 
 
@@ -58,7 +74,7 @@ def test_rule_at_measured_points(tmp_path):
     for t, op, n, bc, _, _ in MEASURED:  # more than 8 right-hand sides
         points += [(t, op, n, bc, r, "tiles") for r in (9, 16, 100)]
     # no batch is large enough where rows never win
-    points += [("d", "T", 512, 2 ** 31 - 1, 1, "tiles")]
+    points += [("d", "T", 512, 2 ** 31 - 1, 1, "tiles"), ("s", "C", 512, 2 ** 31 - 1, 1, "tiles")]
     text = "\n".join(" ".join(map(str, p[:5])) for p in points)
     r = subprocess.run([exe], input=text, capture_output=True, text=True, check=True)
     got = r.stdout.split()
