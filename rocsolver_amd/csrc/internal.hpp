@@ -115,11 +115,12 @@ rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ip
                          int64_t strideP, int* info, int j0, int jb, int o0, int oend, int uend,
                          int bc, bool pivot);
 // The finished block column [o0, o0 + nb), nb <= OUTER_NB, applied to the
-// columns outside it: interchanges, and U12 right of it.
+// columns outside it: interchanges, and U12 right of it, by diagonal blocks of
+// db (8, 16 or 32) rows, each with the roundings of a panel of db columns.
 constexpr int OUTER_NB = 128;
 template <typename T>
 rocblas_status outer_apply(hipStream_t stream, int n, Batch<T> A, int lda, const int* ipiv,
-                           int64_t strideP, int o0, int nb, int bc, bool pivot);
+                           int64_t strideP, int o0, int nb, int bc, bool pivot, int db = 32);
 
 template <typename T>
 rocblas_status getrf_blocked(hipStream_t stream, int m, int n, Batch<T> A, int lda, int* ipiv,

@@ -32,7 +32,9 @@ constexpr int PANEL_THREADS = 512;
 // of 16, 960 of 8), halves once per level (192, 256) at the price of a launch
 // for U12 of the larger ones.  Measured: dgetrf 4096 x 128 x 64 1.40 -> 1.10
 // ms, x 16 (64 MB) 0.69 -> 0.63, but x 4 0.52 -> 0.54; sgetrf 4096 x 128 x 64
-// 0.55 -> 0.51, x 16 0.34 -> 0.36.
+// 0.55 -> 0.51, x 16 0.34 -> 0.36.  The batch decides the order of the work
+// only: both group the sums by panel, so that a matrix's factors are the same
+// bits in any batch.
 constexpr int64_t BISECT_BYTES = int64_t(64) << 20;
 constexpr int64_t MAX_GRID_YZ = 65535; // grid y/z limit: larger batches are launched in chunks
 
@@ -339,11 +341,14 @@ constexpr int GT = 64; // tile
 constexpr int GK = 16; // k chunk
 constexpr int XCDS = 8;
 
-//
 // SHORT (K <= 32, the updates inside a block column): a tile is a chain of two
 // memory round trips rather than a stream, so C is read at the start with A
 // and B (one n = 2000 system 10.6 -> 7.0 us a launch).
-template <typename T, bool SHORT>
+//
+// GROUP (0: one): the products are summed and subtracted from C, in registers,
+// GROUP values of k at a time, so that one update by several panels of GROUP
+// columns rounds as an update by each of them does.
+template <typename T, bool SHORT, int GROUP>
 __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batch<T> AA,
                                                        int64_t offA, int lda, Batch<T> BB,
                                                        int64_t offB, int ldb, Batch<T> CC,
@@ -422,8 +427,9 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
             rb[t] = (kb < K && jb < N) ? Bm[kb + int64_t(jb) * ldb] : T(0);
         }
     };
+    static_assert(GROUP % 4 == 0, "whole steps");
     load(0);
-    if(SHORT)
+    if(SHORT || GROUP)
         load_c();
     int buf = 0;
     for(int k0 = 0; k0 < K; k0 += GK, buf ^= 1)
@@ -457,10 +463,23 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
 #pragma unroll
                 for(int t = 0; t < 2; ++t)
                     acc[s][t] = M_::run(bv[t], a[s], acc[s][t]);
+            if(GROUP && (k0 + kk + 4) % (GROUP ? GROUP : 4) == 0) // uniform
+            {
+#pragma unroll
+                for(int s = 0; s < 2; ++s)
+#pragma unroll
+                    for(int t = 0; t < 2; ++t)
+                    {
+#pragma unroll
+                        for(int r = 0; r < 4; ++r)
+                            c0[s][t][r] -= acc[s][t][r];
+                        acc[s][t] = acc_t{0, 0, 0, 0};
+                    }
+            }
         }
     }
 
-    if(!SHORT)
+    if(!SHORT && !GROUP)
         load_c();
 #pragma unroll
     for(int s = 0; s < 2; ++s)
@@ -473,7 +492,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
             {
                 const int j = j0 + wj + t * 16 + M_::row(lane, r);
                 if(i < M && j < N)
-                    C[i + int64_t(j) * ldc] = c0[s][t][r] - acc[s][t][r];
+                    C[i + int64_t(j) * ldc] = GROUP ? c0[s][t][r] : c0[s][t][r] - acc[s][t][r];
             }
     }
 }
@@ -481,7 +500,8 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
 template <typename T>
 static rocblas_status gemm_sub(hipStream_t stream, int M, int N, int K, Batch<T> A,
                                int64_t offA, int lda, Batch<T> B, int64_t offB, int ldb,
-                               Batch<T> C, int64_t offC, int ldc, int bc, const int* skip)
+                               Batch<T> C, int64_t offC, int ldc, int bc, const int* skip,
+                               int group = 0)
 {
     if(M <= 0 || N <= 0 || K <= 0 || bc <= 0)
         return rocblas_status_success;
@@ -491,16 +511,24 @@ static rocblas_status gemm_sub(hipStream_t stream, int M, int N, int K, Batch<T>
         [&](int64_t b0, int64_t nb, int64_t t0, int64_t nt) {
             const int64_t wgs = nt * (nb >= XCDS ? int64_t(ceil_div(nb, XCDS)) * XCDS : nb);
             const int* sk = skip ? skip + b0 : nullptr;
-            if(K <= 32)
-                hipLaunchKernelGGL((gemm_sub_kernel<T, true>), dim3(unsigned(wgs)), dim3(256), 0,
-                                   stream, M, N, K, batch_from(A, b0), offA, lda, batch_from(B, b0),
-                                   offB, ldb, batch_from(C, b0), offC, ldc, sk, int(nb), tm,
-                                   unsigned(t0), unsigned(nt));
+            auto go = [&](auto is_short, auto grp) {
+                hipLaunchKernelGGL(
+                    (gemm_sub_kernel<T, decltype(is_short)::value, decltype(grp)::value>),
+                    dim3(unsigned(wgs)), dim3(256), 0, stream, M, N, K, batch_from(A, b0), offA,
+                    lda, batch_from(B, b0), offB, ldb, batch_from(C, b0), offC, ldc, sk, int(nb),
+                    tm, unsigned(t0), unsigned(nt));
+            };
+            using std::integral_constant;
+            if(group == 8 && K > 8)
+                go(std::false_type{}, integral_constant<int, 8>{});
+            else if(group == 16 && K > 16)
+                go(std::false_type{}, integral_constant<int, 16>{});
+            else if(group == 32 && K > 32)
+                go(std::false_type{}, integral_constant<int, 32>{});
+            else if(K <= 32)
+                go(std::true_type{}, integral_constant<int, 0>{});
             else
-                hipLaunchKernelGGL((gemm_sub_kernel<T, false>), dim3(unsigned(wgs)), dim3(256), 0,
-                                   stream, M, N, K, batch_from(A, b0), offA, lda, batch_from(B, b0),
-                                   offB, ldb, batch_from(C, b0), offC, ldc, sk, int(nb), tm,
-                                   unsigned(t0), unsigned(nt));
+                go(std::false_type{}, integral_constant<int, 0>{});
             RSA_LAUNCH_CHECK();
             return rocblas_status_success;
         });
@@ -516,14 +544,16 @@ rocblas_status getrf_blocked(hipStream_t stream, int m, int n, Batch<T> A, int l
         return st;
     const int kmax = m < n ? m : n;
     // C[r0:m, r0:jend] -= A[r0:m, j:r0] A[j:r0, r0:jend]
-    auto update = [&](int j, int r0, int jend) {
+    auto update = [&](int j, int r0, int jend, int group = 0) {
         return gemm_sub<T>(stream, m - r0, jend - r0, r0 - j, A, r0 + int64_t(j) * lda, lda,
                            A, j + int64_t(r0) * lda, lda, A, r0 + int64_t(r0) * lda, lda, bc,
-                           nullptr);
+                           nullptr, group);
     };
     // Columns [j, j + w) of the block column [o0, oend) by halves: the left
     // half is factored, applied to the right half at once, then the right
-    // half.  uend: U12 of a single panel is solved up to there.
+    // half.  uend: U12 of a single panel is solved up to there.  The left half
+    // is whole panels of one width and is applied with the roundings of panel
+    // after panel, so that a matrix's factors do not depend on its batch.
     auto bisect = [&](auto&& self, int j, int w, int uend, int o0, int oend) -> rocblas_status {
         const int w0 = panel_reg_width<T>(m - j, lda);
         if(w <= w0)
@@ -532,11 +562,14 @@ rocblas_status getrf_blocked(hipStream_t stream, int m, int n, Batch<T> A, int l
         int w1 = w0;
         while(2 * w1 < w)
             w1 *= 2;
+        for(int c = w0; c < w1; c += w0) // up to where fewer rows allow wider panels
+            if(panel_reg_width<T>(m - j - c, lda) > w0)
+                w1 = c;
         rocblas_status s = self(self, j, w1, w1 == w0 ? j + w : j + w1, o0, oend);
         if(s == rocblas_status_success && w1 > w0) // the panels have moved the rows already
-            s = outer_apply<T>(stream, j + w, A, lda, ipiv, strideP, j, w1, bc, false);
+            s = outer_apply<T>(stream, j + w, A, lda, ipiv, strideP, j, w1, bc, false, w0);
         if(s == rocblas_status_success)
-            s = update(j, j + w1, j + w);
+            s = update(j, j + w1, j + w, w0);
         return s == rocblas_status_success ? self(self, j + w1, w - w1, j + w, o0, oend) : s;
     };
     for(int o0 = 0, nb = 0; o0 < kmax; o0 += nb)

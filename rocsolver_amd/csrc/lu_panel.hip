@@ -266,12 +266,12 @@ __global__ __launch_bounds__(NT, 2) void panel_reg_kernel(int m, Batch<T> AA, in
 // Bound by latency and by the scattered rows of the interchanges (one cache
 // line per row and column), so one block's interchanges are composed into a
 // map and applied once, not panel by panel.  The nb top rows stay in LDS from
-// the interchange to the solve: 32-row diagonal blocks by substitution (four
+// the interchange to the solve: diagonal blocks of DB rows by substitution (four
 // lanes per column), the rows below by matrix-core products.  Each wavefront
 // owns 16 columns from then on, so the solve has no barrier.
 constexpr int OUTER_COLS = 64;
 
-template <typename T, bool PIVOT>
+template <typename T, bool PIVOT, int DB>
 __global__ __launch_bounds__(256, 1) void outer_apply_kernel(int n, Batch<T> AA, int lda,
                                                              const int* __restrict__ ipivA,
                                                              int64_t strideP, int o0, int nb,
@@ -279,7 +279,6 @@ __global__ __launch_bounds__(256, 1) void outer_apply_kernel(int n, Batch<T> AA,
 {
     using M = mfma16<T>;
     constexpr int LS = OUTER_NB + 1; // column stride of the right-hand sides in LDS
-    constexpr int DB = 32; // diagonal block
     constexpr int UC = 16; // columns in flight
     __shared__ T sB[OUTER_COLS * LS];
     __shared__ __align__(16) T sL[OUTER_NB / DB][DB * DB];
@@ -404,7 +403,7 @@ __global__ __launch_bounds__(256, 1) void outer_apply_kernel(int n, Batch<T> AA,
 
 template <typename T>
 rocblas_status outer_apply(hipStream_t stream, int n, Batch<T> A, int lda, const int* ipiv,
-                           int64_t strideP, int o0, int nb, int bc, bool pivot)
+                           int64_t strideP, int o0, int nb, int bc, bool pivot, int db)
 {
     const int left = pivot ? ceil_div(o0, OUTER_COLS) : 0;
     const int chunks = left + ceil_div(n - o0 - nb, OUTER_COLS);
@@ -413,12 +412,20 @@ rocblas_status outer_apply(hipStream_t stream, int n, Batch<T> A, int lda, const
     for(int64_t b0 = 0; b0 < bc; b0 += 65535)
     {
         const int cnt = int((bc - b0) < 65535 ? (bc - b0) : 65535);
-        if(pivot)
-            hipLaunchKernelGGL((outer_apply_kernel<T, true>), dim3(chunks, cnt), dim3(256), 0,
-                               stream, n, A, lda, ipiv, strideP, o0, nb, left, b0);
+        auto go = [&](auto piv, auto d) {
+            hipLaunchKernelGGL((outer_apply_kernel<T, decltype(piv)::value, decltype(d)::value>),
+                               dim3(chunks, cnt), dim3(256), 0, stream, n, A, lda, ipiv, strideP,
+                               o0, nb, left, b0);
+        };
+        using std::integral_constant;
+        if(pivot) // the block column of a matrix
+            go(std::true_type{}, integral_constant<int, 32>{});
+        else if(db == 8) // part of one: by its panels
+            go(std::false_type{}, integral_constant<int, 8>{});
+        else if(db == 16)
+            go(std::false_type{}, integral_constant<int, 16>{});
         else
-            hipLaunchKernelGGL((outer_apply_kernel<T, false>), dim3(chunks, cnt), dim3(256), 0,
-                               stream, n, A, lda, ipiv, strideP, o0, nb, left, b0);
+            go(std::false_type{}, integral_constant<int, 32>{});
         RSA_LAUNCH_CHECK();
     }
     return rocblas_status_success;
@@ -491,7 +498,7 @@ rocblas_status panel_reg(hipStream_t stream, int m, Batch<T> A, int lda, int* ip
 #define RSA_PANEL_INST(T)                                                                       \
     template int panel_reg_width<T>(int, int);                                                  \
     template rocblas_status outer_apply<T>(hipStream_t, int, Batch<T>, int, const int*, int64_t, \
-                                           int, int, int, bool);                                \
+                                           int, int, int, bool, int);                           \
     template rocblas_status panel_reg<T>(hipStream_t, int, Batch<T>, int, int*, int64_t, int*,  \
                                          int, int, int, int, int, int, bool);
 RSA_PANEL_INST(float)
