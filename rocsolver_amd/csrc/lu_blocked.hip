@@ -18,6 +18,7 @@
 #include "internal.hpp"
 #include "mfma.hpp"
 #include "quad_solve.hpp"
+#include "rows_rule.hpp"
 
 #include <climits>
 
@@ -348,7 +349,10 @@ constexpr int XCDS = 8;
 // GROUP (0: one): the products are summed and subtracted from C, in registers,
 // GROUP values of k at a time, so that one update by several panels of GROUP
 // columns rounds as an update by each of them does.
-template <typename T, bool SHORT, int GROUP>
+//
+// TRANSA: the K x M transpose of A is stored; it goes through LDS by rows of
+// the product, as B does by columns.
+template <typename T, bool SHORT, int GROUP, bool TRANSA>
 __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batch<T> AA,
                                                        int64_t offA, int lda, Batch<T> BB,
                                                        int64_t offB, int ldb, Batch<T> CC,
@@ -363,7 +367,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
     constexpr int SR = GT + 16; // [k][i]
     constexpr int SC = GK + 1; // [j][k]
     constexpr int PT = GT * GK / 256; // entries of each operand per thread and chunk
-    __shared__ T sA[2][GK * SR];
+    __shared__ T sA[2][TRANSA ? GT * SC : GK * SR];
     __shared__ T sB[2][GT * SC];
 
     const unsigned id = blockIdx.x;
@@ -421,8 +425,9 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
         for(int t = 0; t < PT; ++t)
         {
             const int e = tid + 256 * t;
-            const int i = i0 + e % GT, k = k0 + e / GT;
-            ra[t] = (i < M && k < K) ? A[i + int64_t(k) * lda] : T(0);
+            const int i = i0 + (TRANSA ? e / GK : e % GT), k = k0 + (TRANSA ? e % GK : e / GT);
+            ra[t] = (i < M && k < K) ? A[TRANSA ? k + int64_t(i) * lda : i + int64_t(k) * lda]
+                                     : T(0);
             const int kb = k0 + e % GK, jb = j0 + e / GK;
             rb[t] = (kb < K && jb < N) ? Bm[kb + int64_t(jb) * ldb] : T(0);
         }
@@ -438,7 +443,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
         for(int t = 0; t < PT; ++t)
         {
             const int e = tid + 256 * t;
-            sA[buf][(e / GT) * SR + e % GT] = ra[t];
+            sA[buf][TRANSA ? (e / GK) * SC + e % GK : (e / GT) * SR + e % GT] = ra[t];
             sB[buf][(e / GK) * SC + e % GK] = rb[t];
         }
         __syncthreads();
@@ -453,7 +458,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
             for(int s = 0; s < 2; ++s)
             {
                 const int i = wi + s * 16 + lane % 16;
-                a[s] = sA[buf][k * SR + i];
+                a[s] = sA[buf][TRANSA ? i * SC + k : k * SR + i];
             }
 #pragma unroll
             for(int t = 0; t < 2; ++t)
@@ -501,7 +506,7 @@ template <typename T>
 static rocblas_status gemm_sub(hipStream_t stream, int M, int N, int K, Batch<T> A,
                                int64_t offA, int lda, Batch<T> B, int64_t offB, int ldb,
                                Batch<T> C, int64_t offC, int ldc, int bc, const int* skip,
-                               int group = 0)
+                               int group = 0, bool transA = false)
 {
     if(M <= 0 || N <= 0 || K <= 0 || bc <= 0)
         return rocblas_status_success;
@@ -511,24 +516,28 @@ static rocblas_status gemm_sub(hipStream_t stream, int M, int N, int K, Batch<T>
         [&](int64_t b0, int64_t nb, int64_t t0, int64_t nt) {
             const int64_t wgs = nt * (nb >= XCDS ? int64_t(ceil_div(nb, XCDS)) * XCDS : nb);
             const int* sk = skip ? skip + b0 : nullptr;
-            auto go = [&](auto is_short, auto grp) {
+            auto go = [&](auto is_short, auto grp, auto tr) {
                 hipLaunchKernelGGL(
-                    (gemm_sub_kernel<T, decltype(is_short)::value, decltype(grp)::value>),
+                    (gemm_sub_kernel<T, decltype(is_short)::value, decltype(grp)::value,
+                                     decltype(tr)::value>),
                     dim3(unsigned(wgs)), dim3(256), 0, stream, M, N, K, batch_from(A, b0), offA,
                     lda, batch_from(B, b0), offB, ldb, batch_from(C, b0), offC, ldc, sk, int(nb),
                     tm, unsigned(t0), unsigned(nt));
             };
             using std::integral_constant;
-            if(group == 8 && K > 8)
-                go(std::false_type{}, integral_constant<int, 8>{});
+            using no = std::false_type;
+            if(transA)
+                go(no{}, integral_constant<int, 0>{}, std::true_type{});
+            else if(group == 8 && K > 8)
+                go(no{}, integral_constant<int, 8>{}, no{});
             else if(group == 16 && K > 16)
-                go(std::false_type{}, integral_constant<int, 16>{});
+                go(no{}, integral_constant<int, 16>{}, no{});
             else if(group == 32 && K > 32)
-                go(std::false_type{}, integral_constant<int, 32>{});
+                go(no{}, integral_constant<int, 32>{}, no{});
             else if(K <= 32)
-                go(std::true_type{}, integral_constant<int, 0>{});
+                go(std::true_type{}, integral_constant<int, 0>{}, no{});
             else
-                go(std::false_type{}, integral_constant<int, 0>{});
+                go(no{}, integral_constant<int, 0>{}, no{});
             RSA_LAUNCH_CHECK();
             return rocblas_status_success;
         });
@@ -837,6 +846,8 @@ static rocblas_status permute_rows(hipStream_t stream, int n, int nrhs, Batch<T>
 // column solving 64-row blocks, with the update in a launch of its own, took
 // 1.7 ms for both triangles at n = 1024 x 64, 8 right-hand sides (transposed)
 // and 3.1 ms for one system of n = 2000; this kernel takes 0.69 and 0.80 ms.
+// Where there is work for the whole chip (trsm_many) a step only solves, and
+// gemm_sub_kernel updates: the same sums, the same bits.
 constexpr int ST = 128; // tile rows
 constexpr int SD = 32; // diagonal block rows
 constexpr int STEP_THREADS = 512;
@@ -1008,34 +1019,53 @@ static rocblas_status trsm_blocked(hipStream_t stream, int n, int nrhs, Batch<T>
                                    Batch<T> B, int ldb, int bc, const int* skip)
 {
     constexpr bool LOWER = KIND == 0 || KIND == 2;
+    constexpr bool TRANS = KIND >= 2;
+    constexpr int WIDE = sizeof(T) == 8 ? 64 : 128; // what the LDS holds
     const int tiles = ceil_div(n, ST);
-    const int cols = nrhs <= 16 ? 16 : 32;
-    for(int64_t b0 = 0; b0 < bc; b0 += MAX_GRID_YZ)
+    const bool many = trsm_many<T>(TRANS, tiles, nrhs, bc);
+    const int cols = nrhs <= 16 ? 16 : nrhs <= 32 || !many ? 32 : nrhs <= 64 ? 64 : WIDE;
+    for(int s = 0; s < tiles; ++s)
     {
-        const int nb = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);
-        for(int s = 0; s < tiles; ++s)
+        // step s solves tile `next`, after the update by the tile before
+        // unless the updates have launches of their own
+        const int next = LOWER ? s : tiles - 1 - s;
+        const int prev = s == 0 || many ? -1 : (LOWER ? s - 1 : next + 1);
+        const int cnt = prev < 0 ? 1 : tiles - s; // tiles not solved yet
+        const int tile0 = LOWER || prev < 0 ? next : 0;
+        for(int64_t b0 = 0; b0 < bc; b0 += MAX_GRID_YZ)
         {
-            // step s solves tile `next` after the update by the tile before
-            const int next = LOWER ? s : tiles - 1 - s;
-            const int prev = s == 0 ? -1 : (LOWER ? s - 1 : next + 1);
-            const int cnt = s == 0 ? 1 : tiles - s; // tiles not solved yet
-            const int tile0 = LOWER || s == 0 ? next : 0;
+            const int nb = int((bc - b0) < MAX_GRID_YZ ? (bc - b0) : MAX_GRID_YZ);
             // right-hand sides in x: more than 65535 groups of them are allowed
             const rocblas_status st = launch_split(
                 1, ceil_div(nrhs, cols), STEP_THREADS, 1,
                 [&](int64_t, int64_t, int64_t g0, int64_t ng) {
-                    const dim3 grid(unsigned(ng), cnt, nb);
+                    auto go = [&](auto c) {
+                        hipLaunchKernelGGL((trsm_step_kernel<T, KIND, decltype(c)::value>),
+                                           dim3(unsigned(ng), cnt, nb), dim3(STEP_THREADS), 0,
+                                           stream, n, nrhs, A, lda, B, ldb, skip, prev, next, tile0,
+                                           unsigned(g0), b0);
+                    };
                     if(cols == 16)
-                        hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 16>), grid,
-                                           dim3(STEP_THREADS), 0, stream, n, nrhs, A, lda, B, ldb,
-                                           skip, prev, next, tile0, unsigned(g0), b0);
+                        go(std::integral_constant<int, 16>{});
+                    else if(cols == 32)
+                        go(std::integral_constant<int, 32>{});
+                    else if(cols == 64)
+                        go(std::integral_constant<int, 64>{});
                     else
-                        hipLaunchKernelGGL((trsm_step_kernel<T, KIND, 32>), grid,
-                                           dim3(STEP_THREADS), 0, stream, n, nrhs, A, lda, B, ldb,
-                                           skip, prev, next, tile0, unsigned(g0), b0);
+                        go(std::integral_constant<int, WIDE>{});
                     RSA_LAUNCH_CHECK();
                     return rocblas_status_success;
                 });
+            if(st != rocblas_status_success)
+                return st;
+        }
+        if(many)
+        {
+            const int k0 = next * ST, k1 = k0 + ST < n ? k0 + ST : n;
+            const int r0 = LOWER ? k1 : 0, r1 = LOWER ? n : k0; // the tiles not solved yet
+            const int64_t offA = TRANS ? k0 + int64_t(r0) * lda : r0 + int64_t(k0) * lda;
+            const rocblas_status st = gemm_sub<T>(stream, r1 - r0, nrhs, k1 - k0, A, offA, lda, B,
+                                                  k0, ldb, B, r0, ldb, bc, skip, 0, TRANS);
             if(st != rocblas_status_success)
                 return st;
         }

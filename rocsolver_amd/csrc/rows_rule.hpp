@@ -1,6 +1,7 @@
 // rows_rule.hpp -- which kernel solves with a factor of order <= 512: the row
-// solver (trsv_rows.hpp) or the tile solver (tile_solve.hpp).  Same operations
-// per row, same bits.  Host code, no HIP.
+// solver (trsv_rows.hpp) or the tile solver (tile_solve.hpp); and how a blocked
+// solve of a larger order is launched.  Same operations per row, same bits.
+// Host code, no HIP.
 //
 // The tile solver works on 16 right-hand sides and whole 32-row blocks whatever
 // the call has; the row solver on what is there, in smaller workgroups that
@@ -136,6 +137,30 @@ inline bool potrs_by_rows(int n, int nrhs, int bc)
                                        {136, 4, 4, NEVER},
                                        {256, 32, NEVER, NEVER}};
     return sizeof(T) == 8 ? rows_win(R64, n, nrhs, bc) : rows_win(R32, n, nrhs, bc);
+}
+
+// Blocked solves (n > 512) of `tiles` tiles of 128 rows: whether the updates get
+// launches of their own (gemm_sub_kernel, which shares its operands through
+// LDS) and the solves up to 64 (FP64) or 128 right-hand sides per workgroup.
+// Where there is work for the whole chip, a step is bound by the operands that
+// every 32 right-hand sides read again, not by the launch that this costs.
+// Same sums, same bits.
+//
+// Step by step against own launches, in ms (a launch per 64 rows with updates
+// of their own, a thread per column, took 2.62, 4.98 and 1.45 in the first
+// three): FP64 n = 513 x 300, op T, 100 right-hand sides 3.37 against 1.52; n =
+// 800 x 64, op T, 600 6.53 against 2.62; n = 513 x 150, op N, 33 0.93 against
+// 0.46; FP32 n = 800 x 64, op T, 600 4.58 against 1.66; but FP64 n = 513 x 1, op
+// N, 2000 0.31 against 0.38, FP32 n = 2500 x 1, op N, 2000 1.58 against 2.03.
+// (FP32 takes half the time for the same steps, few systems share less.)
+template <typename T>
+inline bool trsm_many(bool trans, int tiles, int nrhs, int bc)
+{
+    const int64_t blocks = int64_t(tiles) * ((int64_t(nrhs) + 31) / 32) * bc;
+    const bool few = bc < 16;
+    if(sizeof(T) == 8)
+        return blocks > (trans && nrhs > 16 ? 400 : !trans && few ? 800 : 600);
+    return blocks > (trans ? (few ? 800 : 400) : few ? 2500 : 1400);
 }
 
 } // namespace rsa

@@ -1,4 +1,4 @@
-"""Which of two solvers a call takes (rocsolver_amd/csrc/rows_rule.hpp).
+"""Which of two ways a solve takes (rocsolver_amd/csrc/rows_rule.hpp).
 
 The header has no HIP in it: the host compiler builds it, and the rule is
 checked at points on both sides of its lines where both kernels were timed.
@@ -23,6 +23,14 @@ int main()
     while(scanf(" %c %c %d %d %d", &type, &op, &n, &bc, &nrhs) == 5)
     {
         bool rows;
+        if(n > 512)
+        {
+            const int tiles = (n + 127) / 128;
+            puts((type == 'd' ? rsa::trsm_many<double>(op == 'T', tiles, nrhs, bc)
+                              : rsa::trsm_many<float>(op == 'T', tiles, nrhs, bc))
+                     ? "many" : "step");
+            continue;
+        }
         if(op == 'C')
             rows = type == 'd' ? rsa::potrs_by_rows<double>(n, nrhs, bc)
                                : rsa::potrs_by_rows<float>(n, nrhs, bc);
@@ -49,6 +57,12 @@ MEASURED = [
     ("s", "N", 304, 1280, 4, "rows"), ("s", "N", 512, 512, 1, "tiles"),
     ("s", "T", 65, 8192, 1, "rows"), ("s", "T", 83, 8192, 4, "rows"),
     ("s", "T", 96, 8192, 4, "tiles"), ("s", "T", 512, 1024, 1, "tiles"),
+    # blocked getrs: updates in launches of their own, or with the solves step by step
+    ("d", "T", 513, 300, 100, "many"), ("d", "T", 800, 64, 600, "many"),
+    ("d", "N", 513, 150, 33, "many"), ("s", "T", 800, 64, 600, "many"),
+    ("s", "N", 600, 150, 40, "many"), ("d", "N", 513, 1, 2000, "step"),
+    ("d", "N", 2500, 4, 64, "step"), ("s", "N", 2500, 1, 2000, "step"),
+    ("d", "T", 1024, 64, 8, "step"), ("d", "T", 600, 150, 8, "many"), ("d", "N", 2000, 1, 1, "step"),
     # potrs
     ("d", "C", 1, 65536, 1, "rows"), ("d", "C", 8, 4096, 4, "rows"),
     ("d", "C", 32, 2048, 1, "rows"), ("d", "C", 64, 4096, 1, "rows"),
@@ -72,7 +86,7 @@ def test_rule_at_measured_points(tmp_path):
     subprocess.run([cxx, "-std=c++17", "-Wall", f"-I{CSRC}", src, "-o", exe], check=True)
     points = list(MEASURED)
     for t, op, n, bc, _, _ in MEASURED:  # more than 8 right-hand sides
-        points += [(t, op, n, bc, r, "tiles") for r in (9, 16, 100)]
+        points += [(t, op, n, bc, r, "tiles") for r in (9, 16, 100) if n <= 512]
     # no batch is large enough where rows never win
     points += [("d", "T", 512, 2 ** 31 - 1, 1, "tiles"), ("s", "C", 512, 2 ** 31 - 1, 1, "tiles")]
     text = "\n".join(" ".join(map(str, p[:5])) for p in points)
