@@ -99,7 +99,8 @@ __device__ __forceinline__ void chol_row_solve(const T* L11, const T* res, int l
 // operand loads.  So small workgroups and 128 registers: four matrices share
 // a CU, and the matrix-core products of one run under the pivots of another.
 // n = 300 x 1024 FP64: 0.72 ms (three matrices per CU: 0.78); one thread per
-// row with vector fused multiply-adds took 4.14 ms.
+// row with vector fused multiply-adds took 4.14 ms.  The 128 registers leave
+// FP64 160 bytes a lane in scratch beyond n = 64.
 template <typename T, int NT, bool UP>
 __global__ __launch_bounds__(NT, NT == 64 ? 2 : 4) void potrf_kernel(int n, Batch<T> AA, int lda,
                                                       int* __restrict__ info)

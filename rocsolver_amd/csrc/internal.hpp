@@ -83,13 +83,18 @@ rocblas_status getrs_fused(hipStream_t stream, bool trans, int n, int nrhs, Batc
 // tiles (16 a pass, a workgroup per system); the same operations in the same
 // order.  The team's pass takes a wavefront per system beyond n = 32 and is a
 // chain of n broadcasts, so tiles are the faster ones for large orders, many
-// right-hand sides or few systems.  Team against tile kernels, op T:
-//   n = 56 x 8192, 8 right-hand sides: FP64 223 against 164 us, FP32 148
-//     against 118 (1 right-hand side: 0.6 to 0.8 of the tiles' time);
-//   n = 40 x 8192, 17 right-hand sides: FP64 405 against 307 us, FP32 241
-//     against 208 (n = 33: FP32 1.05 times slower);
-//   n = 32 x 1024, 8 right-hand sides: FP64 25 against 16 us, FP32 21 against
-//     15 (x 8192: 1.3 times slower).
+// right-hand sides or few systems.  Team against tile kernels in us, the
+// smallest gains on the tiles' side (a team's pass costs the same for 2 to 8
+// right-hand sides):
+//   n = 49 x 8192, 2: op N FP64 190 against 144, FP32 122 against 95; op T 204
+//     against 167, 128 against 118 (1 right-hand side: 0.5 to 0.8 of the tiles'
+//     time);
+//   n = 40 x 8192, 16: op N FP64 280 against 145, FP32 162 against 95; op T 282
+//     against 167, 166 against 120 (n = 33: FP32 1.05 times slower);
+//   n = 40 x 1024, 2: op N FP64 33 against 26, FP32 29 against 25; op T 35
+//     against 28, 33 against 28;
+//   n = 28 x 1024, 2: op N FP64 24 against 17, FP32 20 against 17; op T 24
+//     against 18, 21 against 18 (x 8192: 1.3 times slower).
 template <typename T>
 inline bool getrs_small_by_tiles(int n, int nrhs, int bc)
 {

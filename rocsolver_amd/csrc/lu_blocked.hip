@@ -1,20 +1,24 @@
 // lu_blocked.hip -- right-looking blocked LU and blocked triangular solves for
 // any m, n (the path for matrices beyond the register-resident kernels).
 //
-// getrf, per block column j of width jb (reference structure:
+// getrf, per block column of OUTER_NB columns (reference structure:
 // library/src/lapack/roclapack_getrf.hpp:608-752, without rocBLAS):
-//   1. panel_reg (lu_panel.hip): one workgroup per matrix factors
-//      A[j:m, j:j+jb] in registers with partial pivoting, applies its
-//      interchanges to the other columns and solves U12 = L11^-1 A12.
-//      Panels too tall for the registers: panel_kernel, interchanging rows
-//      inside the panel at each column in global memory, then every other
-//      column at once (roclapack_getf2.hpp:41-99 semantics: the same final
-//      rows), and u12_kernel, one thread per column right of the panel.
-//   2. gemm_sub_kernel: A22 -= L21 * U12 on MFMA (v_mfma_f64_16x16x4f64 /
+//   1. panel_reg (lu_panel.hip): one workgroup per matrix factors 8 to 32
+//      columns in registers with partial pivoting, applies its interchanges to
+//      the rest of the block column and solves U12 = L11^-1 A12 there; the
+//      block column's rows below are then updated (gemm_sub_kernel), panel
+//      after panel or, for large batches of narrow panels, by halves;
+//   2. outer_apply (lu_panel.hip): the block column's interchanges, composed
+//      into one map, on all other columns, and U12 right of it;
+//   3. gemm_sub_kernel: A22 -= L21 * U12 on MFMA (v_mfma_f64_16x16x4f64 /
 //      v_mfma_f32_16x16x4f32), 64x64 tiles.
+// Panels too tall for the registers: panel_kernel, interchanging rows inside
+// the panel at each column in global memory, then every other column at once
+// (roclapack_getf2.hpp:41-99 semantics: the same final rows), u12_kernel, one
+// thread per column right of the panel, and the update.
 // getrs (roclapack_getrs.hpp:117-150): the interchanges, then each triangle
 // in 128-row tiles, one launch per tile (update by the tile before, then its
-// own solve).
+// own solve) or, with work for the whole chip, a launch for each.
 #include "internal.hpp"
 #include "mfma.hpp"
 #include "quad_solve.hpp"

@@ -14,8 +14,9 @@
 // holds it, before a second barrier.  Against every wavefront publishing its
 // candidate row before a single barrier: FP64 LU n = 256 x 4096 4.18 -> 3.79
 // ms, n = 300 x 1024 2.96 -> 2.43, n = 128 x 16384 3.06 -> 2.86; FP32 n = 256
-// x 4096 1.81 -> 1.63 ms (a batch of 64 FP32 matrices of n = 96, latency
-// alone, 76 -> 79 us).  Putting off the update of the columns beyond the next
+// x 4096 1.81 -> 1.63 ms.  A batch of 64 FP32 matrices of n = 96, latency
+// alone, lost 3 us to the second barrier and takes 71 us since the diagonal
+// blocks are inverted by four lanes per column (78 before both).  Putting off the update of the columns beyond the next
 // one until after the search's barrier was slower (n = 2000 5.08 -> 5.24 ms).
 #pragma once
 

@@ -46,7 +46,10 @@ constexpr int tile_solve_tpw()
 }
 
 // Wavefronts per SIMD that the registers are cut for: two tiles a wavefront
-// fit four, four tiles two in FP64.
+// fit four, four tiles two in FP64.  (At NMAX = 64 the LDS holds six workgroups
+// of two wavefronts a CU, three a SIMD.)  At four the FP64 kernels of n <= 256
+// keep 12 to 52 bytes a lane in scratch; four tiles a wavefront, two a SIMD,
+// took 91 us for 78 at n = 96 x 2048.
 template <typename T, int NMAX, int NT>
 constexpr int tile_waves()
 {
