@@ -10,8 +10,9 @@
 // block the order fills.
 //
 // The lines come from timing both at about 110 orders and 25 batches per type
-// and op.  Over those the chosen kernel is within 1.15 of the faster one beyond
-// launch noise, and mostly the faster one; the wrong one costs up to 3.5 times.
+// and op.  Over those the chosen kernel is within 1.15 of the faster one (but for
+// launches of a few us, and FP32 potrs of n <= 2 with 9 to 16 right-hand sides,
+// 1.3) and mostly the faster one; the wrong one costs up to 3.5 times.
 #pragma once
 
 #include <cstddef>
