@@ -346,23 +346,30 @@ constexpr int GT = 64; // tile
 constexpr int GK = 16; // k chunk
 constexpr int XCDS = 8;
 
-// SHORT (K <= 32, the updates inside a block column): a tile is a chain of two
-// memory round trips rather than a stream, so C is read at the start with A
-// and B (one n = 2000 system 10.6 -> 7.0 us a launch).
-//
-// GROUP (0: one): the products are summed and subtracted from C, in registers,
-// GROUP values of k at a time, so that one update by several panels of GROUP
-// columns rounds as an update by each of them does.
+// The products are summed and subtracted from C, in registers, GROUP values of
+// k at a time: 32, so that the sums stay short (one sum over K = 128 made the
+// errors of LU and solve 1.1 to 1.2 times larger on random matrices), or a
+// panel's columns, so that one update by several panels rounds as an update by
+// each of them does.  So C is read at the start, with A and B, which is also
+// what an update inside a block column wants, a chain of two memory round trips
+// rather than a stream (one n = 2000 system 10.6 -> 7.0 us a launch).
 //
 // TRANSA: the K x M transpose of A is stored; it goes through LDS by rows of
 // the product, as B does by columns.
-template <typename T, bool SHORT, int GROUP, bool TRANSA>
-__global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batch<T> AA,
-                                                       int64_t offA, int lda, Batch<T> BB,
-                                                       int64_t offB, int ldb, Batch<T> CC,
-                                                       int64_t offC, int ldc,
-                                                       const int* __restrict__ skip, int bc,
-                                                       int tm, unsigned tile0, unsigned tiles)
+constexpr int GG = 32;
+
+// Wavefronts a SIMD in groups of 32: n = 1024 x 64, FP32 with 4 in place of 5
+// 2 % slower (three registers are spilled for 5), FP64 with 3 in place of 4 3 %.
+// Shorter groups: the fewest registers win (6000 x 128 x 64 FP32, groups of 8,
+// with 5 1.00 in place of 0.90 ms).
+template <typename T, int GROUP, bool TRANSA>
+constexpr int GEMM_WAVES = GROUP < 2 * GK ? 1 : sizeof(T) == 4 ? 5 : TRANSA ? 1 : 4;
+
+template <typename T, int GROUP, bool TRANSA>
+__global__ __launch_bounds__(256, (GEMM_WAVES<T, GROUP, TRANSA>)) void gemm_sub_kernel(
+    int M, int N, int K, Batch<T> AA, int64_t offA, int lda, Batch<T> BB, int64_t offB, int ldb,
+    Batch<T> CC, int64_t offC, int ldc, const int* __restrict__ skip, int bc, int tm,
+    unsigned tile0, unsigned tiles)
 {
     using M_ = mfma16<T>;
     using acc_t = typename M_::acc_t;
@@ -436,13 +443,40 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
             rb[t] = (kb < K && jb < N) ? Bm[kb + int64_t(jb) * ldb] : T(0);
         }
     };
-    static_assert(GROUP % 4 == 0, "whole steps");
+    auto subtract = [&]() {
+#pragma unroll
+        for(int s = 0; s < 2; ++s)
+#pragma unroll
+            for(int t = 0; t < 2; ++t)
+            {
+#pragma unroll
+                for(int r = 0; r < 4; ++r)
+                    c0[s][t][r] -= acc[s][t][r];
+                acc[s][t] = acc_t{0, 0, 0, 0};
+            }
+    };
+    static_assert(GROUP % 4 == 0 && (GROUP == 2 * GK || GK % GROUP == 0), "whole groups");
     load(0);
-    if(SHORT || GROUP)
-        load_c();
-    int buf = 0;
-    for(int k0 = 0; k0 < K; k0 += GK, buf ^= 1)
+    // The loop in place keeps C's addresses in registers for the stores, the
+    // call does not: n = 1500 x 32 FP32 1 % faster so, groups of 8 (6000 x 128 x
+    // 64 FP32) 4 % slower.
+    if constexpr(GROUP == 2 * GK)
     {
+#pragma unroll
+        for(int s = 0; s < 2; ++s)
+#pragma unroll
+            for(int t = 0; t < 2; ++t)
+#pragma unroll
+                for(int r = 0; r < 4; ++r)
+                {
+                    const int i = i0 + wi + s * 16 + lane % 16;
+                    const int j = j0 + wj + t * 16 + M_::row(lane, r);
+                    c0[s][t][r] = (i < M && j < N) ? C[i + int64_t(j) * ldc] : T(0);
+                }
+    }
+    else
+        load_c();
+    auto chunk = [&](int k0, int buf) {
 #pragma unroll
         for(int t = 0; t < PT; ++t)
         {
@@ -472,24 +506,37 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
 #pragma unroll
                 for(int t = 0; t < 2; ++t)
                     acc[s][t] = M_::run(bv[t], a[s], acc[s][t]);
-            if(GROUP && (k0 + kk + 4) % (GROUP ? GROUP : 4) == 0) // uniform
+            if(GROUP < 2 * GK && (k0 + kk + 4) % GROUP == 0)
             {
-#pragma unroll
-                for(int s = 0; s < 2; ++s)
-#pragma unroll
-                    for(int t = 0; t < 2; ++t)
-                    {
-#pragma unroll
-                        for(int r = 0; r < 4; ++r)
-                            c0[s][t][r] -= acc[s][t][r];
-                        acc[s][t] = acc_t{0, 0, 0, 0};
-                    }
+                subtract();
+            }
+        }
+    };
+    if constexpr(sizeof(T) == 8 && GROUP == 2 * GK)
+    {
+        // both chunks of a sum unrolled: its first products take a zero
+        // constant (n = 1024 x 64 2 to 3 % faster; FP32 2 % slower)
+        for(int k0 = 0; k0 < K; k0 += 2 * GK)
+        {
+            chunk(k0, 0);
+            if(k0 + GK < K) // uniform
+                chunk(k0 + GK, 1);
+            subtract();
+        }
+    }
+    else
+    {
+        int buf = 0;
+        for(int k0 = 0; k0 < K; k0 += GK, buf ^= 1)
+        {
+            chunk(k0, buf);
+            if(GROUP == 2 * GK && (buf == 1 || k0 + GK >= K)) // uniform
+            {
+                subtract();
             }
         }
     }
 
-    if(!SHORT && !GROUP)
-        load_c();
 #pragma unroll
     for(int s = 0; s < 2; ++s)
     {
@@ -501,7 +548,7 @@ __global__ __launch_bounds__(256) void gemm_sub_kernel(int M, int N, int K, Batc
             {
                 const int j = j0 + wj + t * 16 + M_::row(lane, r);
                 if(i < M && j < N)
-                    C[i + int64_t(j) * ldc] = GROUP ? c0[s][t][r] : c0[s][t][r] - acc[s][t][r];
+                    C[i + int64_t(j) * ldc] = c0[s][t][r];
             }
     }
 }
@@ -510,7 +557,7 @@ template <typename T>
 static rocblas_status gemm_sub(hipStream_t stream, int M, int N, int K, Batch<T> A,
                                int64_t offA, int lda, Batch<T> B, int64_t offB, int ldb,
                                Batch<T> C, int64_t offC, int ldc, int bc, const int* skip,
-                               int group = 0, bool transA = false)
+                               int group = GG, bool transA = false)
 {
     if(M <= 0 || N <= 0 || K <= 0 || bc <= 0)
         return rocblas_status_success;
@@ -520,28 +567,22 @@ static rocblas_status gemm_sub(hipStream_t stream, int M, int N, int K, Batch<T>
         [&](int64_t b0, int64_t nb, int64_t t0, int64_t nt) {
             const int64_t wgs = nt * (nb >= XCDS ? int64_t(ceil_div(nb, XCDS)) * XCDS : nb);
             const int* sk = skip ? skip + b0 : nullptr;
-            auto go = [&](auto is_short, auto grp, auto tr) {
+            auto go = [&](auto grp, auto tr) {
                 hipLaunchKernelGGL(
-                    (gemm_sub_kernel<T, decltype(is_short)::value, decltype(grp)::value,
-                                     decltype(tr)::value>),
+                    (gemm_sub_kernel<T, decltype(grp)::value, decltype(tr)::value>),
                     dim3(unsigned(wgs)), dim3(256), 0, stream, M, N, K, batch_from(A, b0), offA,
                     lda, batch_from(B, b0), offB, ldb, batch_from(C, b0), offC, ldc, sk, int(nb),
                     tm, unsigned(t0), unsigned(nt));
             };
             using std::integral_constant;
-            using no = std::false_type;
             if(transA)
-                go(no{}, integral_constant<int, 0>{}, std::true_type{});
-            else if(group == 8 && K > 8)
-                go(no{}, integral_constant<int, 8>{}, no{});
-            else if(group == 16 && K > 16)
-                go(no{}, integral_constant<int, 16>{}, no{});
-            else if(group == 32 && K > 32)
-                go(no{}, integral_constant<int, 32>{}, no{});
-            else if(K <= 32)
-                go(std::true_type{}, integral_constant<int, 0>{}, no{});
+                go(integral_constant<int, GG>{}, std::true_type{});
+            else if(group == 8)
+                go(integral_constant<int, 8>{}, std::false_type{});
+            else if(group == 16)
+                go(integral_constant<int, 16>{}, std::false_type{});
             else
-                go(no{}, integral_constant<int, 0>{}, no{});
+                go(integral_constant<int, GG>{}, std::false_type{});
             RSA_LAUNCH_CHECK();
             return rocblas_status_success;
         });
@@ -557,7 +598,7 @@ rocblas_status getrf_blocked(hipStream_t stream, int m, int n, Batch<T> A, int l
         return st;
     const int kmax = m < n ? m : n;
     // C[r0:m, r0:jend] -= A[r0:m, j:r0] A[j:r0, r0:jend]
-    auto update = [&](int j, int r0, int jend, int group = 0) {
+    auto update = [&](int j, int r0, int jend, int group = GG) {
         return gemm_sub<T>(stream, m - r0, jend - r0, r0 - j, A, r0 + int64_t(j) * lda, lda,
                            A, j + int64_t(r0) * lda, lda, A, r0 + int64_t(r0) * lda, lda, bc,
                            nullptr, group);
@@ -913,13 +954,24 @@ __global__ __launch_bounds__(STEP_THREADS) void trsm_step_kernel(int n, int nrhs
                     }
     }
 
-    typename M::acc_t acc[RT];
+    // this wavefront's right-hand sides: register r of tile t holds row wr + 16 t
+    // + lane % 16, column M::row(lane, r)
+    T x[RT][4];
 #pragma unroll
     for(int t = 0; t < RT; ++t)
-        acc[t] = typename M::acc_t{0, 0, 0, 0};
+#pragma unroll
+        for(int r = 0; r < 4; ++r)
+        {
+            const int i = r0 + wr + 16 * t + (lane & 15), c = c0 + M::row(lane, r);
+            x[t][r] = i < n && c < nrhs ? Bm[i + int64_t(c) * ldb] : T(0);
+        }
     const int col = c0 + (lane & 15);
     if(prev >= 0)
     {
+        typename M::acc_t acc[RT];
+#pragma unroll
+        for(int t = 0; t < RT; ++t)
+            acc[t] = typename M::acc_t{0, 0, 0, 0};
         const int k0 = prev * ST;
         constexpr int KS = RT == 1 ? 16 : 8; // matrix-core steps whose loads are in flight
 #pragma unroll 1
@@ -942,7 +994,16 @@ __global__ __launch_bounds__(STEP_THREADS) void trsm_step_kernel(int n, int nrhs
             for(int q = 0; q < KS; ++q)
 #pragma unroll
                 for(int t = 0; t < RT; ++t)
+                {
                     acc[t] = M::run(bv[q], av[q][t], acc[t]);
+                    if((4 * q + 4) % GG == 0) // sums of GG products, as gemm_sub_kernel's
+                    {
+#pragma unroll
+                        for(int r = 0; r < 4; ++r)
+                            x[t][r] -= acc[t][r];
+                        acc[t] = typename M::acc_t{0, 0, 0, 0};
+                    }
+                }
         }
     }
 #pragma unroll
@@ -954,13 +1015,10 @@ __global__ __launch_bounds__(STEP_THREADS) void trsm_step_kernel(int n, int nrhs
         for(int r = 0; r < 4; ++r)
         {
             const int c = c0 + M::row(lane, r);
-            const bool in = i < n && c < nrhs;
-            T* p = Bm + i + int64_t(c) * ldb;
-            const T v = in ? *p - acc[t][r] : T(0);
             if(solve)
-                sB[(16 * (wid % CG) + M::row(lane, r)) * LS + li] = v;
-            else if(in)
-                *p = v;
+                sB[(16 * (wid % CG) + M::row(lane, r)) * LS + li] = x[t][r];
+            else if(i < n && c < nrhs)
+                Bm[i + int64_t(c) * ldb] = x[t][r];
         }
     }
     if(!solve)
@@ -1069,7 +1127,7 @@ static rocblas_status trsm_blocked(hipStream_t stream, int n, int nrhs, Batch<T>
             const int r0 = LOWER ? k1 : 0, r1 = LOWER ? n : k0; // the tiles not solved yet
             const int64_t offA = TRANS ? k0 + int64_t(r0) * lda : r0 + int64_t(k0) * lda;
             const rocblas_status st = gemm_sub<T>(stream, r1 - r0, nrhs, k1 - k0, A, offA, lda, B,
-                                                  k0, ldb, B, r0, ldb, bc, skip, 0, TRANS);
+                                                  k0, ldb, B, r0, ldb, bc, skip, GG, TRANS);
             if(st != rocblas_status_success)
                 return st;
         }
