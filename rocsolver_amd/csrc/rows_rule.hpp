@@ -152,7 +152,8 @@ inline bool potrs_by_rows(int n, int nrhs, int bc)
 // three): FP64 n = 513 x 300, op T, 100 right-hand sides 3.37 against 1.52; n =
 // 800 x 64, op T, 600 6.53 against 2.62; n = 513 x 150, op N, 33 0.93 against
 // 0.46; FP32 n = 800 x 64, op T, 600 4.58 against 1.66; but FP64 n = 513 x 1, op
-// N, 2000 0.31 against 0.38, FP32 n = 2500 x 1, op N, 2000 1.58 against 2.03.
+// N, 2000 0.31 against 0.38, FP32 n = 2500 x 1, op N, 2000 1.58 against 2.03, n =
+// 600 x 300, op N, 1 0.34 against 0.39, n = 1100 x 64, op T, 1 0.45 against 0.51.
 // (FP32 takes half the time for the same steps, few systems share less.)
 template <typename T>
 inline bool trsm_many(bool trans, int tiles, int nrhs, int bc)
@@ -161,7 +162,9 @@ inline bool trsm_many(bool trans, int tiles, int nrhs, int bc)
     const bool few = bc < 16;
     if(sizeof(T) == 8)
         return blocks > (trans && nrhs > 16 ? 400 : !trans && few ? 800 : 600);
-    return blocks > (trans ? (few ? 800 : 400) : few ? 2500 : 1400);
+    if(trans)
+        return blocks > (few ? 800 : nrhs <= 16 ? 600 : 400);
+    return blocks > (few ? 2500 : nrhs <= 16 ? 2000 : 1400);
 }
 
 } // namespace rsa

@@ -62,6 +62,8 @@ MEASURED = [
     ("d", "N", 513, 150, 33, "many"), ("s", "T", 800, 64, 600, "many"),
     ("s", "N", 600, 150, 40, "many"), ("d", "N", 513, 1, 2000, "step"),
     ("d", "N", 2500, 4, 64, "step"), ("s", "N", 2500, 1, 2000, "step"),
+    ("s", "N", 600, 300, 1, "step"), ("s", "N", 600, 300, 17, "many"),
+    ("s", "T", 1100, 64, 1, "step"), ("s", "T", 1100, 64, 17, "many"),
     ("d", "T", 1024, 64, 8, "step"), ("d", "T", 600, 150, 8, "many"), ("d", "N", 2000, 1, 1, "step"),
     # potrs
     ("d", "C", 1, 65536, 1, "rows"), ("d", "C", 8, 4096, 4, "rows"),
