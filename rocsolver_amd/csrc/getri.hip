@@ -93,8 +93,15 @@ static dim3 square_grid(int n, int bc)
 // solve skips the blocks that the identity leaves zero (on average half), and
 // no right-hand side is written or read: dgetri n = 100 x 2000 0.81 -> 0.68
 // ms with its two copies.  Scratch a lane: 44 bytes in FP64 up to n = 128, 152
-// (FP32 36) up to 256, 12 (36) beyond.
-template <typename T, int NMAX, int NT, int CT>
+// (FP32 36) up to 256, 12 (36) beyond; with SUMS 28 (36) and 20 (28).
+//
+// SUMS (no interchanges, n > 64): a row adds sums of 32 products, not a chain of
+// n; with interchanges every column has the bits of a solve for it.  FP32 errors
+// against 64 bits, chain -> sums: n = 512, random 5.8e-6 -> 3.9e-6, diagonally
+// dominant 4.3e-7 -> 1.4e-7; n = 200 1.9e-6 -> 1.6e-6, 2.7e-7 -> 1.3e-7.  Times
+// with the chain and with sums: n = 200 x 2000 FP32 0.96 and 0.98 ms, FP64 2.22
+// and 1.84; n = 400 x 512 FP64 2.82 and 2.86.
+template <typename T, int NMAX, int NT, int CT, bool SUMS>
 __global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void inverse_tile_kernel(
     int n, Batch<T> AA, int lda, const int* __restrict__ ipivA, int64_t strideP, Batch<T> XX,
     int ldx, int bc, unsigned chunks)
@@ -103,7 +110,7 @@ __global__ __launch_bounds__(NT, (tile_waves<T, NMAX, NT>())) void inverse_tile_
     const int64_t b = tile_solve_system(blockIdx.x, chunks, chunk);
     if(b >= bc)
         return;
-    tile_inverse_body<T, NMAX, NT, CT>(n, int(chunk) * CT * TSC, AA[b], lda,
+    tile_inverse_body<T, NMAX, NT, CT, SUMS>(n, int(chunk) * CT * TSC, AA[b], lda,
                                    ipivA ? ipivA + b * strideP : nullptr, XX[b], ldx);
 }
 
@@ -130,9 +137,13 @@ static rocblas_status inverse_tiles(hipStream_t stream, int n, Batch<T> LU, int 
         constexpr int NMAX = decltype(nmax)::value;
         constexpr int NT = decltype(nt)::value;
         constexpr int CT = decltype(ct)::value;
+        auto* kernel = inverse_tile_kernel<T, NMAX, NT, CT, false>;
+        if constexpr(NMAX > 64)
+            if(!ipiv)
+                kernel = inverse_tile_kernel<T, NMAX, NT, CT, true>;
         return launch_split(
             bc, chunks, NT, TILE_XCDS, [&](int64_t b0, int64_t nb, int64_t, int64_t) {
-                hipLaunchKernelGGL((inverse_tile_kernel<T, NMAX, NT, CT>),
+                hipLaunchKernelGGL(kernel,
                                    dim3(unsigned(tile_solve_grid(int(nb), chunks))), dim3(NT), 0,
                                    stream, n, batch_from(LU, b0), ldlu,
                                    ipiv ? ipiv + b0 * strideP : nullptr, strideP,

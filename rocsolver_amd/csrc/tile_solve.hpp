@@ -60,8 +60,11 @@ constexpr int tile_waves()
 // of op(A).  Rows past n are zero in and out.  par: parity of the LDS buffers.
 // A forward solve starts at block `begin` (the rows before it are zero).  CT
 // groups of 16 right-hand sides share the factor's entries and the barriers;
-// each has its own solving wavefront.
-template <typename T, int NT, int TPW, int CT, bool LOWER, bool TRANS, bool UNIT>
+// each has its own solving wavefront.  SUMS: a block's 32 products are summed
+// from zero before they are added to a row, so that a row's chain is n / 32
+// sums long in place of n products.
+template <typename T, int NT, int TPW, int CT, bool LOWER, bool TRANS, bool UNIT,
+          bool SUMS = false>
 __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>& A,
                                                     typename mfma16<T>::acc_t (&acc)[TPW][CT],
                                                     T (*sX)[CT * TSC * TSX],
@@ -73,6 +76,11 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
     static_assert(CT <= NW, "a solving wavefront per group");
     constexpr int DL = TSB * TSB / NT; // entries of the diagonal block per thread
     constexpr int KS = TSB / 4;
+    // Solved values read where they are used, not ahead: the sums leave no
+    // registers for them at n = 129 to 256 in FP64 (204 -> 28 bytes of scratch a
+    // lane, n = 200 x 2000 2.50 -> 1.84 ms; up to 512, with none to spare in
+    // either, 5 % slower)
+    constexpr bool LATE = SUMS && sizeof(T) == 8 && CT > 1 && TPW == 2;
     const int D = (n + TSB - 1) / TSB;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
@@ -177,16 +185,38 @@ __device__ __forceinline__ void tile_solve_triangle(int n, const MatrixBuffer<T>
         T* Ln = sL[par ^ 1];
         par ^= 1;
         T bv[CT][KS];
-        {
+        auto load_solved = [&](int ct) {
             const int lane = fresh_tid() & 63;
             const int g = LOWER ? lane >> 4 : 3 - (lane >> 4);
 #pragma unroll
-            for(int ct = 0; ct < CT; ++ct)
+            for(int ks = 0; ks < KS; ++ks)
+                bv[ct][ks] = -X[(16 * ct + (lane & 15)) * TSX + 4 * ks + g];
+        };
+        if constexpr(!LATE)
 #pragma unroll
-                for(int ks = 0; ks < KS; ++ks)
-                    bv[ct][ks] = -X[(16 * ct + (lane & 15)) * TSX + 4 * ks + g];
-        }
+            for(int ct = 0; ct < CT; ++ct)
+                load_solved(ct);
         auto update = [&](int t) {
+            if constexpr(SUMS)
+            {
+#pragma unroll
+                for(int ct = 0; ct < CT; ++ct)
+                {
+                    if constexpr(LATE)
+                        load_solved(ct);
+                    typename M::acc_t sum = {0, 0, 0, 0};
+#pragma unroll
+                    for(int q = 0; q < KS; ++q)
+                    {
+                        const int ks = LOWER ? q : KS - 1 - q;
+                        sum = M::run(bv[ct][ks], av[t][ks], sum);
+                    }
+#pragma unroll
+                    for(int r = 0; r < 4; ++r)
+                        acc[t][ct][r] += sum[r];
+                }
+                return;
+            }
 #pragma unroll
             for(int q = 0; q < KS; ++q)
             {
@@ -373,7 +403,7 @@ __device__ __forceinline__ void tile_solve_body(int n, int c0, int cend, const T
 // the product is column s_row[k] of X (ipiv null: no interchanges).  The
 // right-hand sides are columns of the identity, formed here; their rows before
 // block c0 / 32 are zero through the forward solve, which starts there.
-template <typename T, int NMAX, int NT, int CT>
+template <typename T, int NMAX, int NT, int CT, bool SUMS>
 __device__ __forceinline__ void tile_inverse_body(int n, int c0, const T* __restrict__ Ap, int lda,
                                                   const int* __restrict__ ipiv, T* Xm, int ldx)
 {
@@ -406,8 +436,8 @@ __device__ __forceinline__ void tile_inverse_body(int n, int c0, const T* __rest
             acc[t][r / 4][r % 4] = i < n && i == k ? T(1) : T(0);
         }
     int par = 0;
-    tile_solve_triangle<T, NT, TPW, CT, true, false, true>(n, A, acc, sX, sL, par, c0 / TSB);
-    tile_solve_triangle<T, NT, TPW, CT, false, false, false>(n, A, acc, sX, sL, par);
+    tile_solve_triangle<T, NT, TPW, CT, true, false, true, SUMS>(n, A, acc, sX, sL, par, c0 / TSB);
+    tile_solve_triangle<T, NT, TPW, CT, false, false, false, SUMS>(n, A, acc, sX, sL, par);
 #pragma unroll
     for(int t = 0; t < TPW; ++t)
 #pragma unroll
